@@ -15,7 +15,9 @@
 // An operator Op supplies
 //   kName, kNS (stencil fields), Col (per-column registers), d (Dims),
 //   Stg (registers of the column a thread stages: its own and its ring column),
-//   init_stage(col index, Stg&), stage_level(k), stage(k, a, Stg, v[kNS]),
+//   kMapped (fields read at the source columns cs of their halo values),
+//   init_stage(col index, Stg&), stage_level(k), stage(k, a, am, Stg, v[kNS])
+//   with a the point's address, am its mapped one (a unless kMapped),
 //   init_col(col index, Col&),
 //   point(k, a, Col, nb) with nb(m, f) = field f at stencil neighbour m
 //   (0 (0,0) 1 (+1,0) 2 (+1,+1) 3 (0,+1) 4 (-1,0) 5 (-1,-1) 6 (0,-1)),
@@ -57,13 +59,16 @@ struct ColStencil {
   static constexpr const char* kName = Op::kName;
   static constexpr int kThreads = 256;
   static constexpr int NS = Op::kNS;
+  static constexpr int kWaves = 1;
   Op op;
   StGeom cg;
+  const int* cs = nullptr;   // kMapped: source columns
   static int lds_elems(const StGeom& cg) { return 2 * NS * (cg.TX + 2) * (cg.TY + 2); }
   struct State {
     typename Op::Col col;
     typename Op::Stg sg, rsg;   // staging registers of the own and the ring column
     long a, ra;        // own and ring addresses at the current level
+    int rm;            // kMapped: the ring point's mapped address
     int k, sidx, ridx;
     bool outp, ring;
   };
@@ -102,6 +107,7 @@ struct ColStencil {
       s.ridx = (y + 1) * SW + x + 1;
       s.ra = ((long)(l * d.kall + k0) * g + (j0 + y)) * g + (i0 + x);
       op.init_stage(((long)l * g + (j0 + y)) * g + (i0 + x), s.rsg);
+      if constexpr (Op::kMapped) s.rm = (int)src_at(d, cs, ((long)l * g + (j0 + y)) * g + (i0 + x), k0);
     }
     return k1 - k0;
   }
@@ -111,11 +117,11 @@ struct ColStencil {
     real* buf = lds + (step & 1) * NS * P;
     real v[NS];
     if (s.outp) {
-      op.stage(s.k, s.a, s.sg, v);
+      op.stage(s.k, s.a, s.a, s.sg, v);
       for (int f = 0; f < NS; ++f) buf[f * P + s.sidx] = v[f];
     }
     if (s.ring) {
-      op.stage(s.k, s.ra, s.rsg, v);
+      op.stage(s.k, s.ra, Op::kMapped ? (long)s.rm : s.ra, s.rsg, v);
       for (int f = 0; f < NS; ++f) buf[f * P + s.ridx] = v[f];
     }
   }
@@ -133,6 +139,9 @@ struct ColStencil {
     const long gg = (long)op.d.g * op.d.g;
     s.a += gg;
     s.ra += gg;
+    if constexpr (Op::kMapped) {
+      if (s.ring) s.rm += (int)src_stride(op.d, s.rm);
+    }
     s.k += 1;
   }
 };
@@ -142,6 +151,7 @@ struct ColStencil {
 struct ViMainHC {
   static constexpr const char* kName = "vi_main_h";
   static constexpr int kNS = 8;
+  static constexpr bool kMapped = true;
   ViMainH pk;
   Dims d;
   struct Col {
@@ -150,8 +160,8 @@ struct ViMainHC {
   struct Stg {};
   NH_HD void init_stage(long, Stg&) const {}
   NH_HD bool stage_level(int k) const { return k >= d.kmin && k <= d.kmax; }
-  NH_HD void stage(int, long a, const Stg&, real* v) const {
-    for (int f = 0; f < kNS; ++f) v[f] = pk.stage_ptr(f, 0)[a];
+  NH_HD void stage(int, long a, long am, const Stg&, real* v) const {
+    for (int f = 0; f < kNS; ++f) v[f] = pk.stage_val(f, a, am);
   }
   NH_HD void init_col(long ci, Col& col) const {
     for (int dd = 0; dd < 3; ++dd)
@@ -199,6 +209,7 @@ template <int NFLD, class P>
 struct LapC {
   static constexpr const char* kName = (NFLD == 6) ? "hdiff_pass1" : "hdiff_pass2_lap";
   static constexpr int kNS = NFLD;
+  static constexpr bool kMapped = NFLD == 4;   // the second pass reads the first's output
   P pk;
   Dims d;
   const real* in[NFLD];
@@ -210,8 +221,8 @@ struct LapC {
   struct Stg {};
   NH_HD void init_stage(long, Stg&) const {}
   NH_HD bool stage_level(int) const { return true; }
-  NH_HD void stage(int k, long a, const Stg&, real* v) const {
-    for (int f = 0; f < NFLD; ++f) v[f] = pk.input(f, a, k);
+  NH_HD void stage(int k, long, long am, const Stg&, real* v) const {
+    for (int f = 0; f < NFLD; ++f) v[f] = pk.input(f, am, k);
   }
   NH_HD void init_col(long ci, Col& col) const {
     for (int m = 0; m < 7; ++m) col.c[m] = rc(pk.G.clap, d.nreg, m, ci);
@@ -239,6 +250,7 @@ template <int NFLD>
 struct LapTC {
   static constexpr const char* kName = "hdiff_lap_adj";
   static constexpr int kNS = NFLD;
+  static constexpr bool kMapped = false;
   Dims d; Geo G;
   const real* ob[NFLD];
   real* ib[NFLD];
@@ -248,7 +260,7 @@ struct LapTC {
   struct Stg {};
   NH_HD void init_stage(long, Stg&) const {}
   NH_HD bool stage_level(int) const { return true; }
-  NH_HD void stage(int, long a, const Stg&, real* v) const {
+  NH_HD void stage(int, long a, long, const Stg&, real* v) const {
     for (int f = 0; f < NFLD; ++f) v[f] = ob[f][a];
   }
   NH_HD void init_col(long ci, Col& col) const {
@@ -285,6 +297,7 @@ struct LapTC {
 struct AdvMomC {
   static constexpr const char* kName = "adv_mom";
   static constexpr int kNS = 6;
+  static constexpr bool kMapped = false;
   AdvMomP pk;
   Dims d;
   struct Col {
@@ -298,7 +311,7 @@ struct AdvMomC {
     for (int q = 0; q < 3; ++q) sg.x[q] = pk.G.gx[q * d.nreg + ci];
   }
   NH_HD bool stage_level(int k) const { return k >= d.kmin && k <= d.kmax; }
-  NH_HD void stage(int k, long a, const Stg& sg, real* v) const {
+  NH_HD void stage(int k, long a, long, const Stg& sg, real* v) const {
     const long NF = d.NF, gg = (long)d.g * d.g;
     const real* wd = pk.diag + I_W * NF;
     const real R = pk.c.RADIUS;

@@ -57,6 +57,19 @@ NH_HD inline T ldc(const T* p) {
 #endif
 }
 
+// Values at a 32-bit byte offset from a uniform base: one vector register
+// addresses the same point of every field (the loads take the base from scalar
+// registers).  A field is below 4 GiB: 64 fields of that size already exceed
+// the card's memory.
+template <class T>
+NH_HD inline const T& at_off(const T* p, unsigned off) {
+  return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(p) + off);
+}
+template <class T>
+NH_HD inline T& at_off(T* p, unsigned off) {
+  return *reinterpret_cast<T*>(reinterpret_cast<char*>(p) + off);
+}
+
 // Load of an element that the calling thread alone reads and writes during
 // the kernel, once each and the load first (a read-modify-write of a value
 // the thread owns, such as a column's adjoint bar).  No other thread stores
@@ -312,6 +325,25 @@ NH_HD inline long halo_colbase(const Dims& d, long c, long* ks) {
   long lp = p / 6;
   *ks = 6;
   return d.R + lp * d.kall * 6 + (p - lp * 6);
+}
+
+// Halo values read at their source.  cs[c] is the level-0 field address of the
+// column whose values column c holds after a halo fill: its own for a compute
+// column, the source's for a halo column (or its own for every column, to read
+// the halo values a field itself holds).  A kernel that reads a field through
+// cs needs no halo fill of it.
+NH_HD inline long src_stride(const Dims& d, long b) { return (b < d.R) ? (long)d.g * d.g : 6L; }
+// the same in byte offsets of a field
+NH_HD inline unsigned src_stride_off(const Dims& d, unsigned off) {
+  return (off < (unsigned)(d.R * (long)sizeof(real))) ? (unsigned)(d.g * d.g * (int)sizeof(real)) : 6u * sizeof(real);
+}
+NH_HD inline long src_at(const Dims& d, const int* cs, long col, int k) {
+  const long b = cs[col];
+  return b + (long)k * src_stride(d, b);
+}
+// point v of pole lp (v = 0: the centre) at level k
+NH_HD inline long src_pole(const Dims& d, const int* cs, int lp, int v, int k) {
+  return src_at(d, cs, d.nreg + (long)lp * 6 + v, k);
 }
 
 struct HaloGather {

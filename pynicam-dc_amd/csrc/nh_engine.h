@@ -77,6 +77,13 @@ struct Context {
   int* halo_dst = nullptr;      // level-0 field addresses of the halo map
   int* halo_src = nullptr;
   long halo_n = 0;
+  // per column the level-0 address its values are read from: col_own the
+  // column's own, col_src the source's for halo columns
+  int* col_own = nullptr;
+  int* col_src = nullptr;
+  // the halo map only fills points that are not computed, each once and from
+  // a point it does not fill: kernels may read col_src instead of a filled field
+  bool halo_direct = false;
   real* ws = nullptr;
   double* dws = nullptr;
   // adjoint workspace (allocated by the first adjoint call)
@@ -245,6 +252,9 @@ int upload_geometry(X& x, Context& ctx, const nh_geometry* g) {
   return x.check("upload_geometry");
 }
 
+// largest field (values) whose halo values are read at their source with 8-byte fields
+constexpr long kDirectMax64 = 4000000;
+
 template <class X>
 int upload_halo(X& x, Context& ctx, const int32_t* dst, const int32_t* src, long n) {
   const long ncol = ctx.d.nreg + 12;
@@ -253,7 +263,9 @@ int upload_halo(X& x, Context& ctx, const int32_t* dst, const int32_t* src, long
   }
   if (ctx.halo_dst) { x.release(ctx.halo_dst); ctx.halo_dst = nullptr; }
   if (ctx.halo_src) { x.release(ctx.halo_src); ctx.halo_src = nullptr; }
+  if (ctx.col_own) { x.release(ctx.col_own); ctx.col_own = ctx.col_src = nullptr; }
   ctx.halo_n = n;
+  ctx.halo_direct = false;
   // the adjoint of the gather scatters destination bars onto sources in one
   // pass: that needs every destination once and no destination as a source
   {
@@ -265,6 +277,22 @@ int upload_halo(X& x, Context& ctx, const int32_t* dst, const int32_t* src, long
     }
     for (long h = 0; h < n && ok; ++h) ok = !(role[src[h]] & 1);
     ctx.halo_adj_ok = ok;
+    // col_src reads stand for a filled field only where no filled point is a
+    // compute point (a kernel's own value, or its neighbour's, would differ)
+    const int g = ctx.d.g;
+    for (long h = 0; h < n && ok; ++h) {
+      const long c = dst[h];
+      const long r = c % ((long)g * g), j = r / g, i = r - j * g;
+      ok = c < ctx.d.nreg ? !(i >= 1 && i <= g - 2 && j >= 1 && j <= g - 2) : (c - ctx.d.nreg) % 6 != 0;
+    }
+    // Reading halo values at their source saves three launches per small step
+    // (8 us each at gl05, 12-16 at gl06, 22-26 at gl07) and makes the readers
+    // slower, since the first and last column of a region are one value per
+    // cache line for them too.  With 4-byte fields it is the faster form at
+    // every size (step 4.66 -> 4.41 ms at gl06, 13.6 -> 13.3 at gl07); with
+    // 8-byte fields the corner kernels lose their paired loads (CornerPts),
+    // which pays up to about gl06 (gl05 2.78 -> 2.63 ms) and not at gl07.
+    ctx.halo_direct = ok && (sizeof(real) == 4 || ctx.d.NF <= kDirectMax64);
   }
   if (n == 0) return 0;
   // the kernels index halo slot and level in 32 bits and take level-0 field
@@ -281,6 +309,17 @@ int upload_halo(X& x, Context& ctx, const int32_t* dst, const int32_t* src, long
   if (!ctx.halo_dst || !ctx.halo_src) return NH_ERR_ALLOC;
   x.h2d(ctx.halo_dst, db.data(), n * sizeof(int));
   x.h2d(ctx.halo_src, sb.data(), n * sizeof(int));
+  std::vector<int> cols((size_t)(2 * ncol));
+  for (long c = 0; c < ncol; ++c) {
+    long ks;
+    cols[(size_t)c] = cols[(size_t)(ncol + c)] = (int)halo_colbase(ctx.d, c, &ks);
+  }
+  if (ctx.halo_direct)
+    for (long h = 0; h < n; ++h) cols[(size_t)(ncol + dst[h])] = sb[(size_t)h];
+  ctx.col_own = (int*)x.alloc(2 * ncol * sizeof(int));
+  if (!ctx.col_own) return NH_ERR_ALLOC;
+  ctx.col_src = ctx.col_own + ncol;
+  x.h2d(ctx.col_own, cols.data(), 2 * ncol * sizeof(int));
   return x.check("upload_halo");
 }
 
@@ -317,25 +356,41 @@ constexpr int kDivDampChunks = 4;
 constexpr int kColChunks = 6;
 
 // ----------------------------------------------------------------------------
-// 3-D divergence damping of (vx, vy, vz, w) into out (3 fields)
+// 3-D divergence damping of (vx, vy, vz, w) into out (3 fields); cs: columns
+// the inputs' halo values are read from.  The second operator reads the first
+// one's halo values at their source.
 // ----------------------------------------------------------------------------
+// one operator; map: the inputs' halo values are read through cs.  With
+// 4-byte fields the mapped form runs in any case (CornerPts)
+template <int OP, class X>
+void divdamp_op(X& x, const Context& ctx, const real* const v[3], const real* w, real* const out[3], const int* cs,
+                bool map) {
+  auto run = [&](auto k) {
+    k.d = ctx.d; k.c = ctx.c; k.G = ctx.G;
+    k.cg = col_geom(ctx.d, kDivDampChunks);
+    k.rw = w;
+    k.cs = cs;
+    for (int q = 0; q < 3; ++q) { k.v[q] = v[q]; k.out[q] = out[q]; }
+    x.run_cols(k, k.cg.nblocks, decltype(k)::lds_elems(k.cg));
+  };
+  if constexpr (sizeof(real) == 4) {
+    run(DivDampK<OP, true>{});
+  } else {
+    if (map) run(DivDampK<OP, true>{});
+    else run(DivDampK<OP, false>{});
+  }
+}
+
 template <class X>
 void divdamp(X& x, const Context& ctx, const real* vx, const real* vy, const real* vz, const real* w,
-             real* out0, real* out1, real* out2) {
-  const ColGeom cg = col_geom(ctx.d, kDivDampChunks);
-  DivDampK<1> a;
-  a.d = ctx.d; a.c = ctx.c; a.G = ctx.G; a.cg = cg;
-  a.v[0] = vx; a.v[1] = vy; a.v[2] = vz; a.rw = w;
-  for (int q = 0; q < 3; ++q) a.out[q] = ctx.field(W_DDT + q);
-  x.run_cols(a, cg.nblocks, DivDampK<1>::lds_elems(cg));
+             real* out0, real* out1, real* out2, const int* cs) {
+  const real* v[3] = {vx, vy, vz};
   real* tmp[3] = {ctx.field(W_DDT), ctx.field(W_DDT + 1), ctx.field(W_DDT + 2)};
-  halo(x, ctx, tmp, 3);
-  DivDampK<2> b;
-  b.d = ctx.d; b.c = ctx.c; b.G = ctx.G; b.cg = cg;
-  for (int q = 0; q < 3; ++q) b.v[q] = tmp[q];
-  b.rw = nullptr;
-  b.out[0] = out0; b.out[1] = out1; b.out[2] = out2;
-  x.run_cols(b, cg.nblocks, DivDampK<2>::lds_elems(cg));
+  real* out[3] = {out0, out1, out2};
+  divdamp_op<1>(x, ctx, v, w, tmp, cs, cs != ctx.col_own);
+  if (!ctx.halo_direct) halo(x, ctx, tmp, 3);
+  const real* t[3] = {tmp[0], tmp[1], tmp[2]};
+  divdamp_op<2>(x, ctx, t, nullptr, out, ctx.halo_direct ? ctx.col_src : ctx.col_own, ctx.halo_direct);
 }
 
 // ----------------------------------------------------------------------------
@@ -534,6 +589,12 @@ struct SmallBufs {
   real* we[3];
   real* ddv = nullptr;   // damping force of ps (3 fields); default the step workspace
   real* hv = nullptr;    // divergences of dv (3 fields); default the step workspace
+  // ps holds its own halo values (SplitInit writes every point); otherwise they
+  // are read at their source
+  bool own_halo = true;
+  // fill the halos of dv (the adjoint reads them); otherwise their readers take
+  // the halo values from their source
+  bool fill_halo = false;
 };
 
 // the fields a stage computes that its small steps (and the adjoint) read:
@@ -554,10 +615,12 @@ inline StageFields ws_stage(const Context& ctx) {
 // the iterated Laplacians of (vx, vy, vz, w, T, rho) in two passes, pass 1
 // into sf.hda with a halo fill, pass 2 into sf.hdb (6 fields each).  The halo
 // fill of pass 2 (fill_hdb) is for callers that read hdb off the compute
-// points; the step reads it only at its own compute points (path 0).
+// points; the step reads it only at its own compute points (path 0).  Pass 2
+// reads the halo values of hda at their source; fill_hda is for callers that
+// read hda later (the adjoint's transposes).
 template <class X>
 void hdiff_passes(X& x, const Context& ctx, const real* prog, const real* diag, const StageFields& sf,
-                  bool fill_hdb = true) {
+                  bool fill_hda, bool fill_hdb) {
   const Dims& d = ctx.d;
   const long NF = d.NF;
   HDiffPassP<0> f;
@@ -572,6 +635,8 @@ void hdiff_passes(X& x, const Context& ctx, const real* prog, const real* diag, 
   }
   const ColGeom cg = col_geom(d, kColChunks);
   const StGeom sg = st_geom(d, kColChunks);
+  const bool direct = ctx.halo_direct && !fill_hda;
+  const int* csrc = direct ? ctx.col_src : ctx.col_own;
   {
     ColStencil<LapC<6, HDiffPassP<0>>> cs;
     cs.op.pk = f;
@@ -581,7 +646,7 @@ void hdiff_passes(X& x, const Context& ctx, const real* prog, const real* diag, 
     cs.cg = sg;
     x.run_cols(cs, sg.nblocks, decltype(cs)::lds_elems(sg));
   }
-  halo_block(x, ctx, sf.hda, 6);
+  if (!direct) halo_block(x, ctx, sf.hda, 6);
   // second pass: the Laplacians of fields 0..3, then the Kh-weighted
   // diffusion of fields 4, 5 (whose pole blocks do all six fields)
   HDiffPassP<1> f2;
@@ -591,6 +656,7 @@ void hdiff_passes(X& x, const Context& ctx, const real* prog, const real* diag, 
     f2.out[q] = sf.hdb + q * NF;
   }
   f2.rhog = prog;
+  f2.cs = csrc;
   {
     ColStencil<LapC<4, HDiffPassP<1>>> cs;
     cs.op.pk = f2;
@@ -598,14 +664,19 @@ void hdiff_passes(X& x, const Context& ctx, const real* prog, const real* diag, 
     for (int q = 0; q < 4; ++q) { cs.op.in[q] = f2.in[q]; cs.op.out[q] = f2.out[q]; }
     cs.op.pole_off = true;
     cs.cg = sg;
+    cs.cs = csrc;
     x.run_cols(cs, sg.nblocks, decltype(cs)::lds_elems(sg));
   }
   {
-    DiffKhK k2;
-    k2.d = d; k2.c = ctx.c; k2.G = ctx.G; k2.cg = cg;
-    for (int q = 0; q < 6; ++q) { k2.in[q] = f2.in[q]; k2.out[q] = f2.out[q]; }
-    k2.rhog = prog;
-    x.run_cols(k2, cg.nblocks, DiffKhK::lds_elems(cg));
+    auto run = [&](auto k2) {
+      k2.d = d; k2.c = ctx.c; k2.G = ctx.G; k2.cg = cg;
+      for (int q = 0; q < 6; ++q) { k2.in[q] = f2.in[q]; k2.out[q] = f2.out[q]; }
+      k2.rhog = prog;
+      k2.cs = csrc;
+      x.run_cols(k2, cg.nblocks, decltype(k2)::lds_elems(cg));
+    };
+    if (direct) run(DiffKhK<true>{});
+    else run(DiffKhK<false>{});
   }
   if (fill_hdb) halo_block(x, ctx, sf.hdb, 6);
 }
@@ -616,7 +687,7 @@ void hdiff_passes(X& x, const Context& ctx, const real* prog, const real* diag, 
 // start of the mean fluxes
 template <class X>
 void stage_large(X& x, const Context& ctx, real* prog, const real* rhogq, double dts, const StageFields& sf,
-                 bool means = true) {
+                 bool keep_halo, bool means = true) {
   const Dims& d = ctx.d;
   const long NF = d.NF;
   real* diag = ctx.field(W_DIAG);
@@ -638,10 +709,10 @@ void stage_large(X& x, const Context& ctx, real* prog, const real* rhogq, double
   } else {
     run_staged(x, AdvMomP{d, ctx.c, ctx.G, prog, diag, gadv});
   }
-  hdiff_passes(x, ctx, prog, diag, sf, false);
+  hdiff_passes(x, ctx, prog, diag, sf, keep_halo, false);
   // divergence damping of the large-step momentum
   divdamp(x, ctx, prog + 1 * NF, prog + 2 * NF, prog + 3 * NF, prog + 4 * NF,
-          ctx.field(W_DD), ctx.field(W_DD + 1), ctx.field(W_DD + 2));
+          ctx.field(W_DD), ctx.field(W_DD + 1), ctx.field(W_DD + 2), ctx.col_own);
   {
     ViPath0P f;
     f.d = d; f.c = ctx.c; f.G = ctx.G;
@@ -669,25 +740,29 @@ void small_hv(X& x, const Context& ctx, const real* prog, real* const dv[3], rea
   for (int q = 0; q < 3; ++q) f.dv[q] = dv[q];
   f.eth = ctx.field(W_ETH); f.ethtot = sf.ethtot; f.gT = sf.gT;
   for (int q = 0; q < 3; ++q) f.hv[q] = hv + q * ctx.d.NF;
+  f.cs = ctx.col_src;
   ColStencil<ViMainHC> cs;
   cs.op.pk = f;
   cs.op.d = ctx.d;
   cs.cg = st_geom(ctx.d, kColChunks);
+  cs.cs = ctx.col_src;
   x.run_cols(cs, cs.cg.nblocks, ColStencil<ViMainHC>::lds_elems(cs.cg));
 }
 
 // one small step (mod_vi.py:1283-1450): divergence damping of the split
-// momentum, path1, vi_main (horizontal, tridiagonal, mass/energy), halos
+// momentum, path1, vi_main (horizontal, tridiagonal, mass/energy); last: no
+// small step of the stage follows
 template <class X>
 void small_step(X& x, const Context& ctx, const real* prog, const SmallBufs& s, double dts, double rweight,
-                const StageFields& sf, bool means = true) {
+                const StageFields& sf, bool last, bool means = true) {
   const Dims& d = ctx.d;
   const long NF = d.NF;
   real* gT = sf.gT;
   real* pm = means ? ctx.field(W_PM) : nullptr;   // the tracer's mean mass fluxes
   real* ddv = s.ddv ? s.ddv : ctx.field(W_DDV);
   real* hvb = s.hv ? s.hv : ctx.field(W_HV);
-  divdamp(x, ctx, s.ps[1], s.ps[2], s.ps[3], s.ps[4], ddv, ddv + NF, ddv + 2 * NF);
+  const int* cs = (s.own_halo || !ctx.halo_direct) ? ctx.col_own : ctx.col_src;
+  divdamp(x, ctx, s.ps[1], s.ps[2], s.ps[3], s.ps[4], ddv, ddv + NF, ddv + 2 * NF, cs);
   {
     Path1P f;
     f.d = d; f.c = ctx.c; f.G = ctx.G;
@@ -698,9 +773,10 @@ void small_step(X& x, const Context& ctx, const real* prog, const SmallBufs& s, 
     for (int q = 0; q < 3; ++q) f.dd[q] = ddv + q * NF;
     for (int q = 0; q < 3; ++q) f.dv[q] = s.dv[q];
     f.pm = pm;
+    f.cs = cs;
     run_staged(x, f);
   }
-  halo(x, ctx, s.dv, 3);
+  if (s.fill_halo || !ctx.halo_direct) halo(x, ctx, s.dv, 3);
   small_hv(x, ctx, prog, s.dv, hvb, sf);
   real* hv[3] = {hvb, hvb + NF, hvb + 2 * NF};
   {
@@ -732,7 +808,11 @@ void small_step(X& x, const Context& ctx, const real* prog, const SmallBufs& s, 
     f.pm = pm;
     x.run_pts(f, d);
   }
-  halo(x, ctx, s.we, 3);
+  // of the outputs' halos only rhogw's and rhoge's are read, by the next small step
+  if (!ctx.halo_direct && !last) {
+    real* h[2] = {s.we[1], s.we[2]};
+    halo(x, ctx, h, 2);
+  }
 }
 
 // PROG += PROG_split with the horizontal projection
@@ -800,7 +880,7 @@ int dyn_step(X& x, const Context& ctx, real* prog, real* progq, int nq, double d
     if (tape) x.d2d(tp.input(nl), prog, 6 * NF * sizeof(real));
     else if (record) x.d2d(record + (long)nl * 6 * NF, prog, 6 * NF * sizeof(real));
     const StageFields sf = tape ? tp.stage(nl) : ws_stage(ctx);
-    stage_large(x, ctx, prog, progq, dts, sf);
+    stage_large(x, ctx, prog, progq, dts, sf, tape != nullptr);
     // split state ps[0..5], path1 momentum dv[0..2], vi_main output we[0..2]
     SmallBufs s;
     if (tape) {
@@ -816,18 +896,20 @@ int dyn_step(X& x, const Context& ctx, real* prog, real* progq, int nq, double d
       x.run(f, NF);
     }
     const double rweight = 1.0 / (double)nsub[nl];
+    s.fill_halo = tape != nullptr;
     for (int it = 0; it < nsub[nl]; ++it) {
+      s.own_halo = it == 0;
       if (tape) {
         // outputs straight into the next slot: (we0, dv0, dv1, dv2, we1, we2)
         real* c1 = tp.slot(nl, it + 1);
         s.we[0] = c1; s.dv[0] = c1 + NF; s.dv[1] = c1 + 2 * NF; s.dv[2] = c1 + 3 * NF;
         s.we[1] = c1 + 4 * NF; s.we[2] = c1 + 5 * NF;
         s.hv = tp.slot(nl, it) + 6 * NF;
-        small_step(x, ctx, prog, s, dts, rweight, sf);
+        small_step(x, ctx, prog, s, dts, rweight, sf, it == nsub[nl] - 1);
         for (int q = 0; q < 6; ++q) s.ps[q] = c1 + q * NF;
         continue;
       }
-      small_step(x, ctx, prog, s, dts, rweight, sf);
+      small_step(x, ctx, prog, s, dts, rweight, sf, it == nsub[nl] - 1);
       // rotate buffers: the new split state is (we0, dv0, dv1, dv2, we1, we2)
       real* old[6] = {s.ps[0], s.ps[1], s.ps[2], s.ps[3], s.ps[4], s.ps[5]};
       s.ps[0] = s.we[0]; s.ps[1] = s.dv[0]; s.ps[2] = s.dv[1]; s.ps[3] = s.dv[2]; s.ps[4] = s.we[1];

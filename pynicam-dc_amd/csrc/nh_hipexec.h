@@ -57,7 +57,7 @@ __global__ __launch_bounds__(256) void k_pts(F f, int nx, int nblk) {
 // column tiles: per block init(), then per level level_a, barrier, level_b;
 // the number of levels is uniform over the block
 template <class F>
-__global__ __launch_bounds__(F::kThreads) void k_cols(F f, int nblk) {
+__global__ __launch_bounds__(F::kThreads) __attribute__((amdgpu_waves_per_eu(F::kWaves))) void k_cols(F f, int nblk) {
   extern __shared__ __align__(16) unsigned char nh_lds_bytes[];
   typename F::LdsT* lds = reinterpret_cast<typename F::LdsT*>(nh_lds_bytes);
   const int blk = xcd_block((int)blockIdx.x, nblk);

@@ -58,7 +58,8 @@ void v_destroy(Context* c) {
   if (!c) return;
   NHX x(c->device, nullptr, &c->prof);
   x.sync();
-  void* bufs[9] = {c->ws, c->dws, c->geo_buf, c->geo64_buf, c->int_buf, c->halo_dst, c->halo_src, c->aws, c->adws};
+  void* bufs[10] = {c->ws, c->dws, c->geo_buf, c->geo64_buf, c->int_buf, c->halo_dst, c->halo_src, c->col_own,
+                    c->aws, c->adws};
   for (void* b : bufs)
     if (b) x.release(b);
   x.prof_release();
@@ -158,7 +159,7 @@ int v_op(Context* c, int op, const void* const* in, void* const* out, double dt,
       real* hdb = c->field(W_HDB);
       x.run(FillZero{hda}, 12 * NF);
       const StageFields sf{hda, hdb, c->field(W_GT), c->field(W_ETHTOT), c->dfield(D_MC)};
-      hdiff_passes(x, *c, prog, diag, sf);
+      hdiff_passes(x, *c, prog, diag, sf, false, true);
       HDiffTendOp f;
       f.d = d; f.c = c->c; f.G = c->G;
       f.rhog = prog;
@@ -167,7 +168,7 @@ int v_op(Context* c, int op, const void* const* in, void* const* out, double dt,
       break;
     }
     case OP_DIVDAMP: {
-      divdamp(x, *c, R(0), R(1), R(2), R(3), (real*)out[0], (real*)out[1], (real*)out[2]);
+      divdamp(x, *c, R(0), R(1), R(2), R(3), (real*)out[0], (real*)out[1], (real*)out[2], c->col_own);
       break;
     }
     case OP_LIMITER_V: {

@@ -169,6 +169,7 @@ struct AdvMomP {
   // fields read on the stencil: vx, vy, vz, w(k), w(k+1), rhogvx, rhogvy, rhogvz
   static constexpr int kNStage = 8;
   static constexpr bool kStageF32 = false;
+  static constexpr bool kMapped = false;
   Dims d; Consts c; Geo G;
   const real* prog;
   const real* diag;
@@ -327,8 +328,6 @@ struct AdvMomP {
 template <int LAST>
 struct HDiffPassP {
   static constexpr const char* kName = LAST ? "hdiff_pass2" : "hdiff_pass1";
-  static constexpr int kNStage = 6;    // the six filtered fields (first pass)
-  static constexpr bool kStageF32 = false;
   Dims d; Consts c; Geo G;
   const real* in[6];
   real* out[6];
@@ -336,8 +335,7 @@ struct HDiffPassP {
   // first pass: FP64 k-profile subtracted from input f (tem - tem_bs,
   // rho - rho_bs, mod_numfilter.py:1068-1076), or none
   const double* sub[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
-  NH_HD const real* stage_ptr(int f, int) const { return in[f]; }
-  NH_HD bool stage_level(int) const { return true; }
+  const int* cs = nullptr;   // second pass: source columns of the inputs' halo values
   NH_HD real input(int f, long b, int k) const {
     return sub[f] ? (real)((double)in[f][b] - sub[f][k]) : in[f][b];
   }
@@ -350,6 +348,7 @@ struct HDiffPassP {
     }
     const long a = p.a;
     const Cell cl = cell_of_pt(p);
+    auto pa = [&](int v) { return src_pole(d, cs, p.lp, v, p.k); };
     for (int q = 0; q < 6; ++q) {
       real r;
       if (q >= 4) {
@@ -357,9 +356,9 @@ struct HDiffPassP {
         const real* rg = rhog;
         const real gam = c.GAMMA_H;
         auto kh = [rg, fac, gam](long xx) { return rg[xx] * fac * gam; };
-        r = p.pole ? diffusion_pl(G, p.lp, in[q], kh, a) : diffusion7(G, d, cl, in[q], kh, a);
+        r = p.pole ? diffusion_pl(G, p.lp, in[q], kh, a, pa) : diffusion7(G, d, cl, in[q], kh, a);
       } else {
-        r = p.pole ? lap_pl(G, p.lp, in[q], a) : lap7(G, d.nreg, p.ci, in[q], a, d.g);
+        r = p.pole ? lap_pl_at(G, p.lp, in[q], pa) : lap7(G, d.nreg, p.ci, in[q], a, d.g);
       }
       out[q][a] = -r;
     }
@@ -397,6 +396,7 @@ struct DivDamp1P {
   Dims d; Consts c; Geo G;
   const real *rvx, *rvy, *rvz, *rw;
   real* out[3];
+  const int* cs;   // source columns of the inputs' halo values (read at the poles)
   NH_HD void operator()(int plane, int x) const {
     Pt p;
     if (!pt_of(d, plane, x, p) || !pt_compute(p)) return;
@@ -409,18 +409,19 @@ struct DivDamp1P {
     auto rwv = [&](long aa, int kk) { return (kk >= kmin + 1 && kk <= kmax) ? (real(0.0) * real(1.0) + rw[aa] * real(1.0)) : real(0.0); };
     if (p.pole) {
       real sclt[5];
+      auto pa = [&](int v, int kk) { return src_pole(d, cs, p.lp, v, kk); };
       const real* vv[3] = {rvx, rvy, rvz};
       for (int v = 1; v <= 5; ++v) {
         const int vp = (v == 5) ? 1 : v + 1;
         real s = real(0.0);
         for (int dd = 0; dd < 3; ++dd) {
           const real* cI = G.cintp_pl + ((v * 2 + p.lp) * 3 + dd) * 3;
-          const real t0 = cI[0] * (vv[dd][a] * real(1.0)), t1 = cI[1] * (vv[dd][a + v] * real(1.0)),
-                       t2 = cI[2] * (vv[dd][a + vp] * real(1.0));
+          const real t0 = cI[0] * (vv[dd][a] * real(1.0)), t1 = cI[1] * (vv[dd][pa(v, k)] * real(1.0)),
+                       t2 = cI[2] * (vv[dd][pa(vp, k)] * real(1.0));
           s = (dd == 0) ? (t0 + t1 + t2) : (s + t0 + t1 + t2);
         }
-        const real up = (rwv(a + ks, k + 1) + rwv(a + v + ks, k + 1) + rwv(a + vp + ks, k + 1));
-        const real dn = (rwv(a, k) + rwv(a + v, k) + rwv(a + vp, k));
+        const real up = (rwv(a + ks, k + 1) + rwv(pa(v, k + 1), k + 1) + rwv(pa(vp, k + 1), k + 1));
+        const real dn = (rwv(a, k) + rwv(pa(v, k), k) + rwv(pa(vp, k), k));
         sclt[v - 1] = s + (up - dn) / real(3.0) * G.rdgz[k];
       }
       for (int dd = 0; dd < 3; ++dd) {
@@ -461,6 +462,7 @@ struct DivDamp2P {
   Dims d; Consts c; Geo G;
   const real* in[3];
   real* out[3];
+  const int* cs;   // source columns of the inputs' halo values (read at the poles)
   NH_HD void operator()(int plane, int x) const {
     Pt p;
     if (!pt_of(d, plane, x, p)) return;
@@ -481,7 +483,8 @@ struct DivDamp2P {
         real s = real(0.0);
         for (int dd = 0; dd < 3; ++dd) {
           const real* cI = G.cintp_pl + ((v * 2 + p.lp) * 3 + dd) * 3;
-          const real t0 = cI[0] * (-in[dd][a]), t1 = cI[1] * (-in[dd][a + v]), t2 = cI[2] * (-in[dd][a + vp]);
+          const real t0 = cI[0] * (-in[dd][a]), t1 = cI[1] * (-in[dd][src_pole(d, cs, p.lp, v, k)]),
+                     t2 = cI[2] * (-in[dd][src_pole(d, cs, p.lp, vp, k)]);
           s = (dd == 0) ? (t0 + t1 + t2) : (s + t0 + t1 + t2);
         }
         sclt[v - 1] = s;
@@ -543,6 +546,7 @@ struct ViPath0P {
   // level, the pressure at the level of its gradient (kmin -> kmin+1)
   static constexpr int kNStage = 5;
   static constexpr bool kStageF32 = false;
+  static constexpr bool kMapped = false;
   NH_HD const real* stage_ptr(int f, int k) const {
     const long NF = d.NF;
     if (f < 3) return prog + (long)(1 + f) * NF;
@@ -805,6 +809,7 @@ struct Path1P {
   // gradient the point needs (stage_shift levels above the point's own)
   static constexpr int kNStage = 1;
   static constexpr bool kStageF32 = true;
+  static constexpr bool kMapped = true;
   Dims d; Consts c; Geo G;
   real dt, rweight;
   const real* prog;
@@ -813,6 +818,7 @@ struct Path1P {
   const real* dd[3];
   real* dv[3];
   real* pm;
+  const int* cs;   // source columns of the split rhoge's halo values
   // level of the gradient for a point at level k: kmin -> kmin+1 (first-layer
   // remedy); the ghost rows use the nearest physical level's value, kmin-1 ->
   // kmin (gradient at kmin+1) and kmax+1 -> kmax
@@ -824,11 +830,13 @@ struct Path1P {
   }
   NH_HD const real* stage_ptr(int, int k) const { return ps[I_RHOGE] + (long)stage_shift(k) * d.g * d.g; }
   NH_HD bool stage_level(int) const { return true; }
+  // the staged field at a column on the edge of its region
+  NH_HD real stage_edge(int, int k, long col) const { return ps[I_RHOGE][src_at(d, cs, col, k + stage_shift(k))]; }
+  // a pole level (the regional points run as staged tiles)
   NH_HD void operator()(int plane, int x) const {
     Pt p;
-    if (!pt_of(d, plane, x, p) || !pt_compute(p)) return;
-    const long sh = (long)stage_shift(p.k) * p.ks;
-    at(p, [&](int, long b) { return ps[I_RHOGE][b + sh]; });
+    if (!pt_of(d, plane, x, p) || !p.pole || p.v != 0) return;
+    at(p, [&](int, long b) { return ps[I_RHOGE][src_pole(d, cs, p.lp, (int)(b - p.a), p.k + stage_shift(p.k))]; });
   }
   // momentum of the small step at level k (column address a); the gradient of
   // the split pressure comes through grad(m, dir)
@@ -909,8 +917,6 @@ struct Path1P {
 // ----------------------------------------------------------------------------
 struct ViMainH {
   static constexpr const char* kName = "vi_main_h";
-  static constexpr int kNStage = 8;    // fields read on the stencil: dv 0..2, eth, ethtot, prog 1..3
-  static constexpr bool kStageF32 = false;
   Dims d; Consts c; Geo G;
   const real* prog;
   const real* dv[3];
@@ -918,14 +924,16 @@ struct ViMainH {
   const real* ethtot;
   const real* gT;
   real* hv[3];
-  NH_HD const real* stage_ptr(int f, int) const {
-    return f < 3 ? dv[f] : (f == 3 ? eth : (f == 4 ? ethtot : prog + (long)(f - 4) * d.NF));
+  const int* cs;   // source columns of dv's halo values
+  // field f at a point of the stencil: address a, of dv am (its halo values' source)
+  NH_HD real stage_val(int f, long a, long am) const {
+    return f < 3 ? dv[f][am] : (f == 3 ? eth[a] : (f == 4 ? ethtot[a] : prog[(long)(f - 4) * d.NF + a]));
   }
-  NH_HD bool stage_level(int k) const { return k >= d.kmin && k <= d.kmax; }
+  // a pole level (the regional points run as ViMainHC)
   NH_HD void operator()(int plane, int x) const {
     Pt p;
-    if (!pt_of(d, plane, x, p) || !pt_compute(p)) return;
-    at(p, [&](int f, long b) { return stage_ptr(f, p.k)[b]; });
+    if (!pt_of(d, plane, x, p) || !p.pole || p.v != 0) return;
+    at(p, [&](int f, long b) { return stage_val(f, b, src_pole(d, cs, p.lp, (int)(b - p.a), p.k)); });
   }
   // ld(f, address): field f of the stencil set at an address of the point's stencil
   template <class LD>

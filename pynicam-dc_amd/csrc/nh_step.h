@@ -24,14 +24,19 @@ NH_HD inline real lap7(const Geo& G, long nreg, long ci, const real* f, long a, 
   return s;
 }
 
-NH_HD inline real lap_pl(const Geo& G, int lp, const real* f, long a0) {
-  // a0: address of pole point v=0 at this level; neighbours at a0 + v
+// ad(v): address of pole point v at this level
+template <class AD>
+NH_HD inline real lap_pl_at(const Geo& G, int lp, const real* f, AD ad) {
   real s = real(0.0);
   for (int v = 0; v < 6; ++v) {
-    real pv = G.clap_pl[v * 2 + lp] * f[a0 + v];
+    real pv = G.clap_pl[v * 2 + lp] * f[ad(v)];
     s = (v == 0) ? pv : s + pv;
   }
   return s;
+}
+NH_HD inline real lap_pl(const Geo& G, int lp, const real* f, long a0) {
+  // a0: address of pole point v=0 at this level; neighbours at a0 + v
+  return lap_pl_at(G, lp, f, [a0](int v) { return a0 + v; });
 }
 
 
@@ -89,16 +94,17 @@ NH_HD inline real diffusion7(const Geo& G, const Dims& d, const Cell& cl, const 
   return inner;
 }
 
-template <class KH>
-NH_HD inline real diffusion_pl(const Geo& G, int lp, const real* s, KH kh, long a0) {
+// s at pole point v is read at ad(v), kh at a0 + v
+template <class KH, class AD>
+NH_HD inline real diffusion_pl(const Geo& G, int lp, const real* s, KH kh, long a0, AD ad) {
   real vt[5][3];
   for (int v = 1; v <= 5; ++v) {
     int vp = (v == 5) ? 1 : v + 1;
     for (int dd = 0; dd < 3; ++dd) {
       const real* cI = G.cintp_pl + ((v * 2 + lp) * 3 + dd) * 3;
       real c0 = cI[0], c1 = cI[1], c2 = cI[2];
-      vt[v - 1][dd] = ((real(2.0) * c0 - c1 - c2) * s[a0] + (-c0 + real(2.0) * c1 - c2) * s[a0 + v]
-                       + (-c0 - c1 + real(2.0) * c2) * s[a0 + vp]) / real(3.0);
+      vt[v - 1][dd] = ((real(2.0) * c0 - c1 - c2) * s[ad(0)] + (-c0 + real(2.0) * c1 - c2) * s[ad(v)]
+                       + (-c0 - c1 + real(2.0) * c2) * s[ad(vp)]) / real(3.0);
     }
   }
   real row = real(0.0);

@@ -86,7 +86,15 @@ struct StagedPointT {
     const int npl = (t.rows + 2) * pk.d.g;
     for (int idx = tid; idx < P::kNStage * npl; idx += 256) {
       const int f = idx / npl, e = idx - f * npl;
-      lds[f * sf() + e] = pk.stage_ptr(f, t.k)[b0 + e];
+      if constexpr (P::kMapped) {
+        // halo columns lie on the region's edge: read them at their source
+        const int g = pk.d.g, r = e / g, i = e - r * g, j = t.j0 - 1 + r;
+        lds[f * sf() + e] = (i == 0 || i == g - 1 || j == 0 || j == g - 1)
+                                ? pk.stage_edge(f, t.k, ((long)t.l * g + j) * g + i)
+                                : pk.stage_ptr(f, t.k)[b0 + e];
+      } else {
+        lds[f * sf() + e] = pk.stage_ptr(f, t.k)[b0 + e];
+      }
     }
   }
   NH_HD void phase1(int, int, real*) const {}
@@ -170,15 +178,53 @@ inline ColGeom col_geom(const Dims& d, int nchunk) {
   return c;
 }
 
-template <int OP>
+// The four points of a corner, (0,0) (+1,0) (+1,+1) (0,+1), at one level.  MAP:
+// each at an offset of its own, halo points at their source (cs); otherwise
+// one offset, the neighbours at constant distances, which lets the compiler
+// pair the loads of (0,0) and (+1,0): with 8-byte fields that is worth 45 us of
+// divdamp_3d's 220 at gl07, with 4-byte fields the four offsets are the faster
+// form (92 against 101 us).
+template <bool MAP>
+struct CornerPts {
+  unsigned a[MAP ? 4 : 1];   // byte offsets (a[0]: the corner's own)
+  NH_HD void init(const Dims& d, const int* cs, int l, int j, int i, int k) {
+    const long col = ((long)l * d.g + j) * d.g + i;
+    if constexpr (MAP) {
+      const int off[4] = {0, 1, 1 + d.g, d.g};
+      for (int n = 0; n < 4; ++n) a[n] = (unsigned)(src_at(d, cs, col + off[n], k) * (long)sizeof(real));
+    } else {
+      a[0] = (unsigned)((((long)(l * d.kall + k) * d.g + j) * d.g + i) * (long)sizeof(real));
+    }
+  }
+  NH_HD real at(const Dims& d, const real* p, int n) const {
+    if constexpr (MAP) return at_off(p, a[n]);
+    else return at_off(p + ((n == 0) ? 0 : (n == 1) ? 1 : (n == 2) ? 1 + d.g : d.g), a[0]);
+  }
+  // one level up
+  NH_HD real up(const Dims& d, const real* p, int n) const {
+    if constexpr (MAP) return at_off(p, a[n] + src_stride_off(d, a[n]));
+    else return at(d, p + (long)d.g * d.g, n);
+  }
+  NH_HD void next(const Dims& d) {
+    if constexpr (MAP) {
+      for (int n = 0; n < 4; ++n) a[n] += src_stride_off(d, a[n]);
+    } else {
+      a[0] += (unsigned)(d.g * d.g * (int)sizeof(real));
+    }
+  }
+};
+
+template <int OP, bool MAP>
 struct DivDampK {
   using LdsT = real;
   static constexpr int kThreads = kColThreads;
   static constexpr const char* kName = (OP == 1) ? "divdamp_3d" : "divdamp_post";
+  static constexpr int kWaves = sizeof(real) == 8 ? 4 : (OP == 1 ? 6 : 7);   // waves per SIMD the registers must leave
   Dims d; Consts c; Geo G; ColGeom cg;
   const real* v[3];     // OP 1: the momentum; OP 2: the first result (negated inside)
   const real* rw;       // OP 1: rhogw
   real* out[3];
+  const int* cs;        // source columns of the inputs' halo values
   static int lds_elems(const ColGeom& cg) { return 4 * (cg.TX + 1) * (cg.TY + 1); }
   struct State {
     real ci[2][9];      // cintp of the corner column, [T][dd * 3 + vertex]
@@ -187,28 +233,26 @@ struct DivDampK {
     real dn[2];         // OP 1: the lower w sums of the two triangles at this level
     real pv[12];        // v at the corners a, a+1, a+1+g, a+g of this level, [dd * 4 + n]
     real pw[4];         // OP 1: rw at the same corners one level up
-    long a;             // the corner's address at this level
+    CornerPts<MAP> pt;  // where the corner's values are read (the tile point's own first)
     int k, lidx;
     bool corner, outp, pent, sgp, have_dn;
   };
   NH_HD bool active(int k) const { return k >= d.kmin && k <= d.kmax; }
   NH_HD void pole(int pb) const {
     if (OP == 1) {
-      DivDamp1P p{d, c, G, v[0], v[1], v[2], rw, {out[0], out[1], out[2]}};
+      DivDamp1P p{d, c, G, v[0], v[1], v[2], rw, {out[0], out[1], out[2]}, cs};
       p(d.lall * d.kall + pb, 0);
     } else {
-      DivDamp2P p{d, c, G, {v[0], v[1], v[2]}, {out[0], out[1], out[2]}};
+      DivDamp2P p{d, c, G, {v[0], v[1], v[2]}, {out[0], out[1], out[2]}, cs};
       p(d.lall * d.kall + pb, 0);
     }
   }
-  // loads of an active level k at the corner address a (k + 1 <= kall - 1)
-  NH_HD void fetch(State& s, long a) const {
-    const long g = d.g;
-    const long off[4] = {0, 1, 1 + g, g};
+  // loads of an active level k (k + 1 <= kall - 1)
+  NH_HD void fetch(State& s) const {
     for (int dd = 0; dd < 3; ++dd)
-      for (int n = 0; n < 4; ++n) s.pv[dd * 4 + n] = v[dd][a + off[n]];
+      for (int n = 0; n < 4; ++n) s.pv[dd * 4 + n] = s.pt.at(d, v[dd], n);
     if (OP == 1)
-      for (int n = 0; n < 4; ++n) s.pw[n] = rw[a + g * g + off[n]];
+      for (int n = 0; n < 4; ++n) s.pw[n] = s.pt.up(d, rw, n);
   }
   // the block's number of levels (uniform over the block)
   NH_HD int init(int blk, int tid, State& s) const {
@@ -231,7 +275,7 @@ struct DivDampK {
     s.lidx = ty * W1 + tx;
     const int i = i0 - 1 + tx, j = j0 - 1 + ty;
     const long nreg = d.nreg, col = ((long)l * g + j) * g + i;
-    s.a = ((long)(l * d.kall + k0) * g + j) * g + i;
+    s.pt.init(d, cs, l, j, i, k0);
     for (int T = 0; T < 2; ++T)
       for (int n = 0; n < 9; ++n) s.ci[T][n] = rc(G.cintp, nreg, n * 2 + T, col);
     if (tx >= 1 && ty >= 1) {
@@ -274,11 +318,10 @@ struct DivDampK {
   }
   NH_HD void level_a(int step, State& s, real* lds) const {
     if (!s.corner) return;
-    const long g = d.g;
     if (active(s.k)) {
       const int P = (cg.TX + 1) * (cg.TY + 1);
       real* buf = lds + (step & 1) * 2 * P;
-      fetch(s, s.a);
+      fetch(s);
       real up[2], dn[2];
       if (OP == 1) {
         wsums(s.pw, s.k + 1, up);
@@ -286,7 +329,7 @@ struct DivDampK {
           dn[0] = s.dn[0];
           dn[1] = s.dn[1];
         } else {
-          const real r[4] = {rw[s.a], rw[s.a + 1], rw[s.a + 1 + g], rw[s.a + g]};
+          const real r[4] = {s.pt.at(d, rw, 0), s.pt.at(d, rw, 1), s.pt.at(d, rw, 2), s.pt.at(d, rw, 3)};
           wsums(r, s.k, dn);
         }
       }
@@ -323,15 +366,15 @@ struct DivDampK {
         }
       }
       if (OP == 1) {
-        for (int dd = 0; dd < 3; ++dd) out[dd][s.a] = act ? o[dd] : real(0.0);
+        for (int dd = 0; dd < 3; ++dd) at_off(out[dd], s.pt.a[0]) = act ? o[dd] : real(0.0);
       } else {
         const real Rr = c.RADIUS;
         const real gd[3] = {c.ALPHA_D * o[0], c.ALPHA_D * o[1], c.ALPHA_D * o[2]};
         const real prd = (gd[0] * s.gx[0] + gd[1] * s.gx[1] + gd[2] * s.gx[2]) / Rr;
-        for (int dd = 0; dd < 3; ++dd) out[dd][s.a] = gd[dd] - prd * s.gx[dd] / Rr;
+        for (int dd = 0; dd < 3; ++dd) at_off(out[dd], s.pt.a[0]) = gd[dd] - prd * s.gx[dd] / Rr;
       }
     }
-    s.a += (long)d.g * d.g;
+    s.pt.next(d);
     s.k += 1;
   }
 };
@@ -344,14 +387,17 @@ struct DivDampK {
 // the Kh-weighted hexagon sums from their 18 held cdiff coefficients.
 // Results equal the point form's (diffusion7, kernels/oprtdiffusion.py:59-177).
 // ----------------------------------------------------------------------------
+template <bool MAP>
 struct DiffKhK {
   using LdsT = real;
   static constexpr int kThreads = kColThreads;
   static constexpr const char* kName = "hdiff_pass2_kh";
+  static constexpr int kWaves = sizeof(real) == 8 ? 3 : 5;
   Dims d; Consts c; Geo G; ColGeom cg;
   const real* in[6];        // the pass's six inputs (fields 4, 5 diffused here)
   real* out[6];
   const real* rhog;
+  const int* cs;            // source columns of the inputs' halo values (rhog holds its own)
   // LDS per buffer: [field f][triangle T][component dd][corner]
   static int lds_elems(const ColGeom& cg) { return 2 * 12 * (cg.TX + 1) * (cg.TY + 1); }
   struct State {
@@ -359,6 +405,7 @@ struct DiffKhK {
     real cd[18];
     real rg[7];         // rhog at the tile point and its neighbours, loaded before the barrier
     long a;
+    CornerPts<MAP> pt;  // where the corner's values are read (the tile point's own first)
     int k, lidx;
     bool corner, outp, pent, sgp;
   };
@@ -367,7 +414,7 @@ struct DiffKhK {
     if (blk >= cg.ntiles) {
       if (tid == 0) {
         HDiffPassP<1> p;
-        p.d = d; p.c = c; p.G = G; p.rhog = rhog;
+        p.d = d; p.c = c; p.G = G; p.rhog = rhog; p.cs = cs;
         for (int q = 0; q < 6; ++q) { p.in[q] = in[q]; p.out[q] = out[q]; }
         p(d.lall * d.kall + (blk - cg.ntiles), 0);
       }
@@ -388,6 +435,7 @@ struct DiffKhK {
     const int i = i0 - 1 + tx, j = j0 - 1 + ty;
     const long nreg = d.nreg, col = ((long)l * g + j) * g + i;
     s.a = ((long)(l * d.kall + k0) * g + j) * g + i;
+    s.pt.init(d, cs, l, j, i, k0);
     for (int T = 0; T < 2; ++T)
       for (int n = 0; n < 9; ++n) s.ci[T][n] = rc(G.cintp, nreg, n * 2 + T, col);
     if (tx >= 1 && ty >= 1) {
@@ -412,7 +460,7 @@ struct DiffKhK {
     }
     for (int f = 0; f < 2; ++f) {
       const real* sf = in[4 + f];
-      const real v00 = sf[s.a], v10 = sf[s.a + 1], v11 = sf[s.a + 1 + g], v01 = sf[s.a + g];
+      const real v00 = s.pt.at(d, sf, 0), v10 = s.pt.at(d, sf, 1), v11 = s.pt.at(d, sf, 2), v01 = s.pt.at(d, sf, 3);
       for (int T = 0; T < 2; ++T) {
         // tri_grad with the held coefficients
         const real s0 = v00, s1 = (T == 0) ? v10 : v11, s2 = (T == 0) ? v11 : v01;
@@ -463,6 +511,7 @@ struct DiffKhK {
       }
     }
     s.a += (long)d.g * d.g;
+    s.pt.next(d);
     s.k += 1;
   }
 };
