@@ -104,7 +104,7 @@ void divdamp_adj(X& x, const Context& ctx, real* const ob[3], real* const vb[4])
 // then the border and pole points
 template <int N, class X>
 void lap_adj(X& x, const Context& ctx, const NegLapGA& l) {
-  const StGeom sg = st_geom(ctx.d, kColChunks);
+  const StGeom sg = st_geom(ctx.d);
   ColStencil<LapTC<N>> cs;
   cs.op.d = ctx.d;
   cs.op.G = ctx.G;

@@ -39,16 +39,16 @@ struct StGeom {
   int nblocks;      // + 2 * kall pole blocks
 };
 
-inline StGeom st_geom(const Dims& d, int nchunk) {
+inline StGeom st_geom(const Dims& d) {
   StGeom c;
   const int W = d.g - 2;
   c.TX = (W < 64) ? W : 64;
   c.TY = (256 / c.TX < W) ? 256 / c.TX : W;
   c.nx = W / c.TX;
   c.ny = W / c.TY;
-  c.nchunk = nchunk;
-  c.KC = (d.kall + nchunk - 1) / nchunk;
-  c.ntiles = d.lall * nchunk * c.nx * c.ny;
+  c.KC = chunk_levels((long)d.lall * c.nx * c.ny, d.kall, kColLevels);
+  c.nchunk = (d.kall + c.KC - 1) / c.KC;
+  c.ntiles = d.lall * c.nchunk * c.nx * c.ny;
   c.nblocks = c.ntiles + 2 * d.kall;
   return c;
 }

@@ -351,10 +351,6 @@ void halo_block(X& x, const Context& ctx, real* base, int nf) {
 
 inline long ncols(const Dims& d) { return d.nreg + 12; }
 
-// level chunks of the column tiles (divergence damping, stencil operators)
-constexpr int kDivDampChunks = 4;
-constexpr int kColChunks = 6;
-
 // ----------------------------------------------------------------------------
 // 3-D divergence damping of (vx, vy, vz, w) into out (3 fields); cs: columns
 // the inputs' halo values are read from.  The second operator reads the first
@@ -367,7 +363,7 @@ void divdamp_op(X& x, const Context& ctx, const real* const v[3], const real* w,
                 bool map) {
   auto run = [&](auto k) {
     k.d = ctx.d; k.c = ctx.c; k.G = ctx.G;
-    k.cg = col_geom(ctx.d, kDivDampChunks);
+    k.cg = col_geom(ctx.d, kDivDampLevels);
     k.rw = w;
     k.cs = cs;
     for (int q = 0; q < 3; ++q) { k.v[q] = v[q]; k.out[q] = out[q]; }
@@ -633,8 +629,8 @@ void hdiff_passes(X& x, const Context& ctx, const real* prog, const real* diag, 
     f.sub[4] = ctx.G.tem_bs;
     f.sub[5] = ctx.G.rho_bs;
   }
-  const ColGeom cg = col_geom(d, kColChunks);
-  const StGeom sg = st_geom(d, kColChunks);
+  const ColGeom cg = col_geom(d, kColLevels);
+  const StGeom sg = st_geom(d);
   const bool direct = ctx.halo_direct && !fill_hda;
   const int* csrc = direct ? ctx.col_src : ctx.col_own;
   {
@@ -704,7 +700,7 @@ void stage_large(X& x, const Context& ctx, real* prog, const real* rhogq, double
     ColStencil<AdvMomC> cs;
     cs.op.pk = AdvMomP{d, ctx.c, ctx.G, prog, diag, gadv};
     cs.op.d = d;
-    cs.cg = st_geom(d, kColChunks);
+    cs.cg = st_geom(d);
     x.run_cols(cs, cs.cg.nblocks, decltype(cs)::lds_elems(cs.cg));
   } else {
     run_staged(x, AdvMomP{d, ctx.c, ctx.G, prog, diag, gadv});
@@ -744,7 +740,7 @@ void small_hv(X& x, const Context& ctx, const real* prog, real* const dv[3], rea
   ColStencil<ViMainHC> cs;
   cs.op.pk = f;
   cs.op.d = ctx.d;
-  cs.cg = st_geom(ctx.d, kColChunks);
+  cs.cg = st_geom(ctx.d);
   cs.cs = ctx.col_src;
   x.run_cols(cs, cs.cg.nblocks, ColStencil<ViMainHC>::lds_elems(cs.cg));
 }

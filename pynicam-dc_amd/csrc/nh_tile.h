@@ -164,16 +164,34 @@ struct ColGeom {
 };
 constexpr int kColThreads = 384;   // (64 + 1) x (4 + 1) corners
 
-inline ColGeom col_geom(const Dims& d, int nchunk) {
+// Levels per chunk of a column-tile kernel.  A block walks its levels one after
+// another (a memory round trip and a barrier each) with its coefficients in
+// registers, so few levels shorten a small grid's kernels, whose blocks all run
+// at once, and many save a large grid's coefficient loads: about 1 + sqrt(tiles
+// x levels) / scale of them, up to most.  Against fixed chunks (7 levels, 11 for
+// the divergence damping, both still the values at gl07 z40) the step takes
+// 2.38 instead of 2.62 ms at gl05 FP64, 1.60 instead of 1.86 mixed; at gl06
+// vi_main_h 34 instead of 40 us mixed.
+struct LevelRule {
+  int scale, most;
+};
+constexpr LevelRule kDivDampLevels{10, 11};   // divergence damping
+constexpr LevelRule kColLevels{27, 7};        // stencil operators, Kh-weighted diffusion
+inline int chunk_levels(long tiles, int kall, const LevelRule& r) {
+  const int k = (int)(1.5 + std::sqrt((double)(tiles * kall)) / r.scale);
+  return (k < r.most) ? k : r.most;
+}
+
+inline ColGeom col_geom(const Dims& d, const LevelRule& rule) {
   ColGeom c;
   const int W = d.g - 2;
   c.TX = (W < 64) ? W : 64;
   c.TY = (256 / c.TX < W) ? 256 / c.TX : W;
   c.nx = W / c.TX;
   c.ny = W / c.TY;
-  c.nchunk = nchunk;
-  c.KC = (d.kall + nchunk - 1) / nchunk;
-  c.ntiles = d.lall * nchunk * c.nx * c.ny;
+  c.KC = chunk_levels((long)d.lall * c.nx * c.ny, d.kall, rule);
+  c.nchunk = (d.kall + c.KC - 1) / c.KC;
+  c.ntiles = d.lall * c.nchunk * c.nx * c.ny;
   c.nblocks = c.ntiles + 2 * d.kall;
   return c;
 }
