@@ -59,7 +59,8 @@ enum WsField {
   W_QOUT = 85,            // 2  limiter outflow bounds
   W_RQ = 87,              // 1  tracer after the horizontal step
   W_HV = 88,              // 3  horizontal divergences of the small-step momentum
-  W_NFIELDS = 91
+  W_KIN = 91,             // 1  kinetic energy of the small-step state
+  W_NFIELDS = 92
 };
 
 // FP64 fields (every form): the tridiagonal matrix, the forward-sweep scratch
@@ -84,6 +85,7 @@ struct Context {
   // the halo map only fills points that are not computed, each once and from
   // a point it does not fill: kernels may read col_src instead of a filled field
   bool halo_direct = false;
+  bool halo_full = false;   // the map fills every column that is not computed
   real* ws = nullptr;
   double* dws = nullptr;
   // adjoint workspace (allocated by the first adjoint call)
@@ -265,7 +267,7 @@ int upload_halo(X& x, Context& ctx, const int32_t* dst, const int32_t* src, long
   if (ctx.halo_src) { x.release(ctx.halo_src); ctx.halo_src = nullptr; }
   if (ctx.col_own) { x.release(ctx.col_own); ctx.col_own = ctx.col_src = nullptr; }
   ctx.halo_n = n;
-  ctx.halo_direct = false;
+  ctx.halo_direct = ctx.halo_full = false;
   // the adjoint of the gather scatters destination bars onto sources in one
   // pass: that needs every destination once and no destination as a source
   {
@@ -292,6 +294,7 @@ int upload_halo(X& x, Context& ctx, const int32_t* dst, const int32_t* src, long
     // every size (step 4.66 -> 4.41 ms at gl06, 13.6 -> 13.3 at gl07); with
     // 8-byte fields the corner kernels lose their paired loads (CornerPts),
     // which pays up to about gl06 (gl05 2.78 -> 2.63 ms) and not at gl07.
+    ctx.halo_full = ok && n == ncol - (long)ctx.d.lall * (g - 2) * (g - 2) - 2;
     ctx.halo_direct = ok && (sizeof(real) == 4 || ctx.d.NF <= kDirectMax64);
   }
   if (n == 0) return 0;
@@ -683,7 +686,7 @@ void hdiff_passes(X& x, const Context& ctx, const real* prog, const real* diag, 
 // start of the mean fluxes
 template <class X>
 void stage_large(X& x, const Context& ctx, real* prog, const real* rhogq, double dts, const StageFields& sf,
-                 bool keep_halo, bool means = true) {
+                 bool keep_halo, real* pm) {
   const Dims& d = ctx.d;
   const long NF = d.NF;
   real* diag = ctx.field(W_DIAG);
@@ -722,7 +725,7 @@ void stage_large(X& x, const Context& ctx, real* prog, const real* rhogq, double
     run_staged(x, f);
   }
   {
-    EthTotPMP f{d, ctx.c, ctx.G, prog, eth, sf.ethtot, means ? ctx.field(W_PM) : nullptr};
+    EthTotPMP f{d, ctx.c, ctx.G, prog, eth, sf.ethtot, pm};
     x.run_pts(f, d);
   }
 }
@@ -746,15 +749,14 @@ void small_hv(X& x, const Context& ctx, const real* prog, real* const dv[3], rea
 }
 
 // one small step (mod_vi.py:1283-1450): divergence damping of the split
-// momentum, path1, vi_main (horizontal, tridiagonal, mass/energy); last: no
-// small step of the stage follows
+// momentum, path1, vi_main (horizontal, tridiagonal, mass/energy); first, last:
+// of its stage; mf: the accumulation of the tracer's mean mass fluxes
 template <class X>
 void small_step(X& x, const Context& ctx, const real* prog, const SmallBufs& s, double dts, double rweight,
-                const StageFields& sf, bool last, bool means = true) {
+                const StageFields& sf, bool first, bool last, const MeanFlux& mf) {
   const Dims& d = ctx.d;
   const long NF = d.NF;
   real* gT = sf.gT;
-  real* pm = means ? ctx.field(W_PM) : nullptr;   // the tracer's mean mass fluxes
   real* ddv = s.ddv ? s.ddv : ctx.field(W_DDV);
   real* hvb = s.hv ? s.hv : ctx.field(W_HV);
   const int* cs = (s.own_halo || !ctx.halo_direct) ? ctx.col_own : ctx.col_src;
@@ -768,7 +770,7 @@ void small_step(X& x, const Context& ctx, const real* prog, const SmallBufs& s, 
     f.gT = gT;
     for (int q = 0; q < 3; ++q) f.dd[q] = ddv + q * NF;
     for (int q = 0; q < 3; ++q) f.dv[q] = s.dv[q];
-    f.pm = pm;
+    f.mf = mf;
     f.cs = cs;
     run_staged(x, f);
   }
@@ -792,17 +794,21 @@ void small_step(X& x, const Context& ctx, const real* prog, const SmallBufs& s, 
     else solve(ViMainV<0>{});
   }
   {
-    ViMainPost f;
-    f.d = d; f.c = ctx.c; f.G = ctx.G;
-    f.dt = (real)dts; f.rweight = (real)rweight;
-    f.prog = prog;
-    for (int q = 0; q < 6; ++q) f.ps[q] = s.ps[q];
-    for (int q = 0; q < 3; ++q) f.dv[q] = s.dv[q];
-    f.ethtot = sf.ethtot; f.gT = gT; f.getot = ctx.field(W_GETOT);
-    for (int q = 0; q < 3; ++q) f.hv[q] = hv[q];
-    for (int q = 0; q < 3; ++q) f.we[q] = s.we[q];
-    f.pm = pm;
-    x.run_pts(f, d);
+    auto post = [&](auto f) {
+      f.d = d; f.c = ctx.c; f.G = ctx.G;
+      f.dt = (real)dts; f.rweight = (real)rweight;
+      f.prog = prog;
+      for (int q = 0; q < 6; ++q) f.ps[q] = s.ps[q];
+      for (int q = 0; q < 3; ++q) f.dv[q] = s.dv[q];
+      f.ethtot = sf.ethtot; f.gT = gT; f.getot = ctx.field(W_GETOT);
+      for (int q = 0; q < 3; ++q) f.hv[q] = hv[q];
+      for (int q = 0; q < 3; ++q) f.we[q] = s.we[q];
+      f.kin = ctx.field(W_KIN);
+      f.mf = mf;
+      x.run_pts(f, d);
+    };
+    if (first) post(ViMainPost<false>{});
+    else post(ViMainPost<true>{});
   }
   // of the outputs' halos only rhogw's and rhoge's are read, by the next small step
   if (!ctx.halo_direct && !last) {
@@ -876,7 +882,11 @@ int dyn_step(X& x, const Context& ctx, real* prog, real* progq, int nq, double d
     if (tape) x.d2d(tp.input(nl), prog, 6 * NF * sizeof(real));
     else if (record) x.d2d(record + (long)nl * 6 * NF, prog, 6 * NF * sizeof(real));
     const StageFields sf = tape ? tp.stage(nl) : ws_stage(ctx);
-    stage_large(x, ctx, prog, progq, dts, sf, tape != nullptr);
+    // the tracer transport reads the last stage's mean fluxes; they start from
+    // the large-step state, copied where the halo map leaves columns out
+    real* pm = ctx.field(W_PM);
+    const bool copy_pm = nl == 2 && !ctx.halo_full;
+    stage_large(x, ctx, prog, progq, dts, sf, tape != nullptr, copy_pm ? pm : nullptr);
     // split state ps[0..5], path1 momentum dv[0..2], vi_main output we[0..2]
     SmallBufs s;
     if (tape) {
@@ -895,17 +905,24 @@ int dyn_step(X& x, const Context& ctx, real* prog, real* progq, int nq, double d
     s.fill_halo = tape != nullptr;
     for (int it = 0; it < nsub[nl]; ++it) {
       s.own_halo = it == 0;
+      // every second small step, counted from the last one
+      MeanFlux mf;
+      if (nl == 2 && (nsub[nl] - it) % 2 == 1) {
+        mf.in = (it <= 1 && !copy_pm) ? prog : pm;
+        mf.out = pm;
+        mf.two = it > 0;
+      }
       if (tape) {
         // outputs straight into the next slot: (we0, dv0, dv1, dv2, we1, we2)
         real* c1 = tp.slot(nl, it + 1);
         s.we[0] = c1; s.dv[0] = c1 + NF; s.dv[1] = c1 + 2 * NF; s.dv[2] = c1 + 3 * NF;
         s.we[1] = c1 + 4 * NF; s.we[2] = c1 + 5 * NF;
         s.hv = tp.slot(nl, it) + 6 * NF;
-        small_step(x, ctx, prog, s, dts, rweight, sf, it == nsub[nl] - 1);
+        small_step(x, ctx, prog, s, dts, rweight, sf, it == 0, it == nsub[nl] - 1, mf);
         for (int q = 0; q < 6; ++q) s.ps[q] = c1 + q * NF;
         continue;
       }
-      small_step(x, ctx, prog, s, dts, rweight, sf, it == nsub[nl] - 1);
+      small_step(x, ctx, prog, s, dts, rweight, sf, it == 0, it == nsub[nl] - 1, mf);
       // rotate buffers: the new split state is (we0, dv0, dv1, dv2, we1, we2)
       real* old[6] = {s.ps[0], s.ps[1], s.ps[2], s.ps[3], s.ps[4], s.ps[5]};
       s.ps[0] = s.we[0]; s.ps[1] = s.dv[0]; s.ps[2] = s.dv[1]; s.ps[3] = s.dv[2]; s.ps[4] = s.we[1];
@@ -913,8 +930,6 @@ int dyn_step(X& x, const Context& ctx, real* prog, real* progq, int nq, double d
       s.we[0] = old[0]; s.dv[0] = old[1]; s.dv[1] = old[2]; s.dv[2] = old[3]; s.we[1] = old[4]; s.we[2] = old[5];
     }
     prog_update(x, ctx, prog, s.ps);
-    // the mean fluxes feed the tracer transport after the last stage; each
-    // stage restarts them at every point (EthTotPMP)
     if (nl == 2) halo_block(x, ctx, ctx.field(W_PM), 5);
     if (nl < 2) halo_block(x, ctx, prog, 6);
     int rc = x.check("dyn_step stage");

@@ -764,6 +764,23 @@ struct ViPath0P {
   }
 };
 
+// The time-mean mass fluxes of a stage, accumulated over its small steps.  A
+// small step reads its input state anyway, which is the previous one's output,
+// so the sums are read and written every second small step with both steps'
+// terms (two), in the order one step at a time adds them; the first time they
+// start from the large-step state itself (in).  Null out: nothing this step.
+// Against one accumulation per small step of every stage (the tracer transport
+// reads the last stage's only), 80 of the 960 field passes of a step are gone.
+struct MeanFlux {
+  const real* in = nullptr;   // rhog, rhogvx, rhogvy, rhogvz, rhogw
+  real* out = nullptr;
+  bool two = false;
+  NH_HD real add(real sum, real prev, real cur, real weight) const {
+    if (two) sum = sum + prev * weight;
+    return sum + cur * weight;
+  }
+};
+
 // total specific energy of the large-step state and the start of the time-mean fluxes
 struct EthTotPMP {
   static constexpr const char* kName = "ethtot_mean";
@@ -817,7 +834,7 @@ struct Path1P {
   const real* gT;
   const real* dd[3];
   real* dv[3];
-  real* pm;
+  MeanFlux mf;
   const int* cs;   // source columns of the split rhoge's halo values
   // level of the gradient for a point at level k: kmin -> kmin+1 (first-layer
   // remedy); the ghost rows use the nearest physical level's value, kmin-1 ->
@@ -888,9 +905,12 @@ struct Path1P {
     };
     // the mass-flux sums are read before any store (a store to dv could alias
     // them for all the compiler knows, which would put each read behind it)
-    real pmq[3] = {real(0.0), real(0.0), real(0.0)};
-    if (pm)
-      for (int q = 0; q < 3; ++q) pmq[q] = pm[(1 + q) * NF + a];
+    real pmq[3] = {real(0.0), real(0.0), real(0.0)}, pmp[3] = {real(0.0), real(0.0), real(0.0)};
+    if (mf.out) {
+      for (int q = 0; q < 3; ++q) pmq[q] = mf.in[(1 + q) * NF + a];
+      if (mf.two)
+        for (int q = 0; q < 3; ++q) pmp[q] = ps[1 + q][a];
+    }
     real v[3];
     if (k >= kmin && k <= kmax) {
       level(p, a, grad, v);
@@ -905,7 +925,7 @@ struct Path1P {
     }
     for (int q = 0; q < 3; ++q) {
       dv[q][a] = v[q];
-      if (pm) pm[(1 + q) * NF + a] = pmq[q] + v[q] * rweight;
+      if (mf.out) mf.out[(1 + q) * NF + a] = mf.add(pmq[q], pmp[q], v[q], rweight);
     }
   }
 };
@@ -1071,6 +1091,11 @@ struct ViMainV {
 
 // mass and energy update of the small step from the new rhogw split, one
 // thread per point (kernels/vimain.py:190-262, rhogkin.py:38-79)
+//
+// kin carries the kinetic energy of the state after a small step to the next
+// one, whose state before it is the same: with KIN it is read instead of formed
+// again from four more fields.
+template <bool KIN>
 struct ViMainPost {
   static constexpr const char* kName = "vi_main_post";
   Dims d; Consts c; Geo G;
@@ -1083,7 +1108,8 @@ struct ViMainPost {
   const real* getot;
   const real* hv[3];
   real* we[3];       // we[1] (rhogw split) is read
-  real* pm;
+  real* kin;         // kinetic energy of the state before (KIN: read) and after (written)
+  MeanFlux mf;
   // Every value the point needs is loaded first, at levels clamped into
   // 0..kall-1 (a clamped level's value is never used: the level tests below
   // are the reference's), so that the loads issue together instead of one
@@ -1114,17 +1140,23 @@ struct ViMainPost {
     for (int j = 0; j < 4; ++j) RW[j] = rw1[A[j]];
     for (int j = 0; j < 2; ++j) {
       P4[j] = prog[4 * NF + A[1 + j]];
-      S4[j] = ps[4][A[1 + j]];
+      if (!KIN) S4[j] = ps[4][A[1 + j]];
     }
     for (int q = 0; q < 3; ++q) {
       PQ[q] = prog[(1 + q) * NF + a];
-      SQ[q] = ps[1 + q][a];
+      if (!KIN) SQ[q] = ps[1 + q][a];
       DQ[q] = dv[q][a];
     }
+    const real kin_in = KIN ? kin[a] : real(0.0);
     const real h2 = hv[2][a], ge = getot[a];
     const int ke = (k < kmin) ? kmin : ((k > kmax) ? kmax : k);
     const real pe_k = ps[I_RHOGE][b + (long)ke * ks];
-    const real pm0 = pm ? pm[0 * NF + a] : real(0.0), pm4 = pm ? pm[4 * NF + a] : real(0.0);
+    real pm0 = real(0.0), pm4 = real(0.0), rw0 = real(0.0);
+    if (mf.out) {
+      pm0 = mf.in[0 * NF + a];
+      pm4 = mf.in[4 * NF + a];
+      if (mf.two) rw0 = ps[4][a];
+    }
     // j: window index of level kk (k - 1 + j)
     auto rs1 = [&](int kk, int j) {
       real drhog2 = real(0.0);
@@ -1147,7 +1179,7 @@ struct ViMainPost {
       if (q == 4) return P4[j - 1] + RW[j];
       return PQ[q - 1] + DQ[q - 1];
     };
-    const real kin10 = rhogkin_k(G, kmin, kmax, k, g10);
+    const real kin10 = KIN ? kin_in : rhogkin_k(G, kmin, kmax, k, g10);
     const real kin11 = rhogkin_k(G, kmin, kmax, k, g11);
     real dtot = real(0.0);
     if (k >= kmin && k <= kmax) {
@@ -1164,9 +1196,10 @@ struct ViMainPost {
     const real re1 = pe_k + (ge + dtot) * dt + (kin10 - kin11) + (S0[1] - r1) * G.phi[k];
     we[0][a] = r1;
     we[2][a] = re1;
-    if (pm) {
-      pm[0 * NF + a] = pm0 + r1 * rweight;
-      pm[4 * NF + a] = pm4 + RW[1] * rweight;
+    kin[a] = kin11;
+    if (mf.out) {
+      mf.out[0 * NF + a] = mf.add(pm0, S0[1], r1, rweight);
+      mf.out[4 * NF + a] = mf.add(pm4, rw0, RW[1], rweight);
     }
   }
 };
