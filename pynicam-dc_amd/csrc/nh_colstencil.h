@@ -16,10 +16,11 @@
 //   kName, kNS (stencil fields), Col (per-column registers), d (Dims),
 //   Stg (registers of the column a thread stages: its own and its ring column),
 //   kMapped (fields read at the source columns cs of their halo values),
+//   Pre (registers a point loads before the barrier) and pre(k, a, Pre&),
 //   init_stage(col index, Stg&), stage_level(k), stage(k, a, am, Stg, v[kNS])
 //   with a the point's address, am its mapped one (a unless kMapped),
 //   init_col(col index, Col&),
-//   point(k, a, Col, nb) with nb(m, f) = field f at stencil neighbour m
+//   point(k, a, Col, Pre, nb) with nb(m, f) = field f at stencil neighbour m
 //   (0 (0,0) 1 (+1,0) 2 (+1,+1) 3 (0,+1) 4 (-1,0) 5 (-1,-1) 6 (0,-1)),
 //   pole(pb): the pole centre of pole level pb (its point kernel).
 #pragma once
@@ -67,6 +68,7 @@ struct ColStencil {
   struct State {
     typename Op::Col col;
     typename Op::Stg sg, rsg;   // staging registers of the own and the ring column
+    typename Op::Pre pre;
     long a, ra;        // own and ring addresses at the current level
     int rm;            // kMapped: the ring point's mapped address
     int k, sidx, ridx;
@@ -117,6 +119,7 @@ struct ColStencil {
     real* buf = lds + (step & 1) * NS * P;
     real v[NS];
     if (s.outp) {
+      op.pre(s.k, s.a, s.pre);
       op.stage(s.k, s.a, s.a, s.sg, v);
       for (int f = 0; f < NS; ++f) buf[f * P + s.sidx] = v[f];
     }
@@ -130,7 +133,7 @@ struct ColStencil {
       const int SW = cg.TX + 2, P = SW * (cg.TY + 2);
       const real* buf = lds + (step & 1) * NS * P;
       const int x = s.sidx;
-      op.point(s.k, s.a, s.col, [&](int m, int f) {
+      op.point(s.k, s.a, s.col, s.pre, [&](int m, int f) {
         const int off = (m == 0) ? 0 : (m == 1) ? 1 : (m == 2) ? 1 + SW : (m == 3) ? SW : (m == 4) ? -1
                       : (m == 5) ? -1 - SW : -SW;
         return buf[f * P + x + off];
@@ -158,7 +161,9 @@ struct ViMainHC {
     real c[3][7];
   };
   struct Stg {};
+  struct Pre {};
   NH_HD void init_stage(long, Stg&) const {}
+  NH_HD void pre(int, long, Pre&) const {}
   NH_HD bool stage_level(int k) const { return k >= d.kmin && k <= d.kmax; }
   NH_HD void stage(int, long a, long am, const Stg&, real* v) const {
     for (int f = 0; f < kNS; ++f) v[f] = pk.stage_val(f, a, am);
@@ -170,7 +175,7 @@ struct ViMainHC {
   NH_HD void pole(int pb) const { pk(d.lall * d.kall + pb, 0); }
   // ViMainH::at with hdiv_multi<3>, term for term
   template <class NB>
-  NH_HD void point(int k, long a, const Col& col, NB nb) const {
+  NH_HD void point(int k, long a, const Col& col, const Pre&, NB nb) const {
     if (k < d.kmin || k > d.kmax) return;
     const long NF = d.NF;
     real s[3][3];
@@ -202,6 +207,92 @@ struct ViMainHC {
   }
 };
 
+// path1 (Path1P) as a column operator: the 21 gradient coefficients and the
+// column's position in registers, the split rhoge staged per level at the
+// level of its gradient; the nine pointwise values are loaded before the
+// barrier, with the staged ones, so that a level waits for memory once.  Bound
+// by HBM traffic (13 fields, 19 where the mean fluxes accumulate): 105 us per
+// launch at gl07 mixed, 196 FP64; as level-staged points, re-reading the 24
+// coefficients per level, 141 and 233; as column tiles with the pointwise loads
+// after the barrier slower than those.
+struct Path1C {
+  static constexpr const char* kName = "vi_path1";
+  static constexpr int kNS = 1;
+  static constexpr bool kMapped = true;
+  Path1P pk;
+  Dims d;
+  struct Col {
+    real c[3][7];
+    real x[3];
+  };
+  struct Stg {};
+  struct Pre {
+    real g[3], dd[3], ps[3];
+  };
+  NH_HD void init_stage(long, Stg&) const {}
+  NH_HD bool stage_level(int) const { return true; }
+  NH_HD void stage(int k, long, long am, const Stg&, real* v) const {
+    v[0] = pk.ps[I_RHOGE][am + (long)pk.stage_shift(k) * src_stride(d, am)];
+  }
+  // address of the physical level a point takes its values from (ghost rows: the nearest)
+  NH_HD long phys(int k, long a) const {
+    const long gg = (long)d.g * d.g;
+    return (k < d.kmin) ? a + gg : (k > d.kmax) ? a - gg : a;
+  }
+  NH_HD void pre(int k, long a, Pre& p) const {
+    const long an = phys(k, a);
+    for (int q = 0; q < 3; ++q) {
+      p.g[q] = pk.gT[(1 + q) * d.NF + an];
+      p.dd[q] = pk.dd[q][an];
+      p.ps[q] = pk.ps[1 + q][an];
+    }
+  }
+  NH_HD void init_col(long ci, Col& col) const {
+    for (int dd = 0; dd < 3; ++dd)
+      for (int m = 0; m < 7; ++m) col.c[dd][m] = rc(pk.G.cgrad, d.nreg, dd * 7 + m, ci);
+    for (int q = 0; q < 3; ++q) col.x[q] = pk.G.gx[q * d.nreg + ci];
+  }
+  NH_HD void pole(int pb) const { pk(d.lall * d.kall + pb, 0); }
+  // Path1P's arithmetic for a regional point
+  template <class NB>
+  NH_HD void point(int k, long a, const Col& col, const Pre& p, NB nb) const {
+    const long NF = d.NF;
+    const int kmin = d.kmin, kmax = d.kmax;
+    const real R = pk.c.RADIUS, RovCV = pk.c.Rdry / pk.c.CVdry;
+    const MeanFlux& mf = pk.mf;
+    real pmq[3] = {real(0.0), real(0.0), real(0.0)}, pmp[3] = {real(0.0), real(0.0), real(0.0)};
+    if (mf.out) {
+      for (int q = 0; q < 3; ++q) pmq[q] = mf.in[(1 + q) * NF + a];
+      if (mf.two)
+        for (int q = 0; q < 3; ++q) pmp[q] = pk.ps[1 + q][a];
+    }
+    real pr[7];
+    for (int m = 0; m < 7; ++m) pr[m] = (nb(m, 0) * RovCV) * real(1.0);
+    real gr[3];
+    for (int dd = 0; dd < 3; ++dd) {
+      real acc = col.c[dd][0] * pr[0];
+      for (int m = 1; m < 7; ++m) acc = acc + col.c[dd][m] * pr[m];
+      gr[dd] = acc + real(0.0);
+    }
+    const real prd = (gr[0] * col.x[0] + gr[1] * col.x[1] + gr[2] * col.x[2]) / R;
+    real v[3];
+    for (int q = 0; q < 3; ++q) {
+      const real Pg = gr[q] - prd * col.x[q] / R;
+      const real drv = p.g[q] - Pg + p.dd[q] + real(0.0);
+      v[q] = p.ps[q] + drv * pk.dt;
+    }
+    if (k < kmin || k > kmax) {
+      // free-slip top / rigid bottom, scaled by the large-step density
+      const real rn = pk.prog[phys(k, a)], ra = pk.prog[a];
+      for (int q = 0; q < 3; ++q) v[q] = (k > kmax) ? real(1.0) * (v[q] / rn) * ra : -real(1.0) * (v[q] / rn) * ra;
+    }
+    for (int q = 0; q < 3; ++q) {
+      pk.dv[q][a] = v[q];
+      if (mf.out) mf.out[(1 + q) * NF + a] = mf.add(pmq[q], pmp[q], v[q], pk.rweight);
+    }
+  }
+};
+
 // minus the 7-point Laplacian of NFLD fields (HDiffPassP's Laplacians) as a
 // column operator: the 7 Laplacian coefficients in registers.  P is the point
 // kernel that does the pole centres (all of its fields) unless pole_off.
@@ -219,7 +310,9 @@ struct LapC {
     real c[7];
   };
   struct Stg {};
+  struct Pre {};
   NH_HD void init_stage(long, Stg&) const {}
+  NH_HD void pre(int, long, Pre&) const {}
   NH_HD bool stage_level(int) const { return true; }
   NH_HD void stage(int k, long, long am, const Stg&, real* v) const {
     for (int f = 0; f < NFLD; ++f) v[f] = pk.input(f, am, k);
@@ -231,7 +324,7 @@ struct LapC {
     if (!pole_off) pk(d.lall * d.kall + pb, 0);
   }
   template <class NB>
-  NH_HD void point(int, long a, const Col& col, NB nb) const {
+  NH_HD void point(int, long a, const Col& col, const Pre&, NB nb) const {
     for (int f = 0; f < NFLD; ++f) {
       real r = col.c[0] * nb(0, f);
 #pragma unroll
@@ -258,7 +351,9 @@ struct LapTC {
     real c[7];
   };
   struct Stg {};
+  struct Pre {};
   NH_HD void init_stage(long, Stg&) const {}
+  NH_HD void pre(int, long, Pre&) const {}
   NH_HD bool stage_level(int) const { return true; }
   NH_HD void stage(int, long a, long, const Stg&, real* v) const {
     for (int f = 0; f < NFLD; ++f) v[f] = ob[f][a];
@@ -276,7 +371,7 @@ struct LapTC {
   }
   NH_HD void pole(int) const {}
   template <class NB>
-  NH_HD void point(int, long a, const Col& col, NB nb) const {
+  NH_HD void point(int, long a, const Col& col, const Pre&, NB nb) const {
     // the source x - off(m) is staged neighbour opp(m)
     const int opp[7] = {0, 4, 5, 6, 1, 2, 3};
     for (int f = 0; f < NFLD; ++f) {
@@ -307,6 +402,8 @@ struct AdvMomC {
   struct Stg {
     real x[3];
   };
+  struct Pre {};
+  NH_HD void pre(int, long, Pre&) const {}
   NH_HD void init_stage(long ci, Stg& sg) const {
     for (int q = 0; q < 3; ++q) sg.x[q] = pk.G.gx[q * d.nreg + ci];
   }
@@ -330,7 +427,7 @@ struct AdvMomC {
   }
   NH_HD void pole(int pb) const { pk(d.lall * d.kall + pb, 0); }
   template <class NB>
-  NH_HD void point(int k, long a, const Col& col, NB nb) const {
+  NH_HD void point(int k, long a, const Col& col, const Pre&, NB nb) const {
     const long NF = d.NF, ks = (long)d.g * d.g;
     const int kmin = d.kmin, kmax = d.kmax;
     real* out = pk.out;

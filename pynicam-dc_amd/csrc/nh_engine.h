@@ -772,7 +772,12 @@ void small_step(X& x, const Context& ctx, const real* prog, const SmallBufs& s, 
     for (int q = 0; q < 3; ++q) f.dv[q] = s.dv[q];
     f.mf = mf;
     f.cs = cs;
-    run_staged(x, f);
+    ColStencil<Path1C> k;
+    k.op.pk = f;
+    k.op.d = d;
+    k.cg = st_geom(d);
+    k.cs = cs;
+    x.run_cols(k, k.cg.nblocks, decltype(k)::lds_elems(k.cg));
   }
   if (s.fill_halo || !ctx.halo_direct) halo(x, ctx, s.dv, 3);
   small_hv(x, ctx, prog, s.dv, hvb, sf);

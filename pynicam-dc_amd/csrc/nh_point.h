@@ -168,8 +168,6 @@ struct AdvMomP {
   static constexpr const char* kName = "adv_mom";
   // fields read on the stencil: vx, vy, vz, w(k), w(k+1), rhogvx, rhogvy, rhogvz
   static constexpr int kNStage = 8;
-  static constexpr bool kStageF32 = false;
-  static constexpr bool kMapped = false;
   Dims d; Consts c; Geo G;
   const real* prog;
   const real* diag;
@@ -545,8 +543,6 @@ struct ViPath0P {
   // fields read on the stencil: rhogvx, rhogvy, rhogvz, eth at the point's
   // level, the pressure at the level of its gradient (kmin -> kmin+1)
   static constexpr int kNStage = 5;
-  static constexpr bool kStageF32 = false;
-  static constexpr bool kMapped = false;
   NH_HD const real* stage_ptr(int f, int k) const {
     const long NF = d.NF;
     if (f < 3) return prog + (long)(1 + f) * NF;
@@ -823,10 +819,8 @@ struct EthTotPMP {
 struct Path1P {
   static constexpr const char* kName = "vi_path1";
   // the split rhoge is read on the stencil, at the level whose pressure
-  // gradient the point needs (stage_shift levels above the point's own)
-  static constexpr int kNStage = 1;
-  static constexpr bool kStageF32 = true;
-  static constexpr bool kMapped = true;
+  // gradient the point needs (stage_shift levels above the point's own).  The
+  // regional points run as column tiles (Path1C), this form the pole centres
   Dims d; Consts c; Geo G;
   real dt, rweight;
   const real* prog;
@@ -845,18 +839,14 @@ struct Path1P {
     if (k == kmax + 1) return -1;
     return 0;
   }
-  NH_HD const real* stage_ptr(int, int k) const { return ps[I_RHOGE] + (long)stage_shift(k) * d.g * d.g; }
-  NH_HD bool stage_level(int) const { return true; }
-  // the staged field at a column on the edge of its region
-  NH_HD real stage_edge(int, int k, long col) const { return ps[I_RHOGE][src_at(d, cs, col, k + stage_shift(k))]; }
-  // a pole level (the regional points run as staged tiles)
+  // a pole level
   NH_HD void operator()(int plane, int x) const {
     Pt p;
     if (!pt_of(d, plane, x, p) || !p.pole || p.v != 0) return;
-    at(p, [&](int, long b) { return ps[I_RHOGE][src_pole(d, cs, p.lp, (int)(b - p.a), p.k + stage_shift(p.k))]; });
+    at(p, [&](int v) { return ps[I_RHOGE][src_pole(d, cs, p.lp, v, p.k + stage_shift(p.k))]; });
   }
   // momentum of the small step at level k (column address a); the gradient of
-  // the split pressure comes through grad(m, dir)
+  // the split pressure comes through grad(dir)
   template <class GR>
   NH_HD void level(const Pt& p, long a, GR grad, real out[3]) const {
     const long NF = d.NF;
@@ -865,52 +855,28 @@ struct Path1P {
     for (int dd2 = 0; dd2 < 3; ++dd2) gr[dd2] = grad(dd2);
     for (int q = 0; q < 3; ++q) gr[q] = gr[q] + real(0.0);
     real Pg[3];
-    if (p.pole) {
-      const real gx = G.gx_pl[p.lp * 3 + 0], gy = G.gx_pl[p.lp * 3 + 1], gz = G.gx_pl[p.lp * 3 + 2];
-      const real prd = gr[0] * gx / R + gr[1] * gy / R + gr[2] * gz / R;
-      Pg[0] = gr[0] - prd * gx / R; Pg[1] = gr[1] - prd * gy / R; Pg[2] = gr[2] - prd * gz / R;
-    } else {
-      const real gx = G.gx[p.ci], gy = G.gx[d.nreg + p.ci], gz = G.gx[2 * d.nreg + p.ci];
-      const real prd = (gr[0] * gx + gr[1] * gy + gr[2] * gz) / R;
-      Pg[0] = gr[0] - prd * gx / R; Pg[1] = gr[1] - prd * gy / R; Pg[2] = gr[2] - prd * gz / R;
-    }
+    const real gx = G.gx_pl[p.lp * 3 + 0], gy = G.gx_pl[p.lp * 3 + 1], gz = G.gx_pl[p.lp * 3 + 2];
+    const real prd = gr[0] * gx / R + gr[1] * gy / R + gr[2] * gz / R;
+    Pg[0] = gr[0] - prd * gx / R; Pg[1] = gr[1] - prd * gy / R; Pg[2] = gr[2] - prd * gz / R;
     for (int q = 0; q < 3; ++q) {
       const real drv = gT[(1 + q) * NF + a] - Pg[q] + dd[q][a] + real(0.0);
       out[q] = ps[1 + q][a] + drv * dt;
     }
   }
-  // ld(0, address on the point's level): split rhoge at the gradient's level
+  // ld(v): split rhoge of pole point v at the gradient's level
   template <class LD>
   NH_HD void at(const Pt& p, LD ld) const {
     const long NF = d.NF, a = p.a, ks = p.ks;
     const int kmin = d.kmin, kmax = d.kmax, k = p.k;
     const real RovCV = c.Rdry / c.CVdry;
     auto grad = [&](int dd2) {
-      real acc;
-      if (p.pole) {
-        acc = real(0.0);
-        for (int v = 0; v < 6; ++v) {
-          const real pv = G.cgrad_pl[(v * 2 + p.lp) * 3 + dd2] * ((ld(0, a + v) * RovCV) * real(1.0) * real(1.0));
-          acc = (v == 0) ? pv : acc + pv;
-        }
-      } else {
-        const long g = d.g;
-        acc = rc(G.cgrad, d.nreg, dd2 * 7, p.ci) * ((ld(0, a) * RovCV) * real(1.0));
-        for (int m = 1; m < 7; ++m) {
-          const long off = (((4201 >> (2 * m)) & 3) - 1) + (((421 >> (2 * m)) & 3) - 1) * g;
-          acc = acc + rc(G.cgrad, d.nreg, dd2 * 7 + m, p.ci) * ((ld(0, a + off) * RovCV) * real(1.0));
-        }
+      real acc = real(0.0);
+      for (int v = 0; v < 6; ++v) {
+        const real pv = G.cgrad_pl[(v * 2 + p.lp) * 3 + dd2] * ((ld(v) * RovCV) * real(1.0) * real(1.0));
+        acc = (v == 0) ? pv : acc + pv;
       }
       return acc;
     };
-    // the mass-flux sums are read before any store (a store to dv could alias
-    // them for all the compiler knows, which would put each read behind it)
-    real pmq[3] = {real(0.0), real(0.0), real(0.0)}, pmp[3] = {real(0.0), real(0.0), real(0.0)};
-    if (mf.out) {
-      for (int q = 0; q < 3; ++q) pmq[q] = mf.in[(1 + q) * NF + a];
-      if (mf.two)
-        for (int q = 0; q < 3; ++q) pmp[q] = ps[1 + q][a];
-    }
     real v[3];
     if (k >= kmin && k <= kmax) {
       level(p, a, grad, v);
@@ -924,8 +890,9 @@ struct Path1P {
       for (int q = 0; q < 3; ++q) v[q] = top ? real(1.0) * (vn[q] / rg[an]) * rg[a] : -real(1.0) * (vn[q] / rg[an]) * rg[a];
     }
     for (int q = 0; q < 3; ++q) {
+      const real pmq = mf.out ? mf.in[(1 + q) * NF + a] : real(0.0);
       dv[q][a] = v[q];
-      if (mf.out) mf.out[(1 + q) * NF + a] = mf.add(pmq[q], pmp[q], v[q], rweight);
+      if (mf.out) mf.out[(1 + q) * NF + a] = mf.add(pmq, mf.two ? ps[1 + q][a] : real(0.0), v[q], rweight);
     }
   }
 };

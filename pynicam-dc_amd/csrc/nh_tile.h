@@ -86,15 +86,7 @@ struct StagedPointT {
     const int npl = (t.rows + 2) * pk.d.g;
     for (int idx = tid; idx < P::kNStage * npl; idx += 256) {
       const int f = idx / npl, e = idx - f * npl;
-      if constexpr (P::kMapped) {
-        // halo columns lie on the region's edge: read them at their source
-        const int g = pk.d.g, r = e / g, i = e - r * g, j = t.j0 - 1 + r;
-        lds[f * sf() + e] = (i == 0 || i == g - 1 || j == 0 || j == g - 1)
-                                ? pk.stage_edge(f, t.k, ((long)t.l * g + j) * g + i)
-                                : pk.stage_ptr(f, t.k)[b0 + e];
-      } else {
-        lds[f * sf() + e] = pk.stage_ptr(f, t.k)[b0 + e];
-      }
+      lds[f * sf() + e] = pk.stage_ptr(f, t.k)[b0 + e];
     }
   }
   NH_HD void phase1(int, int, real*) const {}
@@ -122,10 +114,10 @@ struct StagedPointT {
 
 // Staging pays where the stencil loads are 8-byte (the FP64 form: 10-20 %
 // faster on MI355X at gl07); with 4-byte fields the direct point kernel is as
-// fast or faster, except for kernels that set P::kStageF32.
+// fast or faster.
 template <class X, class P>
 void run_staged(X& x, const P& pk) {
-  if (sizeof(real) == sizeof(float) && !P::kStageF32) {
+  if (sizeof(real) == sizeof(float)) {
     x.run_pts(pk, pk.d);
     return;
   }
