@@ -16,7 +16,8 @@
 //   kName, kNS (stencil fields), Col (per-column registers), d (Dims),
 //   Stg (registers of the column a thread stages: its own and its ring column),
 //   kMapped (fields read at the source columns cs of their halo values),
-//   Pre (registers a point loads before the barrier) and pre(k, a, Pre&),
+//   Pre (registers a point keeps from level to level or loads before the
+//   barrier), begin(Pre&) at the start of a chunk and pre(k, a, Pre&) per level,
 //   init_stage(col index, Stg&), stage_level(k), stage(k, a, am, Stg, v[kNS])
 //   with a the point's address, am its mapped one (a unless kMapped),
 //   init_col(col index, Col&),
@@ -97,6 +98,7 @@ struct ColStencil {
       s.a = ((long)(l * d.kall + k0) * g + j) * g + i;
       op.init_col(((long)l * g + j) * g + i, s.col);
       op.init_stage(((long)l * g + j) * g + i, s.sg);
+      op.begin(s.pre);
     }
     // the ring: row -1 (x = -1..TX-1), row TY (x = 0..TX), columns -1 and TX (y = 0..TY-1)
     if (tid < 2 * TX + 2 * TY + 2) {
@@ -114,12 +116,12 @@ struct ColStencil {
     return k1 - k0;
   }
   NH_HD void level_a(int step, State& s, real* lds) const {
+    if (s.outp) op.pre(s.k, s.a, s.pre);
     if (!op.stage_level(s.k)) return;
     const int SW = cg.TX + 2, P = SW * (cg.TY + 2);
     real* buf = lds + (step & 1) * NS * P;
     real v[NS];
     if (s.outp) {
-      op.pre(s.k, s.a, s.pre);
       op.stage(s.k, s.a, s.a, s.sg, v);
       for (int f = 0; f < NS; ++f) buf[f * P + s.sidx] = v[f];
     }
@@ -163,6 +165,7 @@ struct ViMainHC {
   struct Stg {};
   struct Pre {};
   NH_HD void init_stage(long, Stg&) const {}
+  NH_HD void begin(Pre&) const {}
   NH_HD void pre(int, long, Pre&) const {}
   NH_HD bool stage_level(int k) const { return k >= d.kmin && k <= d.kmax; }
   NH_HD void stage(int, long a, long am, const Stg&, real* v) const {
@@ -175,7 +178,7 @@ struct ViMainHC {
   NH_HD void pole(int pb) const { pk(d.lall * d.kall + pb, 0); }
   // ViMainH::at with hdiv_multi<3>, term for term
   template <class NB>
-  NH_HD void point(int k, long a, const Col& col, const Pre&, NB nb) const {
+  NH_HD void point(int k, long a, const Col& col, Pre&, NB nb) const {
     if (k < d.kmin || k > d.kmax) return;
     const long NF = d.NF;
     real s[3][3];
@@ -239,6 +242,7 @@ struct Path1C {
     const long gg = (long)d.g * d.g;
     return (k < d.kmin) ? a + gg : (k > d.kmax) ? a - gg : a;
   }
+  NH_HD void begin(Pre&) const {}
   NH_HD void pre(int k, long a, Pre& p) const {
     const long an = phys(k, a);
     for (int q = 0; q < 3; ++q) {
@@ -255,7 +259,7 @@ struct Path1C {
   NH_HD void pole(int pb) const { pk(d.lall * d.kall + pb, 0); }
   // Path1P's arithmetic for a regional point
   template <class NB>
-  NH_HD void point(int k, long a, const Col& col, const Pre& p, NB nb) const {
+  NH_HD void point(int k, long a, const Col& col, Pre& p, NB nb) const {
     const long NF = d.NF;
     const int kmin = d.kmin, kmax = d.kmax;
     const real R = pk.c.RADIUS, RovCV = pk.c.Rdry / pk.c.CVdry;
@@ -293,6 +297,214 @@ struct Path1C {
   }
 };
 
+// the large-step source terms and the tridiagonal matrix (ViPath0P) as a column
+// operator: the 42 divergence and gradient coefficients in registers, the
+// momentum, eth and the pressure staged per level.  A column marches upward and
+// carries what levels k and k + 1 share (the effective gravity of the half
+// levels, with its divisions, in both precisions, and eth at half levels), where
+// the point form forms each three times; all loads of a level go out before
+// its barrier.
+struct ViPath0C {
+  static constexpr const char* kName = "vi_path0";
+  static constexpr int kNS = 5;
+  static constexpr bool kMapped = false;
+  ViPath0P pk;
+  Dims d;
+  struct Col {
+    real cd[3][7], cg[3][7];
+    real x[3];
+  };
+  struct Stg {};
+  struct Pre {
+    bool have;
+    real rgm, rg0, rg1, pr0, pr1, et0, et1, rw0, rw1;   // levels k-1, k, k+1
+    real dp0, db0, g0, es0;              // half level k: pressure force, buoyancy, gravity, eth
+    double gm64, g064, em64, e064;       // half levels k-1, k in FP64: gravity, eth
+    real vt[6], ga[3], ga3, ga3m, dd[3], vd[3];
+  };
+  NH_HD void init_stage(long, Stg&) const {}
+  NH_HD void begin(Pre& p) const { p.have = false; }
+  NH_HD bool stage_level(int k) const { return k >= d.kmin && k <= d.kmax; }
+  NH_HD void stage(int k, long a, long, const Stg&, real* v) const {
+    const unsigned o = byte_off(a);
+    for (int q = 0; q < 3; ++q) v[q] = at_off(pk.prog + (long)(1 + q) * d.NF, o);
+    v[3] = at_off(pk.eth, o);
+    // the pressure at the level of its gradient (kmin -> kmin+1), pregd
+    const int kg = (k == d.kmin) ? k + 1 : k;
+    v[4] = (real)((double)at_off(pk.diag + I_PRE * d.NF + (long)(kg - k) * d.g * d.g, o) - pk.G.pre_bs[kg]) * real(1.0);
+  }
+  NH_HD void init_col(long ci, Col& col) const {
+    for (int dd = 0; dd < 3; ++dd)
+      for (int m = 0; m < 7; ++m) {
+        col.cd[dd][m] = rc(pk.G.cdiv, d.nreg, dd * 7 + m, ci);
+        col.cg[dd][m] = rc(pk.G.cgrad, d.nreg, dd * 7 + m, ci);
+      }
+    for (int q = 0; q < 3; ++q) col.x[q] = pk.G.gx[q * d.nreg + ci];
+  }
+  NH_HD void pole(int pb) const { pk(d.lall * d.kall + pb, 0); }
+  // vertical pressure force, buoyancy and effective gravity at half level kk
+  // from rhog and the pressure at kk and kk-1 (ViPath0P's dpgw, dbuo, gzt)
+  template <class T>
+  NH_HD void half(const VProf<T>& V, T grav, int kk, T rg, T rgl, double pr, double prl, double rgd, double rgld,
+                  T& dp, T& db, T& g) const {
+    const bool in = kk >= d.kmin + 1 && kk <= d.kmax;
+    const Geo& G = pk.G;
+    const int k1 = in ? kk : d.kmin + 1;   // a level both profiles have, unused otherwise
+    const T prd = (T)(pr - G.pre_bs[k1]) * T(1.0), prdl = (T)(prl - G.pre_bs[k1 - 1]) * T(1.0);
+    const T rd = (T)(rgd - G.rho_bs[k1]) * T(1.0), rdl = (T)(rgld - G.rho_bs[k1 - 1]) * T(1.0);
+    dp = in ? T(1.0) * (prd * T(1.0) - prdl * T(1.0)) * V.rdgzh[k1] : T(0.0);
+    db = in ? -grav * (V.c2w0[k1] * rd + V.c2w1[k1] * rdl) : T(0.0);
+    const int k2 = (kk < d.kmin) ? d.kmin : (kk > d.kall - 1) ? d.kall - 1 : kk;
+    g = grav - (dp - db) / (V.c2w0[k2] * rg + V.c2w1[k2] * rgl);
+  }
+  NH_HD void half_both(int kk, real rg, real rgl, real pr, real prl, real& dp, real& db, real& g, double& g64) const {
+    half<real>(pk.G, pk.c.GRAV, kk, rg, rgl, (double)pr, (double)prl, (double)(rg / real(1.0)),
+               (double)(rgl / real(1.0)), dp, db, g);
+    if constexpr (sizeof(real) == 8) {
+      g64 = g;
+    } else {
+      double a, b;
+      half<double>(pk.G.v64, pk.c.d.GRAV, kk, (double)rg, (double)rgl, (double)pr, (double)prl, (double)rg, (double)rgl,
+                   a, b, g64);
+    }
+  }
+  NH_HD double eth64(int kk, real e, real el) const {
+    const VProf<double>& V = pk.G.v64;
+    const int k2 = (kk < d.kmin) ? d.kmin : (kk > d.kall - 1) ? d.kall - 1 : kk;
+    return V.afact[k2] * (double)e + V.bfact[k2] * (double)el;
+  }
+  NH_HD real eth_h(int kk, real e, real el) const {
+    const int k2 = (kk > d.kall - 1) ? d.kall - 1 : kk;
+    return pk.G.afact[k2] * e + pk.G.bfact[k2] * el;
+  }
+  NH_HD void pre(int k, long a, Pre& p) const {
+    const long NF = d.NF, gg = (long)d.g * d.g;
+    const real* rg = pk.prog;
+    const real* rw = pk.prog + 4 * NF;
+    const real* pr = pk.diag + I_PRE * NF;
+    const unsigned o = byte_off(a);
+    if (p.have) {
+      p.rgm = p.rg0; p.rg0 = p.rg1;
+      p.pr0 = p.pr1; p.et0 = p.et1; p.rw0 = p.rw1;
+      p.ga3m = p.ga3;
+    } else {
+      // levels k-2, k-1, k, clamped into range (a clamped value is not used)
+      const long m1 = (k > 0) ? -gg : 0, m2 = (k > 1) ? m1 - gg : m1;
+      const real rg2 = at_off(rg + m2, o), pr2 = at_off(pr + m2, o), et2 = at_off(pk.eth + m2, o);
+      const real prm = at_off(pr + m1, o), etm = at_off(pk.eth + m1, o);
+      p.rgm = at_off(rg + m1, o); p.rg0 = at_off(rg, o);
+      p.pr0 = at_off(pr, o); p.et0 = at_off(pk.eth, o); p.rw0 = at_off(rw, o);
+      p.ga3m = at_off(pk.gadv + 3 * NF + m1, o);
+      real dp, db, g;
+      half_both(k - 1, p.rgm, rg2, prm, pr2, dp, db, g, p.gm64);
+      half_both(k, p.rg0, p.rgm, p.pr0, prm, p.dp0, p.db0, p.g0, p.g064);
+      p.em64 = eth64(k - 1, etm, et2);
+      p.e064 = eth64(k, p.et0, etm);
+      p.es0 = eth_h(k, p.et0, etm);
+      p.have = true;
+    }
+    const long up = (k < d.kall - 1) ? gg : 0;
+    p.rg1 = at_off(rg + up, o); p.pr1 = at_off(pr + up, o); p.et1 = at_off(pk.eth + up, o); p.rw1 = at_off(rw + up, o);
+    for (int q = 0; q < 6; ++q) p.vt[q] = at_off(pk.vt[q], o);
+    for (int q = 0; q < 3; ++q) {
+      p.ga[q] = at_off(pk.gadv + q * NF, o);
+      p.dd[q] = at_off(pk.dd[q], o);
+      p.vd[q] = at_off(pk.diag + (I_VX + q) * NF, o);
+    }
+    p.ga3 = at_off(pk.gadv + 3 * NF, o);
+  }
+  // ViPath0P::at for a regional point, term for term
+  template <class NB>
+  NH_HD void point(int k, long a, const Col& col, Pre& p, NB nb) const {
+    const long NF = d.NF;
+    const unsigned o = byte_off(a);
+    const int kmin = d.kmin, kmax = d.kmax;
+    const Geo& G = pk.G;
+    const real R = pk.c.RADIUS;
+    const real gx = col.x[0], gy = col.x[1], gz = col.x[2];
+    const real Kh = pk.c.GAMMA_H;
+    real dp1, db1, g1;
+    double g164;
+    half_both(k + 1, p.rg1, p.rg0, p.pr1, p.pr0, dp1, db1, g1, g164);
+    const double e164 = eth64(k + 1, p.et1, p.et0);
+    const real es1 = eth_h(k + 1, p.et1, p.et0);
+    // hyperdiffusion tendency + momentum advection = large-step tendency
+    real fvx = -(p.vt[0] * Kh + real(0.0)) * p.rg0;
+    real fvy = -(p.vt[1] * Kh + real(0.0)) * p.rg0;
+    real fvz = -(p.vt[2] * Kh + real(0.0)) * p.rg0;
+    const real rgh = (k >= kmin) ? G.c2w0[k] * p.rg0 + G.c2w1[k] * p.rgm : real(0.0);
+    const real fw = -(p.vt[3] * Kh + real(0.0)) * rgh;
+    const real fe = -(p.vt[4] + real(0.0));
+    const real fr = -(p.vt[5] + real(0.0));
+    {
+      const real prd = (fvx * gx + fvy * gy + fvz * gz) / R;
+      fvx = fvx - prd * gx / R; fvy = fvy - prd * gy / R; fvz = fvz - prd * gz / R;
+    }
+    const real gadv_w = (k > kmin && k <= kmax) ? (G.c2w0[k] * p.ga3 + G.c2w1[k] * p.ga3m) : real(0.0);
+    const real g00 = real(0.0) + fr, g05 = real(0.0) + fe;
+    const real g01 = p.ga[0] + fvx, g02 = p.ga[1] + fvy, g03 = p.ga[2] + fvz;
+    const real g04 = gadv_w + fw;
+    real drhog = real(0.0), drhoge = real(0.0), pw = real(0.0);
+    real dpg[3] = {real(0.0), real(0.0), real(0.0)};
+    if (k >= kmin && k <= kmax) {
+      // div(rhogv), div(rhogv eth) and the pressure gradient
+      real s[2][3], gr[3];
+#pragma unroll
+      for (int m = 0; m < 7; ++m) {
+        const real e = nb(m, 3), pm = nb(m, 4) * real(1.0);
+        for (int q = 0; q < 3; ++q) {
+          const real r3 = nb(m, q);
+          const real t0 = col.cd[q][m] * (r3 * real(1.0)), t1 = col.cd[q][m] * (r3 * e * real(1.0));
+          const real tg = col.cg[q][m] * pm;
+          s[0][q] = (m == 0) ? t0 : s[0][q] + t0;
+          s[1][q] = (m == 0) ? t1 : s[1][q] + t1;
+          gr[q] = (m == 0) ? tg : gr[q] + tg;
+        }
+      }
+      const real hd = s[0][0] + s[0][1] + s[0][2], he = s[1][0] + s[1][1] + s[1][2];
+      const real vmh_hi = (k + 1 <= kmax) ? real(0.0) * real(1.0) + real(1.0) * p.rw1 * real(1.0) : real(0.0);
+      const real vmh_lo = (k >= kmin + 1) ? real(0.0) * real(1.0) + real(1.0) * p.rw0 * real(1.0) : real(0.0);
+      drhog = -hd - (vmh_hi - vmh_lo) * G.rdgz[k];
+      const real ws_hi = (k + 1 <= kmax) ? real(0.0) * real(1.0) + real(1.0) * (p.rw1 * es1) * real(1.0) : real(0.0);
+      const real ws_lo = (k >= kmin + 1) ? real(0.0) * real(1.0) + real(1.0) * (p.rw0 * p.es0) * real(1.0) : real(0.0);
+      drhoge = -he - (ws_hi - ws_lo) * G.rdgz[k];
+      for (int q = 0; q < 3; ++q) gr[q] = gr[q] + real(0.0);
+      const real prd = (gr[0] * gx + gr[1] * gy + gr[2] * gz) / R;
+      dpg[0] = gr[0] - prd * gx / R;
+      dpg[1] = gr[1] - prd * gy / R;
+      dpg[2] = gr[2] - prd * gz / R;
+      pw = p.vd[0] * dpg[0] + p.vd[1] * dpg[1] + p.vd[2] * dpg[2] + G.w2c0[k] * (-g1 * p.rw1)
+         + G.w2c1[k] * (-p.g0 * p.rw0);
+    }
+    at_off(pk.getot, o) = g05;
+    at_off(pk.frhog, o) = g00;
+    at_off(pk.gT + 0 * NF, o) = g00 + drhog;
+    at_off(pk.gT + 1 * NF, o) = g01 - dpg[0] + p.dd[0] + real(0.0);
+    at_off(pk.gT + 2 * NF, o) = g02 - dpg[1] + p.dd[1] + real(0.0);
+    at_off(pk.gT + 3 * NF, o) = g03 - dpg[2] + p.dd[2] + real(0.0);
+    at_off(pk.gT + 4 * NF, o) = g04 + real(0.0) * pk.c.ALPHA - p.dp0 + p.db0;
+    at_off(pk.gT + 5 * NF, o) = g05 + drhoge + pw;
+    if (k >= kmin + 1 && k <= kmax) {
+      const VProf<double>& V = G.v64;
+      const ConstsT<double>& C = pk.c.d;
+      const double GCVovR = C.GRAV * C.CVdry / C.Rdry;
+      const double ACVovRt2 = C.ALPHA * C.CVdry / C.Rdry / (pk.dt * pk.dt);
+      const double Ca = (1.0 * V.rdgz[k] + 1.0 * V.rdgz[k - 1]) * 1.0;
+      const double Cb = V.dfact[k] - V.cfact[k - 1];
+      const double Cu1 = 1.0 * V.rdgz[k] * 1.0;
+      const double Cu2 = 1.0 * 1.0 * GCVovR;
+      const double Cl1 = 1.0 * V.rdgz[k] * 1.0;
+      const double Cl2 = 1.0 * 1.0 * GCVovR;
+      pk.Mc[a] = ACVovRt2 / 1.0 + V.rdgzh[k] * (Ca * p.e064 - Cb * (p.g064 + GCVovR));
+      pk.Mu[a] = -V.rdgzh[k] * (Cu1 * e164 + V.cfact[k] * (g164 + Cu2));
+      pk.Ml[a] = -V.rdgzh[k] * (Cl1 * p.em64 - V.dfact[k - 1] * (p.gm64 + Cl2));
+    }
+    p.dp0 = dp1; p.db0 = db1; p.g0 = g1; p.es0 = es1;
+    p.gm64 = p.g064; p.g064 = g164;
+    p.em64 = p.e064; p.e064 = e164;
+  }
+};
+
 // minus the 7-point Laplacian of NFLD fields (HDiffPassP's Laplacians) as a
 // column operator: the 7 Laplacian coefficients in registers.  P is the point
 // kernel that does the pole centres (all of its fields) unless pole_off.
@@ -312,6 +524,7 @@ struct LapC {
   struct Stg {};
   struct Pre {};
   NH_HD void init_stage(long, Stg&) const {}
+  NH_HD void begin(Pre&) const {}
   NH_HD void pre(int, long, Pre&) const {}
   NH_HD bool stage_level(int) const { return true; }
   NH_HD void stage(int k, long, long am, const Stg&, real* v) const {
@@ -324,7 +537,7 @@ struct LapC {
     if (!pole_off) pk(d.lall * d.kall + pb, 0);
   }
   template <class NB>
-  NH_HD void point(int, long a, const Col& col, const Pre&, NB nb) const {
+  NH_HD void point(int, long a, const Col& col, Pre&, NB nb) const {
     for (int f = 0; f < NFLD; ++f) {
       real r = col.c[0] * nb(0, f);
 #pragma unroll
@@ -353,6 +566,7 @@ struct LapTC {
   struct Stg {};
   struct Pre {};
   NH_HD void init_stage(long, Stg&) const {}
+  NH_HD void begin(Pre&) const {}
   NH_HD void pre(int, long, Pre&) const {}
   NH_HD bool stage_level(int) const { return true; }
   NH_HD void stage(int, long a, long, const Stg&, real* v) const {
@@ -371,7 +585,7 @@ struct LapTC {
   }
   NH_HD void pole(int) const {}
   template <class NB>
-  NH_HD void point(int, long a, const Col& col, const Pre&, NB nb) const {
+  NH_HD void point(int, long a, const Col& col, Pre&, NB nb) const {
     // the source x - off(m) is staged neighbour opp(m)
     const int opp[7] = {0, 4, 5, 6, 1, 2, 3};
     for (int f = 0; f < NFLD; ++f) {
@@ -403,6 +617,7 @@ struct AdvMomC {
     real x[3];
   };
   struct Pre {};
+  NH_HD void begin(Pre&) const {}
   NH_HD void pre(int, long, Pre&) const {}
   NH_HD void init_stage(long ci, Stg& sg) const {
     for (int q = 0; q < 3; ++q) sg.x[q] = pk.G.gx[q * d.nreg + ci];
@@ -427,7 +642,7 @@ struct AdvMomC {
   }
   NH_HD void pole(int pb) const { pk(d.lall * d.kall + pb, 0); }
   template <class NB>
-  NH_HD void point(int k, long a, const Col& col, const Pre&, NB nb) const {
+  NH_HD void point(int k, long a, const Col& col, Pre&, NB nb) const {
     const long NF = d.NF, ks = (long)d.g * d.g;
     const int kmin = d.kmin, kmax = d.kmax;
     real* out = pk.out;

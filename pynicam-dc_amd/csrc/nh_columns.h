@@ -61,6 +61,7 @@ NH_HD inline T ldc(const T* p) {
 // addresses the same point of every field (the loads take the base from scalar
 // registers).  A field is below 4 GiB: 64 fields of that size already exceed
 // the card's memory.
+NH_HD inline unsigned byte_off(long a) { return (unsigned)a * (unsigned)sizeof(real); }
 template <class T>
 NH_HD inline const T& at_off(const T* p, unsigned off) {
   return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(p) + off);

@@ -722,7 +722,11 @@ void stage_large(X& x, const Context& ctx, real* prog, const real* rhogq, double
     f.gT = sf.gT;
     f.Mc = sf.M; f.Mu = sf.M + NF; f.Ml = sf.M + 2 * NF;
     f.getot = ctx.field(W_GETOT); f.frhog = ctx.field(W_FRHOG);
-    run_staged(x, f);
+    ColStencil<ViPath0C> k;
+    k.op.pk = f;
+    k.op.d = d;
+    k.cg = st_geom(d);
+    x.run_cols(k, k.cg.nblocks, decltype(k)::lds_elems(k.cg));
   }
   {
     EthTotPMP f{d, ctx.c, ctx.G, prog, eth, sf.ethtot, pm};
