@@ -17,11 +17,13 @@
 //   Stg (registers of the column a thread stages: its own and its ring column),
 //   kMapped (fields read at the source columns cs of their halo values),
 //   Pre (registers a point keeps from level to level or loads before the
-//   barrier), begin(Pre&) at the start of a chunk and pre(k, a, Pre&) per level,
-//   init_stage(col index, Stg&), stage_level(k), stage(k, a, am, Stg, v[kNS])
-//   with a the point's address, am its mapped one (a unless kMapped),
+//   barrier), begin(Pre&) at the start of a chunk and pre(k, o, Stg, Pre&) per
+//   level, with o the point's byte offset in a field (at_off),
+//   init_stage(col index, Stg&), stage_level(k), stage(k, o, om, Stg, v[kNS])
+//   with om the mapped offset (o unless kMapped), stage_own the same for the
+//   thread's own point (Pre at hand),
 //   init_col(col index, Col&),
-//   point(k, a, Col, Pre, nb) with nb(m, f) = field f at stencil neighbour m
+//   point(k, o, Col, Pre, nb) with nb(m, f) = field f at stencil neighbour m
 //   (0 (0,0) 1 (+1,0) 2 (+1,+1) 3 (0,+1) 4 (-1,0) 5 (-1,-1) 6 (0,-1)),
 //   pole(pb): the pole centre of pole level pb (its point kernel).
 #pragma once
@@ -70,8 +72,8 @@ struct ColStencil {
     typename Op::Col col;
     typename Op::Stg sg, rsg;   // staging registers of the own and the ring column
     typename Op::Pre pre;
-    long a, ra;        // own and ring addresses at the current level
-    int rm;            // kMapped: the ring point's mapped address
+    unsigned o, ro;    // own and ring offsets at the current level
+    unsigned rm;       // kMapped: the ring point's mapped offset
     int k, sidx, ridx;
     bool outp, ring;
   };
@@ -95,7 +97,7 @@ struct ColStencil {
       const int i = i0 + tx, j = j0 + ty;
       s.outp = true;
       s.sidx = (ty + 1) * SW + tx + 1;
-      s.a = ((long)(l * d.kall + k0) * g + j) * g + i;
+      s.o = byte_off(((long)(l * d.kall + k0) * g + j) * g + i);
       op.init_col(((long)l * g + j) * g + i, s.col);
       op.init_stage(((long)l * g + j) * g + i, s.sg);
       op.begin(s.pre);
@@ -109,24 +111,24 @@ struct ColStencil {
       else { x = TX; y = tid - (2 * TX + TY + 2); }
       s.ring = true;
       s.ridx = (y + 1) * SW + x + 1;
-      s.ra = ((long)(l * d.kall + k0) * g + (j0 + y)) * g + (i0 + x);
+      s.ro = byte_off(((long)(l * d.kall + k0) * g + (j0 + y)) * g + (i0 + x));
       op.init_stage(((long)l * g + (j0 + y)) * g + (i0 + x), s.rsg);
-      if constexpr (Op::kMapped) s.rm = (int)src_at(d, cs, ((long)l * g + (j0 + y)) * g + (i0 + x), k0);
+      if constexpr (Op::kMapped) s.rm = byte_off(src_at(d, cs, ((long)l * g + (j0 + y)) * g + (i0 + x), k0));
     }
     return k1 - k0;
   }
   NH_HD void level_a(int step, State& s, real* lds) const {
-    if (s.outp) op.pre(s.k, s.a, s.pre);
+    if (s.outp) op.pre(s.k, s.o, s.sg, s.pre);
     if (!op.stage_level(s.k)) return;
     const int SW = cg.TX + 2, P = SW * (cg.TY + 2);
     real* buf = lds + (step & 1) * NS * P;
     real v[NS];
     if (s.outp) {
-      op.stage(s.k, s.a, s.a, s.sg, v);
+      op.stage_own(s.k, s.o, s.sg, s.pre, v);
       for (int f = 0; f < NS; ++f) buf[f * P + s.sidx] = v[f];
     }
     if (s.ring) {
-      op.stage(s.k, s.ra, Op::kMapped ? (long)s.rm : s.ra, s.rsg, v);
+      op.stage(s.k, s.ro, Op::kMapped ? s.rm : s.ro, s.rsg, v);
       for (int f = 0; f < NS; ++f) buf[f * P + s.ridx] = v[f];
     }
   }
@@ -135,17 +137,17 @@ struct ColStencil {
       const int SW = cg.TX + 2, P = SW * (cg.TY + 2);
       const real* buf = lds + (step & 1) * NS * P;
       const int x = s.sidx;
-      op.point(s.k, s.a, s.col, s.pre, [&](int m, int f) {
+      op.point(s.k, s.o, s.col, s.pre, [&](int m, int f) {
         const int off = (m == 0) ? 0 : (m == 1) ? 1 : (m == 2) ? 1 + SW : (m == 3) ? SW : (m == 4) ? -1
                       : (m == 5) ? -1 - SW : -SW;
         return buf[f * P + x + off];
       });
     }
-    const long gg = (long)op.d.g * op.d.g;
-    s.a += gg;
-    s.ra += gg;
+    const unsigned ls = byte_off((long)op.d.g * op.d.g);
+    s.o += ls;
+    s.ro += ls;
     if constexpr (Op::kMapped) {
-      if (s.ring) s.rm += (int)src_stride(op.d, s.rm);
+      if (s.ring) s.rm += src_stride_off(op.d, s.rm);
     }
     s.k += 1;
   }
@@ -163,13 +165,23 @@ struct ViMainHC {
     real c[3][7];
   };
   struct Stg {};
-  struct Pre {};
+  struct Pre {
+    real g5;
+  };
   NH_HD void init_stage(long, Stg&) const {}
   NH_HD void begin(Pre&) const {}
-  NH_HD void pre(int, long, Pre&) const {}
+  NH_HD void pre(int k, unsigned o, const Stg&, Pre& p) const {
+    if (stage_level(k)) p.g5 = at_off(pk.gT + 5 * d.NF, o);
+  }
+  NH_HD void stage_own(int k, unsigned o, const Stg& sg, const Pre&, real* v) const { stage(k, o, o, sg, v); }
   NH_HD bool stage_level(int k) const { return k >= d.kmin && k <= d.kmax; }
-  NH_HD void stage(int, long a, long am, const Stg&, real* v) const {
-    for (int f = 0; f < kNS; ++f) v[f] = pk.stage_val(f, a, am);
+  NH_HD void stage(int, unsigned o, unsigned om, const Stg&, real* v) const {
+    for (int q = 0; q < 3; ++q) {
+      v[q] = at_off(pk.dv[q], om);
+      v[5 + q] = at_off(pk.prog + (long)(1 + q) * d.NF, o);
+    }
+    v[3] = at_off(pk.eth, o);
+    v[4] = at_off(pk.ethtot, o);
   }
   NH_HD void init_col(long ci, Col& col) const {
     for (int dd = 0; dd < 3; ++dd)
@@ -178,9 +190,8 @@ struct ViMainHC {
   NH_HD void pole(int pb) const { pk(d.lall * d.kall + pb, 0); }
   // ViMainH::at with hdiv_multi<3>, term for term
   template <class NB>
-  NH_HD void point(int k, long a, const Col& col, Pre&, NB nb) const {
+  NH_HD void point(int k, unsigned o, const Col& col, Pre& p, NB nb) const {
     if (k < d.kmin || k > d.kmax) return;
-    const long NF = d.NF;
     real s[3][3];
 #pragma unroll
     for (int m = 0; m < 7; ++m) {
@@ -203,10 +214,10 @@ struct ViMainHC {
     const real he = s[1][0] + s[1][1] + s[1][2];
     const real hd = s[2][0] + s[2][1] + s[2][2];
     const real drhoge = -he - (real(0.0) - real(0.0)) * pk.G.rdgz[k];
-    const real grhoge1 = pk.gT[5 * NF + a] + drhoge;
-    pk.hv[0][a] = divs1;
-    pk.hv[1][a] = grhoge1 * pk.c.Rdry / pk.c.CVdry;
-    pk.hv[2][a] = hd;
+    const real grhoge1 = p.g5 + drhoge;
+    at_off(pk.hv[0], o) = divs1;
+    at_off(pk.hv[1], o) = grhoge1 * pk.c.Rdry / pk.c.CVdry;
+    at_off(pk.hv[2], o) = hd;
   }
 };
 
@@ -231,24 +242,30 @@ struct Path1C {
   struct Stg {};
   struct Pre {
     real g[3], dd[3], ps[3];
+    real mq[3], mp[3];   // mean fluxes: the sums and the previous step's momentum
   };
   NH_HD void init_stage(long, Stg&) const {}
   NH_HD bool stage_level(int) const { return true; }
-  NH_HD void stage(int k, long, long am, const Stg&, real* v) const {
-    v[0] = pk.ps[I_RHOGE][am + (long)pk.stage_shift(k) * src_stride(d, am)];
+  NH_HD void stage(int k, unsigned, unsigned om, const Stg&, real* v) const {
+    v[0] = at_off(pk.ps[I_RHOGE], om + (unsigned)pk.stage_shift(k) * src_stride_off(d, om));
   }
-  // address of the physical level a point takes its values from (ghost rows: the nearest)
-  NH_HD long phys(int k, long a) const {
+  NH_HD void stage_own(int k, unsigned o, const Stg& sg, const Pre&, real* v) const { stage(k, o, o, sg, v); }
+  // values from a point to the physical level it takes its momentum from (ghost rows: the nearest)
+  NH_HD long phys(int k) const {
     const long gg = (long)d.g * d.g;
-    return (k < d.kmin) ? a + gg : (k > d.kmax) ? a - gg : a;
+    return (k < d.kmin) ? gg : (k > d.kmax) ? -gg : 0;
   }
   NH_HD void begin(Pre&) const {}
-  NH_HD void pre(int k, long a, Pre& p) const {
-    const long an = phys(k, a);
+  NH_HD void pre(int k, unsigned o, const Stg&, Pre& p) const {
+    const long n = phys(k);
     for (int q = 0; q < 3; ++q) {
-      p.g[q] = pk.gT[(1 + q) * d.NF + an];
-      p.dd[q] = pk.dd[q][an];
-      p.ps[q] = pk.ps[1 + q][an];
+      p.g[q] = at_off(pk.gT + (1 + q) * d.NF + n, o);
+      p.dd[q] = at_off(pk.dd[q] + n, o);
+      p.ps[q] = at_off(pk.ps[1 + q] + n, o);
+      if (pk.mf.out) {
+        p.mq[q] = at_off(pk.mf.in + (1 + q) * d.NF, o);
+        if (pk.mf.two) p.mp[q] = at_off(pk.ps[1 + q], o);
+      }
     }
   }
   NH_HD void init_col(long ci, Col& col) const {
@@ -259,17 +276,10 @@ struct Path1C {
   NH_HD void pole(int pb) const { pk(d.lall * d.kall + pb, 0); }
   // Path1P's arithmetic for a regional point
   template <class NB>
-  NH_HD void point(int k, long a, const Col& col, Pre& p, NB nb) const {
-    const long NF = d.NF;
+  NH_HD void point(int k, unsigned o, const Col& col, Pre& p, NB nb) const {
     const int kmin = d.kmin, kmax = d.kmax;
     const real R = pk.c.RADIUS, RovCV = pk.c.Rdry / pk.c.CVdry;
     const MeanFlux& mf = pk.mf;
-    real pmq[3] = {real(0.0), real(0.0), real(0.0)}, pmp[3] = {real(0.0), real(0.0), real(0.0)};
-    if (mf.out) {
-      for (int q = 0; q < 3; ++q) pmq[q] = mf.in[(1 + q) * NF + a];
-      if (mf.two)
-        for (int q = 0; q < 3; ++q) pmp[q] = pk.ps[1 + q][a];
-    }
     real pr[7];
     for (int m = 0; m < 7; ++m) pr[m] = (nb(m, 0) * RovCV) * real(1.0);
     real gr[3];
@@ -287,12 +297,12 @@ struct Path1C {
     }
     if (k < kmin || k > kmax) {
       // free-slip top / rigid bottom, scaled by the large-step density
-      const real rn = pk.prog[phys(k, a)], ra = pk.prog[a];
+      const real rn = at_off(pk.prog + phys(k), o), ra = at_off(pk.prog, o);
       for (int q = 0; q < 3; ++q) v[q] = (k > kmax) ? real(1.0) * (v[q] / rn) * ra : -real(1.0) * (v[q] / rn) * ra;
     }
     for (int q = 0; q < 3; ++q) {
-      pk.dv[q][a] = v[q];
-      if (mf.out) mf.out[(1 + q) * NF + a] = mf.add(pmq[q], pmp[q], v[q], pk.rweight);
+      at_off(pk.dv[q], o) = v[q];
+      if (mf.out) at_off(mf.out + (1 + q) * d.NF, o) = mf.add(p.mq[q], p.mp[q], v[q], pk.rweight);
     }
   }
 };
@@ -303,7 +313,9 @@ struct Path1C {
 // carries what levels k and k + 1 share (the effective gravity of the half
 // levels, with its divisions, in both precisions, and eth at half levels), where
 // the point form forms each three times; all loads of a level go out before
-// its barrier.
+// its barrier.  Bound by memory latency at the 3 (FP64 2) waves per SIMD its
+// registers leave: 340 us per launch at gl07 mixed, 533 FP64 (34 fields, 3 FP64
+// fields: 222 and 425 us of streaming); one thread per point 454 and 788.
 struct ViPath0C {
   static constexpr const char* kName = "vi_path0";
   static constexpr int kNS = 5;
@@ -325,8 +337,8 @@ struct ViPath0C {
   NH_HD void init_stage(long, Stg&) const {}
   NH_HD void begin(Pre& p) const { p.have = false; }
   NH_HD bool stage_level(int k) const { return k >= d.kmin && k <= d.kmax; }
-  NH_HD void stage(int k, long a, long, const Stg&, real* v) const {
-    const unsigned o = byte_off(a);
+  NH_HD void stage_own(int k, unsigned o, const Stg& sg, const Pre&, real* v) const { stage(k, o, o, sg, v); }
+  NH_HD void stage(int k, unsigned o, unsigned, const Stg&, real* v) const {
     for (int q = 0; q < 3; ++q) v[q] = at_off(pk.prog + (long)(1 + q) * d.NF, o);
     v[3] = at_off(pk.eth, o);
     // the pressure at the level of its gradient (kmin -> kmin+1), pregd
@@ -377,12 +389,11 @@ struct ViPath0C {
     const int k2 = (kk > d.kall - 1) ? d.kall - 1 : kk;
     return pk.G.afact[k2] * e + pk.G.bfact[k2] * el;
   }
-  NH_HD void pre(int k, long a, Pre& p) const {
+  NH_HD void pre(int k, unsigned o, const Stg&, Pre& p) const {
     const long NF = d.NF, gg = (long)d.g * d.g;
     const real* rg = pk.prog;
     const real* rw = pk.prog + 4 * NF;
     const real* pr = pk.diag + I_PRE * NF;
-    const unsigned o = byte_off(a);
     if (p.have) {
       p.rgm = p.rg0; p.rg0 = p.rg1;
       p.pr0 = p.pr1; p.et0 = p.et1; p.rw0 = p.rw1;
@@ -415,9 +426,9 @@ struct ViPath0C {
   }
   // ViPath0P::at for a regional point, term for term
   template <class NB>
-  NH_HD void point(int k, long a, const Col& col, Pre& p, NB nb) const {
+  NH_HD void point(int k, unsigned o, const Col& col, Pre& p, NB nb) const {
     const long NF = d.NF;
-    const unsigned o = byte_off(a);
+    const long a = (long)(o / (unsigned)sizeof(real));   // the FP64 matrix is indexed in 64 bits
     const int kmin = d.kmin, kmax = d.kmax;
     const Geo& G = pk.G;
     const real R = pk.c.RADIUS;
@@ -525,10 +536,14 @@ struct LapC {
   struct Pre {};
   NH_HD void init_stage(long, Stg&) const {}
   NH_HD void begin(Pre&) const {}
-  NH_HD void pre(int, long, Pre&) const {}
+  NH_HD void pre(int, unsigned, const Stg&, Pre&) const {}
+  NH_HD void stage_own(int k, unsigned o, const Stg& sg, const Pre&, real* v) const { stage(k, o, o, sg, v); }
   NH_HD bool stage_level(int) const { return true; }
-  NH_HD void stage(int k, long, long am, const Stg&, real* v) const {
-    for (int f = 0; f < NFLD; ++f) v[f] = pk.input(f, am, k);
+  NH_HD void stage(int k, unsigned, unsigned om, const Stg&, real* v) const {
+    for (int f = 0; f < NFLD; ++f) {
+      const real x = at_off(in[f], om);
+      v[f] = pk.sub[f] ? (real)((double)x - pk.sub[f][k]) : x;   // HDiffPassP::input
+    }
   }
   NH_HD void init_col(long ci, Col& col) const {
     for (int m = 0; m < 7; ++m) col.c[m] = rc(pk.G.clap, d.nreg, m, ci);
@@ -537,12 +552,12 @@ struct LapC {
     if (!pole_off) pk(d.lall * d.kall + pb, 0);
   }
   template <class NB>
-  NH_HD void point(int, long a, const Col& col, Pre&, NB nb) const {
+  NH_HD void point(int, unsigned o, const Col& col, Pre&, NB nb) const {
     for (int f = 0; f < NFLD; ++f) {
       real r = col.c[0] * nb(0, f);
 #pragma unroll
       for (int m = 1; m < 7; ++m) r = r + col.c[m] * nb(m, f);
-      out[f][a] = -r;
+      at_off(out[f], o) = -r;
     }
   }
 };
@@ -564,13 +579,18 @@ struct LapTC {
     real c[7];
   };
   struct Stg {};
-  struct Pre {};
+  struct Pre {
+    real ib[NFLD];
+  };
   NH_HD void init_stage(long, Stg&) const {}
   NH_HD void begin(Pre&) const {}
-  NH_HD void pre(int, long, Pre&) const {}
+  NH_HD void pre(int, unsigned o, const Stg&, Pre& p) const {
+    for (int f = 0; f < NFLD; ++f) p.ib[f] = at_off(ib[f], o);
+  }
+  NH_HD void stage_own(int k, unsigned o, const Stg& sg, const Pre&, real* v) const { stage(k, o, o, sg, v); }
   NH_HD bool stage_level(int) const { return true; }
-  NH_HD void stage(int, long a, long, const Stg&, real* v) const {
-    for (int f = 0; f < NFLD; ++f) v[f] = ob[f][a];
+  NH_HD void stage(int, unsigned o, unsigned, const Stg&, real* v) const {
+    for (int f = 0; f < NFLD; ++f) v[f] = at_off(ob[f], o);
   }
   NH_HD void init_col(long ci, Col& col) const {
     const long gg = (long)d.g * d.g;
@@ -585,14 +605,14 @@ struct LapTC {
   }
   NH_HD void pole(int) const {}
   template <class NB>
-  NH_HD void point(int, long a, const Col& col, Pre&, NB nb) const {
+  NH_HD void point(int, unsigned o, const Col& col, Pre& p, NB nb) const {
     // the source x - off(m) is staged neighbour opp(m)
     const int opp[7] = {0, 4, 5, 6, 1, 2, 3};
     for (int f = 0; f < NFLD; ++f) {
       real acc = real(0.0);
 #pragma unroll
       for (int m = 0; m < 7; ++m) acc += col.c[m] * nb(opp[m], f);
-      ib[f][a] += -acc;
+      at_off(ib[f], o) = p.ib[f] + -acc;
     }
   }
 };
@@ -601,8 +621,12 @@ struct LapTC {
 // divergence coefficients and the column's position in registers; staged per
 // level are the merged velocity v + w_full r/|r| (formed once per point, where
 // the point kernel forms it once per neighbour) and the three momentum
-// components.  Term for term the point kernel's arithmetic; pole centres run
-// the point kernel.
+// components.  A column marches upward and carries its own merged velocity at
+// k - 1, k and k + 1; all loads of a level go out before its barrier.  Term for
+// term the point kernel's arithmetic; pole centres run the point kernel.  At
+// gl07 166 us per launch mixed, 314 FP64 (13 fields: 80 and 155 us of streaming);
+// with the neighbouring levels loaded after the barrier 187 mixed, level-staged
+// points 464 FP64.
 struct AdvMomC {
   static constexpr const char* kName = "adv_mom";
   static constexpr int kNS = 6;
@@ -616,24 +640,61 @@ struct AdvMomC {
   struct Stg {
     real x[3];
   };
-  struct Pre {};
-  NH_HD void begin(Pre&) const {}
-  NH_HD void pre(int, long, Pre&) const {}
+  struct Pre {
+    bool have;
+    real vm[3], v0[3], v1[3];   // merged velocity at levels k-1, k, k+1
+    real w1, w2;                // w at half levels k+1, k+2
+    real rw0, rw1, rg;          // rhogw at half levels k, k+1; density
+  };
   NH_HD void init_stage(long ci, Stg& sg) const {
     for (int q = 0; q < 3; ++q) sg.x[q] = pk.G.gx[q * d.nreg + ci];
   }
+  NH_HD void begin(Pre& p) const { p.have = false; }
   NH_HD bool stage_level(int k) const { return k >= d.kmin && k <= d.kmax; }
-  NH_HD void stage(int k, long a, long, const Stg& sg, real* v) const {
+  // merged velocity at level kk (up levels above the point's) from w at its half levels
+  NH_HD void merged(int kk, long up, unsigned o, const Stg& sg, real whi, real wlo, real* v) const {
+    const long NF = d.NF;
+    const real R = pk.c.RADIUS;
+    const real wc = pk.G.cfact[kk] * whi + pk.G.dfact[kk] * wlo;
+    v[0] = at_off(pk.diag + I_VX * NF + up, o) + wc * sg.x[0] / R;
+    v[1] = at_off(pk.diag + I_VY * NF + up, o) + wc * sg.x[1] / R;
+    v[2] = at_off(pk.diag + I_VZ * NF + up, o) + wc * sg.x[2] / R;
+  }
+  NH_HD void pre(int k, unsigned o, const Stg& sg, Pre& p) const {
+    const long NF = d.NF, gg = (long)d.g * d.g;
+    if (!stage_level(k)) return;
+    const real* wd = pk.diag + I_W * NF;
+    const real* rw = pk.prog + 4 * NF;
+    if (p.have) {
+      for (int q = 0; q < 3; ++q) { p.vm[q] = p.v0[q]; p.v0[q] = p.v1[q]; }
+      p.w1 = p.w2;
+      p.rw0 = p.rw1;
+    } else {
+      const real w0 = at_off(wd, o);
+      p.w1 = at_off(wd + gg, o);
+      p.rw0 = at_off(rw, o);
+      if (k >= d.kmin + 1) merged(k - 1, -gg, o, sg, w0, at_off(wd - gg, o), p.vm);
+      merged(k, 0, o, sg, p.w1, w0, p.v0);
+      p.have = true;
+    }
+    if (k + 1 <= d.kmax) {
+      p.w2 = at_off(wd + 2 * gg, o);
+      merged(k + 1, gg, o, sg, p.w2, p.w1, p.v1);
+      p.rw1 = at_off(rw + gg, o);
+    }
+    p.rg = at_off(pk.prog, o);
+  }
+  NH_HD void stage(int k, unsigned o, unsigned, const Stg& sg, real* v) const {
     const long NF = d.NF, gg = (long)d.g * d.g;
     const real* wd = pk.diag + I_W * NF;
-    const real R = pk.c.RADIUS;
-    const real wc = pk.G.cfact[k] * wd[a + gg] + pk.G.dfact[k] * wd[a];
-    v[0] = pk.diag[I_VX * NF + a] + wc * sg.x[0] / R;
-    v[1] = pk.diag[I_VY * NF + a] + wc * sg.x[1] / R;
-    v[2] = pk.diag[I_VZ * NF + a] + wc * sg.x[2] / R;
-    v[3] = pk.prog[1 * NF + a];
-    v[4] = pk.prog[2 * NF + a];
-    v[5] = pk.prog[3 * NF + a];
+    merged(k, 0, o, sg, at_off(wd + gg, o), at_off(wd, o), v);
+    for (int q = 0; q < 3; ++q) v[3 + q] = at_off(pk.prog + (1 + q) * NF, o);
+  }
+  NH_HD void stage_own(int, unsigned o, const Stg&, const Pre& p, real* v) const {
+    for (int q = 0; q < 3; ++q) {
+      v[q] = p.v0[q];
+      v[3 + q] = at_off(pk.prog + (1 + q) * d.NF, o);
+    }
   }
   NH_HD void init_col(long ci, Col& col) const {
     for (int dd = 0; dd < 3; ++dd)
@@ -642,29 +703,17 @@ struct AdvMomC {
   }
   NH_HD void pole(int pb) const { pk(d.lall * d.kall + pb, 0); }
   template <class NB>
-  NH_HD void point(int k, long a, const Col& col, Pre&, NB nb) const {
-    const long NF = d.NF, ks = (long)d.g * d.g;
+  NH_HD void point(int k, unsigned o, const Col& col, Pre& p, NB nb) const {
+    const long NF = d.NF;
     const int kmin = d.kmin, kmax = d.kmax;
     real* out = pk.out;
     if (k < kmin || k > kmax) {
-      for (int q = 0; q < 4; ++q) out[q * NF + a] = real(0.0);
+      for (int q = 0; q < 4; ++q) at_off(out + q * NF, o) = real(0.0);
       return;
     }
     const Geo& G = pk.G;
     const real R = pk.c.RADIUS;
-    const real* rw = pk.prog + 4 * NF;
-    const real* rg = pk.prog;
-    const real* vxd = pk.diag + I_VX * NF;
-    const real* vyd = pk.diag + I_VY * NF;
-    const real* vzd = pk.diag + I_VZ * NF;
-    const real* wd = pk.diag + I_W * NF;
     const real* x0 = col.x;
-    auto vv3 = [&](long b, int kk, real* o) {
-      const real wc = G.cfact[kk] * wd[b + ks] + G.dfact[kk] * wd[b];
-      o[0] = vxd[b] + wc * x0[0] / R;
-      o[1] = vyd[b] + wc * x0[1] / R;
-      o[2] = vzd[b] + wc * x0[2] / R;
-    };
     real sd[3][3];
 #pragma unroll
     for (int m = 0; m < 7; ++m) {
@@ -682,34 +731,25 @@ struct AdvMomC {
     }
     real div[3];
     for (int q = 0; q < 3; ++q) div[q] = sd[0][q] + sd[1][q] + sd[2][q];
-    const real vvm0[3] = {nb(0, 0), nb(0, 1), nb(0, 2)};
     real hi[3] = {real(0.0), real(0.0), real(0.0)}, lo[3] = {real(0.0), real(0.0), real(0.0)};
-    if (k + 1 <= kmax) {
-      real up[3];
-      vv3(a + ks, k + 1, up);
-      const real wup = rw[a + ks];
+    if (k + 1 <= kmax)
       for (int q = 0; q < 3; ++q)
-        hi[q] = real(0.0) * real(1.0) + wup * (G.afact[k + 1] * up[q] + G.bfact[k + 1] * vvm0[q]) * real(1.0);
-    }
-    if (k >= kmin + 1) {
-      real dn[3];
-      vv3(a - ks, k - 1, dn);
-      const real w0 = rw[a];
+        hi[q] = real(0.0) * real(1.0) + p.rw1 * (G.afact[k + 1] * p.v1[q] + G.bfact[k + 1] * p.v0[q]) * real(1.0);
+    if (k >= kmin + 1)
       for (int q = 0; q < 3; ++q)
-        lo[q] = real(0.0) * real(1.0) + w0 * (G.afact[k] * vvm0[q] + G.bfact[k] * dn[q]) * real(1.0);
-    }
+        lo[q] = real(0.0) * real(1.0) + p.rw0 * (G.afact[k] * p.v0[q] + G.bfact[k] * p.vm[q]) * real(1.0);
     real dvv[3];
     for (int q = 0; q < 3; ++q) dvv[q] = -div[q] - (hi[q] - lo[q]) * G.rdgz[k];
     const real gxc = x0[0] / R, gyc = x0[1] / R, gzc = x0[2] / R;
-    const real rh = rg[a];
-    const real dx = dvv[0] - (-real(2.0) * rh * (pk.c.OHM * vvm0[1]));
-    const real dy = dvv[1] - (real(2.0) * rh * (pk.c.OHM * vvm0[0]));
+    const real rh = p.rg;
+    const real dx = dvv[0] - (-real(2.0) * rh * (pk.c.OHM * p.v0[1]));
+    const real dy = dvv[1] - (real(2.0) * rh * (pk.c.OHM * p.v0[0]));
     const real dz = dvv[2];
     const real prd = dx * gxc + dy * gyc + dz * gzc;
-    out[0 * NF + a] = dx - prd * gxc;
-    out[1 * NF + a] = dy - prd * gyc;
-    out[2 * NF + a] = dz - prd * gzc;
-    out[3 * NF + a] = prd * pk.c.ALPHA;
+    at_off(out + 0 * NF, o) = dx - prd * gxc;
+    at_off(out + 1 * NF, o) = dy - prd * gyc;
+    at_off(out + 2 * NF, o) = dz - prd * gzc;
+    at_off(out + 3 * NF, o) = prd * pk.c.ALPHA;
   }
 };
 

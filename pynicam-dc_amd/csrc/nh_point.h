@@ -164,151 +164,67 @@ struct PrePostP {
 // out[0..2]: momentum tendencies; out[3]: the radial part gwc at full levels
 // (the half-level w tendency c2w0*gwc(k) + c2w1*gwc(k-1) is formed by its user)
 // ----------------------------------------------------------------------------
+// the pole centres (the regional points run as AdvMomC)
 struct AdvMomP {
-  static constexpr const char* kName = "adv_mom";
-  // fields read on the stencil: vx, vy, vz, w(k), w(k+1), rhogvx, rhogvy, rhogvz
-  static constexpr int kNStage = 8;
   Dims d; Consts c; Geo G;
   const real* prog;
   const real* diag;
   real* out;
-  // field f of the stencil set, positioned so that the point's own level reads it
-  NH_HD const real* stage_ptr(int f, int) const {
-    const long NF = d.NF;
-    switch (f) {
-      case 0: return diag + I_VX * NF;
-      case 1: return diag + I_VY * NF;
-      case 2: return diag + I_VZ * NF;
-      case 3: return diag + I_W * NF;
-      case 4: return diag + I_W * NF + (long)d.g * d.g;   // next level of the region
-      default: return prog + (long)(f - 4) * NF;
-    }
-  }
-  NH_HD bool stage_level(int k) const { return k >= d.kmin && k <= d.kmax; }
   NH_HD void operator()(int plane, int x) const {
     Pt p;
-    if (!pt_of(d, plane, x, p)) return;
-    if (!pt_compute(p)) {
-      for (int q = 0; q < 4; ++q) out[q * d.NF + p.a] = real(0.0);
-      return;
-    }
-    const long ks = p.ks;
-    at(p, [&](int f, long b) { return f == 4 ? diag[I_W * d.NF + b + ks] : stage_ptr(f, p.k)[b]; });
-  }
-  template <class LD>
-  NH_HD void at(const Pt& p, LD ld) const {
-    const long NF = d.NF, a = p.a;
+    if (!pt_of(d, plane, x, p) || !p.pole || p.v != 0) return;
+    const long NF = d.NF, a = p.a, ks = p.ks;
     const int kmin = d.kmin, kmax = d.kmax, k = p.k;
     if (k < kmin || k > kmax) {
       for (int q = 0; q < 4; ++q) out[q * NF + a] = real(0.0);
       return;
     }
-    // separate instances for the 6-point pole and 7-point regional stencils:
-    // fixed trip counts keep the per-neighbour arrays in registers
-    if (p.pole) point<true>(p, ld);
-    else point<false>(p, ld);
-  }
-  template <bool POLE, class LD>
-  NH_HD void point(const Pt& p, LD ld) const {
-    constexpr int NN = POLE ? 6 : 7;
-    const long NF = d.NF, a = p.a, ks = p.ks;
-    const int kmin = d.kmin, kmax = d.kmax, k = p.k;
     const real R = c.RADIUS;
     const real* rw = prog + 4 * NF;
-    const real* rg = prog;
-    const real* vxd = diag + I_VX * NF;
-    const real* vyd = diag + I_VY * NF;
-    const real* vzd = diag + I_VZ * NF;
     const real* wd = diag + I_W * NF;
-    const long g = d.g;
-    // stencil offset of neighbour m: (di, dj) + 1 packed two bits per point,
-    // (0,0) (+1,0) (+1,+1) (0,+1) (-1,0) (-1,-1) (0,-1)
-    auto off = [&](int m) -> long {
-      const int di = ((4201 >> (2 * m)) & 3) - 1, dj = ((421 >> (2 * m)) & 3) - 1;
-      return di + dj * g;
-    };
-    // address and position of neighbour m
-    auto nbr = [&](int m) { return POLE ? a + m : a + off(m); };
-    auto pos = [&](int m, real* x) {
-      if (POLE) {
-        for (int q = 0; q < 3; ++q) x[q] = G.gx_pl[(m * 2 + p.lp) * 3 + q];
-      } else {
-        for (int q = 0; q < 3; ++q) x[q] = G.gx[q * d.nreg + p.ci + off(m)];
-      }
+    auto pos = [&](int m, real* x3) {
+      for (int q = 0; q < 3; ++q) x3[q] = G.gx_pl[(m * 2 + p.lp) * 3 + q];
     };
     // merged velocity v + w_full r/|r| at address b (level kk) with position x
-    auto vv3 = [&](long b, int kk, const real* x, real* o) {
+    auto vv3 = [&](long b, int kk, const real* x3, real* o) {
       const real wc = G.cfact[kk] * wd[b + ks] + G.dfact[kk] * wd[b];
-      o[0] = vxd[b] + wc * x[0] / R;
-      o[1] = vyd[b] + wc * x[1] / R;
-      o[2] = vzd[b] + wc * x[2] / R;
+      for (int q = 0; q < 3; ++q) o[q] = diag[(I_VX + q) * NF + b] + wc * x3[q] / R;
     };
-    real x0[3];
+    real x0[3], vvm0[3], div[3];
     pos(0, x0);
-    // divergence of rhogv * vv_q, one neighbour at a time: per direction and
-    // component the sum over the neighbours runs in stencil order, as in
-    // div7 / div_pl, without keeping every neighbour's values live
-    real vvm0[3];
-    real sd[3][3];   // [direction][q] (regional); the pole sums the directions per point
-    real div[3];
-#ifdef NH_ADV_UNROLL
-#pragma unroll
-#else
-#pragma unroll 1
-#endif
-    for (int m = 0; m < NN; ++m) {
+    // divergence of rhogv * vv_q: the directions summed per point, as in div_pl
+    for (int m = 0; m < 6; ++m) {
       real xm[3], vv[3];
       pos(m, xm);
-      const long bm = nbr(m);
-      {
-        const real wc = G.cfact[k] * ld(4, bm) + G.dfact[k] * ld(3, bm);
-        vv[0] = ld(0, bm) + wc * xm[0] / R;
-        vv[1] = ld(1, bm) + wc * xm[1] / R;
-        vv[2] = ld(2, bm) + wc * xm[2] / R;
-      }
+      vv3(a + m, k, xm, vv);
       if (m == 0)
         for (int q = 0; q < 3; ++q) vvm0[q] = vv[q];
-      const real fx0 = ld(5, bm), fy0 = ld(6, bm), fz0 = ld(7, bm);
-      if (POLE) {
-        const real* cc = G.cdiv_pl + (m * 2 + p.lp) * 3;
-        for (int q = 0; q < 3; ++q) {
-          const real pv = cc[0] * (fx0 * vv[q] * real(1.0)) + cc[1] * (fy0 * vv[q] * real(1.0)) +
-                          cc[2] * (fz0 * vv[q] * real(1.0));
-          div[q] = (m == 0) ? pv : div[q] + pv;
-        }
-      } else {
-        const real cx = rc(G.cdiv, d.nreg, m, p.ci), cy = rc(G.cdiv, d.nreg, 7 + m, p.ci),
-                   cz = rc(G.cdiv, d.nreg, 14 + m, p.ci);
-        for (int q = 0; q < 3; ++q) {
-          const real tx = cx * (fx0 * vv[q] * real(1.0));
-          const real ty = cy * (fy0 * vv[q] * real(1.0));
-          const real tz = cz * (fz0 * vv[q] * real(1.0));
-          sd[0][q] = (m == 0) ? tx : sd[0][q] + tx;
-          sd[1][q] = (m == 0) ? ty : sd[1][q] + ty;
-          sd[2][q] = (m == 0) ? tz : sd[2][q] + tz;
-        }
+      const real fx0 = prog[1 * NF + a + m], fy0 = prog[2 * NF + a + m], fz0 = prog[3 * NF + a + m];
+      const real* cc = G.cdiv_pl + (m * 2 + p.lp) * 3;
+      for (int q = 0; q < 3; ++q) {
+        const real pv = cc[0] * (fx0 * vv[q] * real(1.0)) + cc[1] * (fy0 * vv[q] * real(1.0)) +
+                        cc[2] * (fz0 * vv[q] * real(1.0));
+        div[q] = (m == 0) ? pv : div[q] + pv;
       }
     }
-    if (!POLE)
-      for (int q = 0; q < 3; ++q) div[q] = sd[0][q] + sd[1][q] + sd[2][q];
     // vertical fluxes at the half levels k+1 and k (zero at kmin and kmax+1)
     real hi[3] = {real(0.0), real(0.0), real(0.0)}, lo[3] = {real(0.0), real(0.0), real(0.0)};
     if (k + 1 <= kmax) {
       real up[3];
       vv3(a + ks, k + 1, x0, up);
-      const real wup = rw[a + ks];
-      for (int q = 0; q < 3; ++q) hi[q] = real(0.0) * real(1.0) + wup * (G.afact[k + 1] * up[q] + G.bfact[k + 1] * vvm0[q]) * real(1.0);
+      for (int q = 0; q < 3; ++q)
+        hi[q] = real(0.0) * real(1.0) + rw[a + ks] * (G.afact[k + 1] * up[q] + G.bfact[k + 1] * vvm0[q]) * real(1.0);
     }
     if (k >= kmin + 1) {
       real dn[3];
       vv3(a - ks, k - 1, x0, dn);
-      const real w0 = rw[a];
-      for (int q = 0; q < 3; ++q) lo[q] = real(0.0) * real(1.0) + w0 * (G.afact[k] * vvm0[q] + G.bfact[k] * dn[q]) * real(1.0);
+      for (int q = 0; q < 3; ++q)
+        lo[q] = real(0.0) * real(1.0) + rw[a] * (G.afact[k] * vvm0[q] + G.bfact[k] * dn[q]) * real(1.0);
     }
     real dvv[3];
     for (int q = 0; q < 3; ++q) dvv[q] = -div[q] - (hi[q] - lo[q]) * G.rdgz[k];
     const real gxc = x0[0] / R, gyc = x0[1] / R, gzc = x0[2] / R;
-    const real rh = rg[a];
+    const real rh = prog[a];
     const real dx = dvv[0] - (-real(2.0) * rh * (c.OHM * vvm0[1]));
     const real dy = dvv[1] - (real(2.0) * rh * (c.OHM * vvm0[0]));
     const real dz = dvv[2];
@@ -540,22 +456,17 @@ struct ViPath0P {
   double* Mc; double* Mu; double* Ml;   // FP64 in every form
   real* getot;
   real* frhog;
-  // fields read on the stencil: rhogvx, rhogvy, rhogvz, eth at the point's
-  // level, the pressure at the level of its gradient (kmin -> kmin+1)
-  static constexpr int kNStage = 5;
-  NH_HD const real* stage_ptr(int f, int k) const {
-    const long NF = d.NF;
-    if (f < 3) return prog + (long)(1 + f) * NF;
-    if (f == 3) return eth;
-    return diag + I_PRE * NF + (k == d.kmin ? (long)d.g * d.g : 0L);
-  }
-  NH_HD bool stage_level(int k) const { return k >= d.kmin && k <= d.kmax; }
+  // the pole centres (the regional points run as ViPath0C)
   NH_HD void operator()(int plane, int x) const {
     Pt p;
-    if (!pt_of(d, plane, x, p) || !pt_compute(p)) return;
-    const long sh = (p.k == d.kmin) ? p.ks : 0;   // the level stride differs at the poles
-    at(p, [&](int f, long b) { return f < 4 ? stage_ptr(f, p.k)[b] : diag[I_PRE * d.NF + b + sh]; });
+    if (!pt_of(d, plane, x, p) || !p.pole || p.v != 0) return;
+    const long sh = (p.k == d.kmin) ? p.ks : 0;
+    at(p, [&](int f, long b) {
+      return f < 3 ? prog[(long)(1 + f) * d.NF + b] : f == 3 ? eth[b] : diag[I_PRE * d.NF + b + sh];
+    });
   }
+  // ld(f, address): rhogvx, rhogvy, rhogvz, eth at the point's level, the
+  // pressure at the level of its gradient (kmin -> kmin+1)
   template <class LD>
   NH_HD void at(const Pt& p, LD ld) const {
     const long NF = d.NF, ks = p.ks, a = p.a;
@@ -605,12 +516,7 @@ struct ViPath0P {
     };
     auto gzt = [&](int kk) { return c.GRAV - (dpgw(kk) - dbuo(kk)) / rhog_h(kk); };
     auto pwh = [&](int kk) { return -gzt(kk) * RW(kk); };
-    real gx, gy, gz;
-    if (p.pole) {
-      gx = G.gx_pl[p.lp * 3 + 0]; gy = G.gx_pl[p.lp * 3 + 1]; gz = G.gx_pl[p.lp * 3 + 2];
-    } else {
-      gx = G.gx[p.ci]; gy = G.gx[d.nreg + p.ci]; gz = G.gx[2 * d.nreg + p.ci];
-    }
+    const real gx = G.gx_pl[p.lp * 3 + 0], gy = G.gx_pl[p.lp * 3 + 1], gz = G.gx_pl[p.lp * 3 + 2];
     const real Kh = c.GAMMA_H;
     // hyperdiffusion tendency + momentum advection = large-step tendency g0
     const real rgk = RG(k);
@@ -621,11 +527,8 @@ struct ViPath0P {
     const real fw = -(vt[3][a] * Kh + real(0.0)) * rgh;
     const real fe = -(vt[4][a] + real(0.0));
     const real fr = -(vt[5][a] + real(0.0));
-    if (p.pole) {
+    {
       const real prd = fvx * gx / R + fvy * gy / R + fvz * gz / R;
-      fvx = fvx - prd * gx / R; fvy = fvy - prd * gy / R; fvz = fvz - prd * gz / R;
-    } else {
-      const real prd = (fvx * gx + fvy * gy + fvz * gz) / R;
       fvx = fvx - prd * gx / R; fvy = fvy - prd * gy / R; fvz = fvz - prd * gz / R;
     }
     const real gadv_w = (k > kmin && k <= kmax) ? (G.c2w0[k] * gadv[3 * NF + a] + G.c2w1[k] * gadv[3 * NF + a - ks]) : real(0.0);
@@ -714,49 +617,28 @@ struct ViPath0P {
       Ml[a] = -V.rdgzh[k] * (Cl1 * eth_h64(k - 1) - V.dfact[k - 1] * (gzt64(k - 1) + Cl2));
     }
   }
-  // horizontal pressure-gradient force at the point with the first-layer
-  // remedy (presgrad_h), the pressure of the gradient's level read as ld(4, .)
+  // horizontal pressure-gradient force at the pole centre with the first-layer
+  // remedy, the pressure of the gradient's level read as ld(4, .)
   template <class LD>
   NH_HD void presgrad_ld(const Pt& p, LD ld, real R, real o[3]) const {
     const long a = p.a;
     real gr[3];
-    if (p.pole) {
-      for (int dd2 = 0; dd2 < 3; ++dd2) {
-        real acc = real(0.0);
-        for (int v = 0; v < 6; ++v) {
-          const real pv = G.cgrad_pl[(v * 2 + p.lp) * 3 + dd2] * (ld(4, a + v) * real(1.0) * real(1.0));
-          acc = (v == 0) ? pv : acc + pv;
-        }
-        gr[dd2] = acc;
+    for (int dd2 = 0; dd2 < 3; ++dd2) {
+      real acc = real(0.0);
+      for (int v = 0; v < 6; ++v) {
+        const real pv = G.cgrad_pl[(v * 2 + p.lp) * 3 + dd2] * (ld(4, a + v) * real(1.0) * real(1.0));
+        acc = (v == 0) ? pv : acc + pv;
       }
-    } else {
-      const long g = d.g;
-      for (int dd2 = 0; dd2 < 3; ++dd2) {
-        real acc = rc(G.cgrad, d.nreg, dd2 * 7 + 0, p.ci) * (ld(4, a) * real(1.0));
-        for (int m = 1; m < 7; ++m) {
-          const long off = (((4201 >> (2 * m)) & 3) - 1) + (((421 >> (2 * m)) & 3) - 1) * g;
-          acc = acc + rc(G.cgrad, d.nreg, dd2 * 7 + m, p.ci) * (ld(4, a + off) * real(1.0));
-        }
-        gr[dd2] = acc;
-      }
+      gr[dd2] = acc;
     }
     for (int q = 0; q < 3; ++q) gr[q] = gr[q] + real(0.0);
-    real gx, gy, gz;
-    if (p.pole) {
-      gx = G.gx_pl[(0 * 2 + p.lp) * 3 + 0];
-      gy = G.gx_pl[(0 * 2 + p.lp) * 3 + 1];
-      gz = G.gx_pl[(0 * 2 + p.lp) * 3 + 2];
-      const real prd = gr[0] * gx / R + gr[1] * gy / R + gr[2] * gz / R;
-      o[0] = gr[0] - prd * gx / R;
-      o[1] = gr[1] - prd * gy / R;
-      o[2] = gr[2] - prd * gz / R;
-    } else {
-      gx = G.gx[p.ci]; gy = G.gx[d.nreg + p.ci]; gz = G.gx[2 * d.nreg + p.ci];
-      const real prd = (gr[0] * gx + gr[1] * gy + gr[2] * gz) / R;
-      o[0] = gr[0] - prd * gx / R;
-      o[1] = gr[1] - prd * gy / R;
-      o[2] = gr[2] - prd * gz / R;
-    }
+    const real gx = G.gx_pl[(0 * 2 + p.lp) * 3 + 0];
+    const real gy = G.gx_pl[(0 * 2 + p.lp) * 3 + 1];
+    const real gz = G.gx_pl[(0 * 2 + p.lp) * 3 + 2];
+    const real prd = gr[0] * gx / R + gr[1] * gy / R + gr[2] * gz / R;
+    o[0] = gr[0] - prd * gx / R;
+    o[1] = gr[1] - prd * gy / R;
+    o[2] = gr[2] - prd * gz / R;
   }
 };
 

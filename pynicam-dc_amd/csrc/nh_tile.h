@@ -1,15 +1,9 @@
 // LDS-tiled kernels.
 //
-// Level tiles (StagedPointT): a block owns all interior i (W = g-2 points) of
-// TH rows of one region level; phase 0 stages the fields a point kernel reads
-// on its stencil (the tile's rows and one halo row on each side) into LDS, and
-// the point kernel then reads its stencil from there.  Blocks past the
-// regional tiles do the pole levels with the point kernel itself.
-//
 // Column tiles (DivDampK, DiffKhK; the stencil engine of nh_colstencil.h): a
-// block owns a 16 x 16 tile of one region over a chunk of levels, each
-// thread one corner column with its coefficients in registers; per level the
-// corner threads form their two triangle values into double-buffered LDS, one
+// block owns a 64 x 4 tile of one region over a chunk of levels, each thread
+// one corner column with its coefficients in registers; per level the corner
+// threads form their two triangle values into double-buffered LDS, one
 // barrier, then the tile points form their hexagon sums.
 //
 // On the GPU the phases are separated by a workgroup barrier; the host test
@@ -19,113 +13,6 @@
 #include "nh_point.h"
 
 NH_BEGIN
-
-struct TileGeom {
-  int W, TH;          // tile width (interior points of a row) and height
-  int ntp;            // tiles per region level
-  int ntiles;         // regional tiles (lall * kall * ntp)
-  int nblocks;        // + 2 * kall pole blocks
-  int lds;            // LDS elements (real) per block
-};
-
-inline TileGeom tile_geom(const Dims& d, int per_corner) {
-  TileGeom t;
-  t.W = d.g - 2;
-  t.TH = 256 / t.W;
-  if (t.TH < 1) t.TH = 1;
-  t.ntp = (t.W + t.TH - 1) / t.TH;
-  t.ntiles = d.lall * d.kall * t.ntp;
-  t.nblocks = t.ntiles + 2 * d.kall;
-  t.lds = per_corner * (t.W + 1) * (t.TH + 1);
-  return t;
-}
-
-// tile decode: region l, level k, first row j0
-struct TileAt {
-  int l, k, j0, rows;
-};
-
-NH_HD inline TileAt tile_at(const Dims& d, const TileGeom& tg, int blk) {
-  TileAt t;
-  const int plane = blk / tg.ntp;
-  const int tile = blk - plane * tg.ntp;
-  t.l = plane / d.kall;
-  t.k = plane - t.l * d.kall;
-  t.j0 = 1 + tile * tg.TH;
-  t.rows = (d.g - 1 - t.j0 < tg.TH) ? d.g - 1 - t.j0 : tg.TH;   // rows j0..j0+rows-1 <= g-2
-  return t;
-}
-
-// ----------------------------------------------------------------------------
-// stencil point kernels on staged tiles: the fields a point kernel P reads on
-// its 7-point stencil (P::kNStage of them; P::stage_ptr(f, k) positions field
-// f so that level k's addresses read the level P needs there) are staged for
-// the tile's rows j0-1 .. j0+rows (on the levels where P::stage_level holds);
-// every cell of the tile then runs P::at with a loader that reads them from
-// LDS.  Rows of a region level are contiguous, so
-// the staged copy is the address range [base0, base0 + (rows+2)*g) and a
-// stencil address b maps to b - base0.  Pole levels run P on the pole centre.
-// ----------------------------------------------------------------------------
-template <class P>
-struct StagedPointT {
-  using LdsT = real;
-  static constexpr bool kStage = true;
-  static constexpr const char* kName = P::kName;
-  P pk;
-  TileGeom tg;
-  NH_HD int sf() const { return (tg.TH + 2) * pk.d.g; }
-  NH_HD long base0(const TileAt& t) const {
-    const long g = pk.d.g;
-    return (long)(t.l * pk.d.kall + t.k) * g * g + (long)(t.j0 - 1) * g;
-  }
-  NH_HD void phase0(int blk, int tid, real* lds) const {
-    if (blk >= tg.ntiles) return;
-    const TileAt t = tile_at(pk.d, tg, blk);
-    if (!pk.stage_level(t.k)) return;     // P::at does not read the stencil on this level
-    const long b0 = base0(t);
-    const int npl = (t.rows + 2) * pk.d.g;
-    for (int idx = tid; idx < P::kNStage * npl; idx += 256) {
-      const int f = idx / npl, e = idx - f * npl;
-      lds[f * sf() + e] = pk.stage_ptr(f, t.k)[b0 + e];
-    }
-  }
-  NH_HD void phase1(int, int, real*) const {}
-  NH_HD void phase2(int blk, int tid, const real* lds) const {
-    const Dims& d = pk.d;
-    if (blk >= tg.ntiles) {
-      if (tid == 0) pk(d.lall * d.kall + (blk - tg.ntiles), 0);
-      return;
-    }
-    const TileAt t = tile_at(d, tg, blk);
-    const int ti = tid % tg.W, tj = tid / tg.W;
-    if (tj >= t.rows) return;
-    const int g = d.g, i = ti + 1, j = t.j0 + tj;
-    Pt p;
-    p.pole = false; p.inner = true;
-    p.i = i; p.j = j; p.l = t.l; p.k = t.k; p.v = 0; p.lp = 0;
-    p.ks = (long)g * g;
-    p.a = ((long)(t.l * d.kall + t.k) * g + j) * g + i;
-    p.ci = ((long)t.l * g + j) * g + i;
-    const long b0 = base0(t);
-    const int s = sf();
-    pk.at(p, [&](int f, long b) { return lds[f * s + (b - b0)]; });
-  }
-};
-
-// Staging pays where the stencil loads are 8-byte (the FP64 form: 10-20 %
-// faster on MI355X at gl07); with 4-byte fields the direct point kernel is as
-// fast or faster.
-template <class X, class P>
-void run_staged(X& x, const P& pk) {
-  if (sizeof(real) == sizeof(float)) {
-    x.run_pts(pk, pk.d);
-    return;
-  }
-  StagedPointT<P> f;
-  f.pk = pk;
-  f.tg = tile_geom(pk.d, 0);
-  x.run_tiles(f, f.tg.nblocks, P::kNStage * (f.tg.TH + 2) * pk.d.g);
-}
 
 // ----------------------------------------------------------------------------
 // divergence damping as column tiles.  A block owns a TX x TY tile of one
