@@ -263,6 +263,26 @@ NH_HD inline bool src_of(const Dims& d, const Pt& x, int m, long* a, long* ci) {
   return true;
 }
 
+// The points the column-tile transposes leave out, t < border_threads(d): with
+// t < lall * kall * 4 (g - 1) border point e of plane t / (4 (g - 1)), going
+// round the region (j = 0, i = g - 1, j = g - 1, i = 0); then the pole points.
+inline long border_threads(const Dims& d) { return (long)d.lall * d.kall * 4 * (d.g - 1) + 2L * d.kall * 6; }
+NH_HD inline bool border_pt(const Dims& d, long t, Pt& p) {
+  const int g = d.g, per = 4 * (g - 1);
+  const long nb = (long)d.lall * d.kall * per;
+  if (t < nb) {
+    const int plane = (int)(t / per), e = (int)(t - (long)plane * per);
+    int i, j;
+    if (e < g - 1) { i = e; j = 0; }
+    else if (e < 2 * (g - 1)) { i = g - 1; j = e - (g - 1); }
+    else if (e < 3 * (g - 1)) { i = g - 1 - (e - 2 * (g - 1)); j = g - 1; }
+    else { i = 0; j = g - 1 - (e - 3 * (g - 1)); }
+    return pt_of(d, plane, j * g + i, p);
+  }
+  const long u = t - nb;
+  return pt_of(d, d.lall * d.kall + (int)(u / 6), (int)(u % 6), p);
+}
+
 // -lap transposed, gather form: ib[q](x) += -sum over the compute points a
 // whose stencil holds x of clap(a, m) ob[q](a) (both hyperdiffusion passes)
 // (the interior points run as column tiles, LapTC; this functor's 1-D form
@@ -274,32 +294,9 @@ struct NegLapGA {
   int nq;
   const real* ob[6];
   real* ib[6];
-  NH_HD void operator()(int plane, int x) const {
-    Pt p;
-    if (!pt_of(d, plane, x, p)) return;
-    point(p);
-  }
-  // t < lall * kall * 4 (g - 1): border point e of plane t / (4 (g - 1)),
-  // going round the region (j = 0, i = g - 1, j = g - 1, i = 0); then the
-  // pole points
-  NH_HD long border_threads() const { return (long)d.lall * d.kall * 4 * (d.g - 1) + 2L * d.kall * 6; }
   NH_HD void operator()(long t) const {
-    const int g = d.g, per = 4 * (g - 1);
-    const long nb = (long)d.lall * d.kall * per;
     Pt p;
-    if (t < nb) {
-      const int plane = (int)(t / per), e = (int)(t - (long)plane * per);
-      int i, j;
-      if (e < g - 1) { i = e; j = 0; }
-      else if (e < 2 * (g - 1)) { i = g - 1; j = e - (g - 1); }
-      else if (e < 3 * (g - 1)) { i = g - 1 - (e - 2 * (g - 1)); j = g - 1; }
-      else { i = 0; j = g - 1 - (e - 3 * (g - 1)); }
-      if (!pt_of(d, plane, j * g + i, p)) return;
-    } else {
-      const long u = t - nb;
-      if (!pt_of(d, d.lall * d.kall + (int)(u / 6), (int)(u % 6), p)) return;
-    }
-    point(p);
+    if (border_pt(d, t, p)) point(p);
   }
   NH_HD void point(const Pt& p) const {
     const long a = p.a;
@@ -1046,9 +1043,32 @@ struct Path1A {
     for (int q = 0; q < 3; ++q) gb[q] = -vb[q] * dt;
     proj_t(xx, c.RADIUS, gb);
   }
-  NH_HD void operator()(int plane, int x) const {
+  // the folded ghost rows of a compute point at kmin or kmax (address a): their
+  // bars onto the point's output bar vt and the densities
+  NH_HD void ghost_terms(long a, long ks, int k, real vt[3]) const {
+    real rnb = real(0.0);
+    for (int s2 = 0; s2 < 2; ++s2) {
+      if (s2 == 0 ? k != d.kmin : k != d.kmax) continue;
+      const bool top = (s2 == 1);
+      const long ag = top ? a + ks : a - ks;     // the ghost row
+      const real sgn = top ? real(1.0) : -real(1.0);
+      const real rgn = prog[a], rgg = prog[ag];
+      real rgb = real(0.0);
+      for (int q = 0; q < 3; ++q) {
+        const real vb = dv_b[q][ag];
+        const real vn = dv[q][a];
+        rgb += sgn * vb * vn / rgn;
+        rnb -= sgn * vb * vn * rgg / (rgn * rgn);
+        vt[q] += sgn * vb * rgg / rgn;
+      }
+      prog_b[ag] += rgb;
+    }
+    prog_b[a] += rnb;
+  }
+  // region borders and pole points (the interior: Path1TC)
+  NH_HD void operator()(long t) const {
     Pt p;
-    if (!pt_of(d, plane, x, p)) return;
+    if (!border_pt(d, t, p)) return;
     const long NF = d.NF, a = p.a, ks = p.ks;
     const int kmin = d.kmin, kmax = d.kmax, k = p.k;
     const real RovCV = c.Rdry / c.CVdry;
@@ -1090,24 +1110,7 @@ struct Path1A {
     }
     real vt[3];
     for (int q = 0; q < 3; ++q) vt[q] = dv_b[q][a];
-    real rnb = real(0.0);
-    for (int s2 = 0; s2 < 2; ++s2) {
-      if (s2 == 0 ? k != kmin : k != kmax) continue;
-      const bool top = (s2 == 1);
-      const long ag = top ? a + ks : a - ks;     // the ghost row
-      const real sgn = top ? real(1.0) : -real(1.0);
-      const real rgn = prog[a], rgg = prog[ag];
-      real rgb = real(0.0);
-      for (int q = 0; q < 3; ++q) {
-        const real vb = dv_b[q][ag];
-        const real vn = dv[q][a];
-        rgb += sgn * vb * vn / rgn;
-        rnb -= sgn * vb * vn * rgg / (rgn * rgn);
-        vt[q] += sgn * vb * rgg / rgn;
-      }
-      prog_b[ag] += rgb;
-    }
-    prog_b[a] += rnb;
+    if (k == kmin || k == kmax) ghost_terms(a, ks, k, vt);
     for (int q = 0; q < 3; ++q) {
       ps_b[1 + q][a] += vt[q];
       gT_b[(1 + q) * NF + a] += vt[q] * dt;

@@ -9,6 +9,7 @@
 // reverse order.  The tracer masses are held at progq (see nh_adjoint.h).
 #pragma once
 
+#include "nh_adjcol.h"
 #include "nh_adjoint.h"
 #include "nh_engine.h"
 #include "nh_tracer_adj.h"
@@ -111,7 +112,7 @@ void lap_adj(X& x, const Context& ctx, const NegLapGA& l) {
   for (int q = 0; q < N; ++q) { cs.op.ob[q] = l.ob[q]; cs.op.ib[q] = l.ib[q]; }
   cs.cg = sg;
   x.run_cols(cs, sg.nblocks, decltype(cs)::lds_elems(sg));
-  x.run(l, l.border_threads());
+  x.run(l, border_threads(ctx.d));
 }
 
 // reverse of one small step: ck = its input split state, nx = its output
@@ -191,7 +192,13 @@ void small_step_adj(X& x, const Context& ctx, const real* prog, real* const ck[6
     for (int q = 0; q < 6; ++q) f.ps_b[q] = psb2[q];
     for (int q = 0; q < 3; ++q) { f.dv[q] = dvn[q]; f.dv_b[q] = dvb[q]; f.dd_b[q] = ddvb[q]; }
     f.prog_b = prog_b; f.gT_b = gTb;
-    x.run_pts(f, d);
+    // interior points as column tiles, then the border and pole points
+    ColStencil<Path1TC> cs;
+    cs.op.pk = f;
+    cs.op.d = d;
+    cs.cg = st_geom(d);
+    x.run_cols(cs, cs.cg.nblocks, decltype(cs)::lds_elems(cs.cg));
+    x.run(f, border_threads(d));
   }
   real* vb[4] = {psb2[1], psb2[2], psb2[3], psb2[4]};
   divdamp_adj(x, ctx, ddvb, vb);
