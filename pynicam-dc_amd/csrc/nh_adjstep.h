@@ -581,13 +581,7 @@ int tracer_step_adj(X& x, const Context& ctx, const real* prog, const real* prog
     // forward: first half step (also the vertical flux and rhog1), then the
     // horizontal step up to its output rqh
     x.d2d(rq1, q0, NF * sizeof(real));
-    {
-      TrcVert1 f;
-      f.d = d; f.c = ctx.c; f.G = ctx.G;
-      f.dt = dt; f.rw_mean = prog + 4 * NF; f.rhog_in = prog; f.frhog = frhog;
-      f.flxv = flxv; f.rhog1 = rhog1; f.rhogq = rq1; f.nq = 1; f.limiter = lim;
-      x.run(f, nc);
-    }
+    trc_first_half(x, ctx, rq1, 1, dt, prog + 4 * NF, prog, frhog);
     if (iq == 0) {
       TrcRhog2 f;
       f.d = d; f.c = ctx.c; f.G = ctx.G;

@@ -57,7 +57,7 @@ enum WsField {
   W_GQ = 79,              // 3  gradient of the mixing ratio
   W_QA = 82,              // 3  upwind face values (faces 0..2)
   W_QOUT = 85,            // 2  limiter outflow bounds
-  W_RQ = 87,              // 1  tracer after the horizontal step
+  W_RQ = 87,              // 1  tracer after the horizontal step (adjoint)
   W_HV = 88,              // 3  horizontal divergences of the small-step momentum
   W_KIN = 91,             // 1  kinetic energy of the small-step state
   W_NFIELDS = 92
@@ -396,28 +396,36 @@ void divdamp(X& x, const Context& ctx, const real* vx, const real* vy, const rea
 // tracer transport with the time-mean mass fluxes of the last stage
 // (mod_dynamics.py:2346-2461 -> mod_src_tracer.py:83-1228)
 // ----------------------------------------------------------------------------
+// the first vertical half step of nq tracers: flux and density into the
+// workspace, the tracers in place
+template <class X>
+void trc_first_half(X& x, const Context& ctx, real* rhogq, int nq, double dt, const real* rw_mean,
+                    const real* rhog_in, const real* frhog) {
+  TrcFlux f0;
+  f0.d = ctx.d; f0.G = ctx.G;
+  f0.dt = (real)dt;
+  f0.rw_mean = rw_mean; f0.rhog_in = rhog_in; f0.frhog = frhog;
+  f0.flxv = ctx.field(W_FLXV); f0.rhog1 = ctx.field(W_RHOG1);
+  x.run_pts(f0, ctx.d);
+  TrcVert1 f;
+  f.d = ctx.d; f.c = ctx.c; f.G = ctx.G;
+  f.dt = (real)dt;
+  f.rw_mean = rw_mean; f.rhog_in = rhog_in; f.frhog = frhog;
+  f.rhogq = rhogq;
+  f.limiter = ctx.c.THUBURN_LIM;
+  x.run(f, nq * f.columns());
+}
+
 // pm: mass fluxes (rhog, rhogvx, rhogvy, rhogvz, rhogw) with field stride NF;
 // rhog_in: density at the start of the step; frhog: density tendency
 template <class X>
 void tracer_transport(X& x, const Context& ctx, real* progq, int nq, double dt, const real* pm,
                       const real* rhog_in, const real* frhog) {
   const Dims& d = ctx.d;
-  const long NF = d.NF, nc = ncols(d);
+  const long NF = d.NF;
   real* rhog1 = ctx.field(W_RHOG1);
   real* rhog2 = ctx.field(W_RHOG2);
-  real* flxv = ctx.field(W_FLXV);
-  {
-    TrcVert1 f;
-    f.d = d; f.c = ctx.c; f.G = ctx.G;
-    f.dt = (real)dt;
-    f.rw_mean = pm + 4 * NF;
-    f.rhog_in = rhog_in;
-    f.frhog = frhog;
-    f.flxv = flxv; f.rhog1 = rhog1;
-    f.rhogq = progq; f.nq = nq;
-    f.limiter = ctx.c.THUBURN_LIM;
-    x.run(f, nc);
-  }
+  trc_first_half(x, ctx, progq, nq, dt, pm + 4 * NF, rhog_in, frhog);
   real* fa[3] = {ctx.field(W_FA), ctx.field(W_FA + 1), ctx.field(W_FA + 2)};
   real* xc[9];
   for (int q = 0; q < 9; ++q) xc[q] = ctx.field(W_XC + q);
@@ -440,9 +448,15 @@ void tracer_transport(X& x, const Context& ctx, real* progq, int nq, double dt, 
   real* gq[3] = {ctx.field(W_GQ), ctx.field(W_GQ + 1), ctx.field(W_GQ + 2)};
   real* qa[3] = {ctx.field(W_QA), ctx.field(W_QA + 1), ctx.field(W_QA + 2)};
   real* qout[2] = {ctx.field(W_QOUT), ctx.field(W_QOUT + 1)};
-  real* rqh = ctx.field(W_RQ);
+  // tracers after the horizontal step: the second vertical half step runs for
+  // groups of kGroup tracers at once (one column thread per tracer, which a
+  // single tracer's columns are too few for: 0.7 waves per SIMD at gl06).  The
+  // group's fields are the second hyperdiffusion pass's, dead by now.
+  constexpr int kGroup = 6;
+  real* rqg = ctx.field(W_HDB);
   for (int iq = 0; iq < nq; ++iq) {
     real* rq = progq + (long)iq * NF;
+    real* rqh = rqg + (long)(iq % kGroup) * NF;
     {
       TrcGradQ f;
       f.d = d; f.G = ctx.G;
@@ -479,13 +493,14 @@ void tracer_transport(X& x, const Context& ctx, real* progq, int nq, double dt, 
       for (int q = 0; q < 9; ++q) f.xc[q] = xc[q];
       x.run_pts(f, d);
     }
-    {
+    if (iq % kGroup == kGroup - 1 || iq == nq - 1) {
+      const int n = iq % kGroup + 1;
       TrcVert2 f;
       f.d = d; f.c = ctx.c; f.G = ctx.G;
-      f.dt = (real)dt; f.flxv = flxv; f.rhog2 = rhog2; f.frhog = frhog;
-      f.in = rqh; f.out = rq;
+      f.dt = (real)dt; f.flxv = ctx.field(W_FLXV); f.rhog2 = rhog2; f.frhog = frhog;
+      f.in = rqg; f.out = progq + (long)(iq + 1 - n) * NF;
       f.limiter = ctx.c.THUBURN_LIM;
-      x.run(f, nc);
+      x.run(f, n * f.columns());
     }
   }
 }

@@ -1,11 +1,12 @@
 // Tracer transport of the last RK stage: MIURA2004 flux form with the
 // Thuburn (1996) limiters (nhm/dynamics/mod_src_tracer.py:83-1228).
 //
-//   vertical half step   TrcVert (phase 1, every column, all tracers in place)
+//   vertical half step   TrcFlux (fluxes, density), TrcVert1 (every column, all
+//                        tracers in place)
 //   horizontal step      TrcHFlux (arc mass fluxes, mass centroids), TrcRhog2,
 //                        then per tracer TrcGradQ -> halo -> TrcRemap -> TrcQout
 //                        -> halo -> TrcApply
-//   vertical half step   TrcVert (phase 2, compute cells, per tracer)
+//   vertical half step   TrcVert2 (compute cells, a group of tracers)
 //
 // The face mass fluxes of the reference's flx_h(i, j, face) are formed on the
 // fly from one value per hexagon arc: face 0/1/2 of (i, j) is the AI/AIJ/AJ arc
@@ -37,25 +38,44 @@ NH_HD inline real upwind_mask(real ch) { return real(0.5) - nsign(real(0.5), ch 
 
 // ----------------------------------------------------------------------------
 // vertical half step of one tracer column (mod_src_tracer.py:420-533 and the
-// limiter mod_src_tracer.py:1909-2074), streamed in k
+// limiter mod_src_tracer.py:1909-2074), streamed in k.  A column is a serial
+// chain over its levels; the loads of level k + 3 go out while level k is formed
+// (in place is allowed: every element is loaded once, before its store).
+// den(k), flx(k): density and vertical mass flux; fr(k): the density tendency,
+// from which dvk(fr, den) forms the divergence term.
 // ----------------------------------------------------------------------------
-template <class DEN, class FLX, class DV>
+template <class DEN, class FLX, class FR, class DVK>
 NH_HD inline void vert_sweep(const Geo& G, int kmin, int kmax, const real* in, real* out, long base, long ks,
-                             DEN den, FLX flx, DV dv, bool limiter, bool clipneg) {
-  auto ck0 = [&](int k) -> real { return (k >= kmin && k <= kmax) ? -flx(k) / den(k) * G.rdgz[k] : real(0.0); };
-  real r_km1 = in[base + (kmin - 1) * ks];
-  real r_k = in[base + kmin * ks];
+                             DEN den, FLX flx, FR fr, DVK dvk, bool limiter, bool clipneg) {
+  struct Lev {
+    real r, den, flx, fr;   // tracer, density, flux at kk; tendency at kk - 1
+  };
+  auto load = [&](int kk) {
+    const int k2 = (kk > kmax + 1) ? kmax + 1 : kk;   // past the top: not used
+    return Lev{ld_own(in + base + (long)k2 * ks), den(k2), flx(k2), fr(k2 - 1)};
+  };
+  auto ck0 = [&](int k, real f, real dn) -> real {
+    return (k >= kmin && k <= kmax) ? -f / dn * G.rdgz[k] : real(0.0);
+  };
+  Lev n1 = load(kmin + 1), n2 = load(kmin + 2), n3 = load(kmin + 3);
+  const real r_km1 = ld_own(in + base + (long)(kmin - 1) * ks);
+  real r_k = ld_own(in + base + (long)kmin * ks);
+  real den_k = den(kmin);
   real q_km1 = r_km1 / den(kmin - 1);
-  real q_k = r_k / den(kmin);
+  real q_k = r_k / den_k;
   real omin_prev = real(0.0), omax_prev = real(0.0);
   real qh_prev = real(0.0);      // limited face value at k-1 (zero at kmin)
   real r_prev = r_km1;
-  real c0_k = ck0(kmin);
+  real f_km1 = real(0.0), f_k = flx(kmin);
+  real c0_k = ck0(kmin, f_k, den_k);
   for (int k = kmin; k <= kmax; ++k) {
-    const real r_kp1 = in[base + (k + 1) * ks];
-    const real q_kp1 = r_kp1 / den(k + 1);
-    const real c0_kp1 = ck0(k + 1);
-    const real c1_k = flx(k + 1) / den(k) * G.rdgz[k];
+    const Lev c = n1;
+    n1 = n2;
+    n2 = n3;
+    n3 = load(k + 4);
+    const real q_kp1 = c.r / c.den;
+    const real c0_kp1 = ck0(k + 1, c.flx, c.den);
+    const real c1_k = c.flx / den_k * G.rdgz[k];
     real qh = G.afact[k] * q_k + G.bfact[k] * q_km1;
     real omin = real(0.0), omax = real(0.0);
     if (limiter) {
@@ -72,7 +92,7 @@ NH_HD inline void vert_sweep(const Geo& G, int kmin, int kmax, const real* in, r
       const real CQmin = inL * c0_k * minL + inU * c1_k * minU;
       const real CQmax = inL * c0_k * maxL + inU * c1_k * maxU;
       const real zsw = real(0.5) - nsign(real(0.5), nabs(Cout) - NH_EPS);
-      const real dk = dv(k);
+      const real dk = dvk(c.fr, den_k);
       omin = ((q_k - nmax) + nmax * (Cin + Cout - dk) - CQmax) / (Cout + zsw) * (real(1.0) - zsw) + q_k * zsw;
       omax = ((q_k - nmin) + nmin * (Cin + Cout - dk) - CQmin) / (Cout + zsw) * (real(1.0) - zsw) + q_k * zsw;
       if (k > kmin) qh = inL * clip(qh, omin_prev, omax_prev) + (real(1.0) - inL) * clip(qh, omin, omax);
@@ -80,32 +100,68 @@ NH_HD inline void vert_sweep(const Geo& G, int kmin, int kmax, const real* in, r
     if (k == kmin) qh = real(0.0);
     if (k > kmin) {
       // update of level k-1 with the face values at k-1 and k
-      real o = r_prev - (flx(k) * qh - flx(k - 1) * qh_prev) * G.rdgz[k - 1];
+      real o = r_prev - (f_k * qh - f_km1 * qh_prev) * G.rdgz[k - 1];
       if (clipneg && o > -real(1.0e-10) && o < real(0.0)) o = real(0.0);
-      out[base + (k - 1) * ks] = o;
+      out[base + (long)(k - 1) * ks] = o;
     }
     omin_prev = omin;
     omax_prev = omax;
     qh_prev = qh;
     r_prev = r_k;
-    r_k = r_kp1;
+    r_k = c.r;
     q_km1 = q_k;
     q_k = q_kp1;
     c0_k = c0_kp1;
+    den_k = c.den;
+    f_km1 = f_k;
+    f_k = c.flx;
   }
   {
-    real o = r_prev - (flx(kmax + 1) * real(0.0) - flx(kmax) * qh_prev) * G.rdgz[kmax];
+    // f_k, f_km1: the fluxes at kmax + 1 and kmax
+    real o = r_prev - (f_k * real(0.0) - f_km1 * qh_prev) * G.rdgz[kmax];
     if (clipneg && o > -real(1.0e-10) && o < real(0.0)) o = real(0.0);
-    out[base + kmax * ks] = o;
+    out[base + (long)kmax * ks] = o;
   }
-  out[base + (kmin - 1) * ks] = real(0.0);
-  out[base + (kmax + 1) * ks] = real(0.0);
+  out[base + (long)(kmin - 1) * ks] = real(0.0);
+  out[base + (long)(kmax + 1) * ks] = real(0.0);
 }
 
-// Phase 1: vertical flux of the mean mass flux, half-step density and the
-// first vertical half step of every tracer, on every column (the horizontal
-// step reads halo values; computing them here equals filling them).
-// (kernels/tracervertflux.py:44-122)
+// the vertical mass flux of a half step from the mean flux rw (zero at the
+// boundaries), and the density after the first one
+NH_HD inline real half_flux(const Dims& d, const real* rw, long b, long ks, int k, real dt) {
+  return (k >= d.kmin + 1 && k <= d.kmax) ? (real(0.0) + ldc(rw + b + (long)k * ks) * real(1.0)) * real(0.5) * dt
+                                          : real(0.0);
+}
+
+// Phase 1, one thread per point: vertical flux of the mean mass flux and the
+// half-step density (kernels/tracervertflux.py:44-122), on every column
+struct TrcFlux {
+  static constexpr const char* kName = "trc_flux";
+  Dims d; Geo G;
+  real dt;
+  const real* rw_mean;    // time-mean rhogw
+  const real* rhog_in;    // density at the start of the large step
+  const real* frhog;      // hyperdiffusion density tendency
+  real* flxv;             // out
+  real* rhog1;            // out
+  NH_HD void operator()(int plane, int x) const {
+    Pt p;
+    if (!pt_of(d, plane, x, p)) return;
+    const long a = p.a, ks = p.ks, b = a - (long)p.k * ks;
+    const int k = p.k;
+    const real f = half_flux(d, rw_mean, b, ks, k, dt);
+    real r;
+    if (k < d.kmin) r = rhog_in[a + ks];
+    else if (k > d.kmax) r = rhog_in[a - ks];
+    else r = rhog_in[a] - (half_flux(d, rw_mean, b, ks, k + 1, dt) - f) * G.rdgz[k] + real(0.0) * frhog[a] * dt;
+    flxv[a] = f;
+    rhog1[a] = r;
+  }
+};
+
+// Phase 1: first vertical half step of every tracer, on every column (the
+// horizontal step reads halo values; computing them here equals filling
+// them), one thread per column and tracer.
 struct TrcVert1 {
   static constexpr const char* kName = "trc_vert1";
   Dims d; Consts c; Geo G;
@@ -113,35 +169,25 @@ struct TrcVert1 {
   const real* rw_mean;    // time-mean rhogw
   const real* rhog_in;    // density at the start of the large step
   const real* frhog;      // hyperdiffusion density tendency
-  real* flxv;             // out
-  real* rhog1;            // out
   real* rhogq;            // nq tracer fields, in place
-  int nq;
   int limiter;
+  NH_HD long columns() const { return d.nreg + 12; }
+  // t < nq * columns()
   NH_HD void operator()(long t) const {
-    Cell cl = cell_of(d, t);
+    const long q = t / columns();
+    const Cell cl = cell_of(d, t - q * columns());
     const long ks = cl.ks, b = cl.base;
-    const int kmin = d.kmin, kmax = d.kmax;
-    auto flx = [&](int k) -> real {
-      return (k >= kmin + 1 && k <= kmax) ? (real(0.0) + rw_mean[b + k * ks] * real(1.0)) * real(0.5) * dt : real(0.0);
-    };
-    for (int k = 0; k < d.kall; ++k) flxv[b + k * ks] = flx(k);
-    for (int k = kmin; k <= kmax; ++k)
-      rhog1[b + k * ks] = rhog_in[b + k * ks] - (flx(k + 1) - flx(k)) * G.rdgz[k] + real(0.0) * frhog[b + k * ks] * dt;
-    rhog1[b + (kmin - 1) * ks] = rhog_in[b + kmin * ks];
-    rhog1[b + (kmax + 1) * ks] = rhog_in[b + kmax * ks];
-    auto den = [&](int k) { return rhog_in[b + k * ks]; };
-    auto dv = [&](int k) { return real(0.0) * frhog[b + k * ks] / rhog_in[b + k * ks] * dt; };
-    for (int q = 0; q < nq; ++q) {
-      real* f = rhogq + (long)q * d.NF;
-      vert_sweep(G, kmin, kmax, f, f, b, ks, den, flx, dv, limiter != 0, false);
-    }
+    real* f = rhogq + q * d.NF;
+    vert_sweep(G, d.kmin, d.kmax, f, f, b, ks, [&](int k) { return ldc(rhog_in + b + (long)k * ks); },
+               [&](int k) { return half_flux(d, rw_mean, b, ks, k, dt); },
+               [&](int k) { return ldc(frhog + b + (long)k * ks); },
+               [&](real fr, real den) { return real(0.0) * fr / den * dt; }, limiter != 0, false);
   }
 };
 
-// Phase 2: second vertical half step of one tracer on the compute cells,
-// with the density after the horizontal step, and the small-negative clip
-// (mod_src_tracer.py:947-1204).
+// Phase 2: second vertical half step of nq tracers on the compute cells, with
+// the density after the horizontal step, and the small-negative clip
+// (mod_src_tracer.py:947-1204), one thread per column and tracer.
 struct TrcVert2 {
   static constexpr const char* kName = "trc_vert2";
   Dims d; Consts c; Geo G;
@@ -149,17 +195,21 @@ struct TrcVert2 {
   const real* flxv;
   const real* rhog2;
   const real* frhog;
-  const real* in;     // tracer after the horizontal step
-  real* out;          // tracer field
+  const real* in;     // nq tracers after the horizontal step
+  real* out;          // nq tracer fields
   int limiter;
+  NH_HD long columns() const { return d.nreg + 12; }
+  // t < nq * columns()
   NH_HD void operator()(long t) const {
-    Cell cl = cell_of(d, t);
+    const long q = t / columns();
+    const Cell cl = cell_of(d, t - q * columns());
     if (cl.pole ? cl.v != 0 : !cl.inner) return;
     const long ks = cl.ks, b = cl.base;
-    auto flx = [&](int k) { return flxv[b + k * ks]; };
-    auto den = [&](int k) { return rhog2[b + k * ks]; };
-    auto dv = [&](int k) { return real(0.0) * frhog[b + k * ks] / rhog2[b + k * ks] * dt; };
-    vert_sweep(G, d.kmin, d.kmax, in, out, b, ks, den, flx, dv, limiter != 0, true);
+    vert_sweep(G, d.kmin, d.kmax, in + q * d.NF, out + q * d.NF, b, ks,
+               [&](int k) { return ldc(rhog2 + b + (long)k * ks); },
+               [&](int k) { return ldc(flxv + b + (long)k * ks); },
+               [&](int k) { return ldc(frhog + b + (long)k * ks); },
+               [&](real fr, real den) { return real(0.0) * fr / den * dt; }, limiter != 0, true);
   }
 };
 
