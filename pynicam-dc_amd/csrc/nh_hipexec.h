@@ -134,7 +134,10 @@ class HipExec {
   template <class F>
   void run(const F& f, long n) {
     if (n <= 0) return;
-    const int bs = 256;
+    // up to 512 wavefronts (the column sweeps at gl05) go out as single-wave blocks,
+    // one per CU: trc_vert1 64 -> 54 us, vi_main_v 22 -> 20 at gl05 FP64; from gl06 on
+    // four-wave blocks are level or faster (trc_vert1 66 against 75 us at gl06 FP64)
+    const int bs = (n <= 512L * 64) ? 64 : 256;
     long nb = (n + bs - 1) / bs;
     hipEvent_t* pair = timed(F::kName) ? next_pair(F::kName) : nullptr;
     if (pair) note(hipEventRecord(pair[0], s_), "hipEventRecord");

@@ -841,6 +841,8 @@ template <int NK>
 struct ViMainV {
   static constexpr const char* kName = "vi_main_v";
   static constexpr int kUnroll = NK > 0 ? NK : 4;
+  // rows in flight (the registers of the z40 form leave room for one of 8-byte fields)
+  static constexpr int kAhead = (NK > 0 && sizeof(real) == 8) ? 1 : 3;
   Dims d; Consts c; Geo G;
   double dt;
   const real* ps[6];
@@ -874,6 +876,22 @@ struct ViMainV {
     real* __restrict__ Xo = out;
     const int N = (NK > 0) ? NK : kmax - kmin;
     double ub[NK > 0 ? NK : 1], gb[NK > 0 ? NK : 1];
+    // what a level's row needs, loaded kAhead levels before it is formed: the
+    // sweep is a serial chain of few waves per SIMD (2.7 at gl07, 0.2 at gl05), so
+    // a row must not wait for its loads.  At gl06 the scratch form (NK = 0) 139 -> 75 us
+    // mixed with 57 levels, 77 -> 49 FP64 with 33; the z40 form is at the HBM rate
+    // at gl07 (90 us mixed, 130 FP64) and at the chain's latency at gl05 (20 us).
+    struct Row {
+      real pe, hv1, pg, gT0, hv0, gT4, pw;
+      double mc, mu, ml;
+    };
+    auto load = [&](int n) {
+      const long a = b + (long)(kmin + 1 + (n < N ? n : N - 1)) * ks;
+      return Row{ldc(pe + a), ldc(hv1 + a), ldc(pg + a), ldc(gT0 + a), ldc(hv0 + a), ldc(gT4 + a), ldc(pw + a),
+                 ldc(mc + a), ldc(mu + a), ldc(ml + a)};
+    };
+    Row ahead[kAhead];
+    for (int q = 0; q < kAhead; ++q) ahead[q] = load(q);
     // level k-1 values, starting at kmin
     long am = b + (long)kmin * ks;
     double pe_m = pe[am], hv1_m = hv1[am], pg_m = pg[am];
@@ -883,14 +901,17 @@ struct ViMainV {
     for (int n = 0; n < N; ++n) {
       const int k = kmin + 1 + n;
       const long a = am + ks;
-      const double pe_k = pe[a], hv1_k = hv1[a], pg_k = pg[a];
-      const double gr_k = (double)gT0[a] + (-(double)hv0[a] - (0.0 - 0.0) * V.rdgz[k]);
-      const double sw = (double)gT4[a] + 0.0 * C.ALPHA;
-      const double A = ((double)pw[a] * C.ALPHA + dt * sw) * 1.0;
+      const Row r = ahead[0];
+      for (int q = 0; q + 1 < kAhead; ++q) ahead[q] = ahead[q + 1];
+      ahead[kAhead - 1] = load(n + kAhead);
+      const double pe_k = r.pe, hv1_k = r.hv1, pg_k = r.pg;
+      const double gr_k = (double)r.gT0 + (-(double)r.hv0 - (0.0 - 0.0) * V.rdgz[k]);
+      const double sw = (double)r.gT4 + 0.0 * C.ALPHA;
+      const double A = ((double)r.pw * C.ALPHA + dt * sw) * 1.0;
       const double B = (pe_k * RovCV + dt * hv1_k) * 1.0 - (pe_m * RovCV + dt * hv1_m) * 1.0;
       const double Cc = (pg_k + dt * gr_k) * 1.0 * V.afact[k] + (pg_m + dt * gr_m) * 1.0 * V.bfact[k];
       double S = (A - B * dt * V.rdgzh[k] - Cc * dt * C.GRAV) * CVovRt2;
-      const double mc_k = mc[a], ml_k = ml[a], mu_k = mu[a];
+      const double mc_k = r.mc, ml_k = r.ml, mu_k = r.mu;
       if (n == 0) S = S - ml_k * (0.0 * 1.0);
       if (n == N - 1) S = S - mu_k * (-0.0 * 1.0);
       double u;
