@@ -594,7 +594,7 @@ int tracer_step_adj(X& x, const Context& ctx, const real* prog, const real* prog
       TrcGradQ f;
       f.d = d; f.G = ctx.G; f.rq = rq1; f.rhog1 = rhog1;
       for (int q = 0; q < 3; ++q) f.gq[q] = gq[q];
-      x.run_pts(f, d);
+      run_oper7<3>(x, d, f, SrcRatio{rq1, rhog1}, ctx.G.cgrad, gq);
     }
     halo(x, ctx, gq, 3);
     {

@@ -153,6 +153,87 @@ struct ColStencil {
   }
 };
 
+// The single 7-point operators as column operators, P the point kernel that does
+// the pole centres: the Laplacian of one field (NC = 1), the gradient of one
+// (NC = 3) and the divergence of three, with their 7 or 21 coefficients in
+// registers.  A source SRC gives the staged values: src(f, o).  Gradient of a
+// tracer's mixing ratio at gl06 z60 FP64: 81 us per launch as points (21 coefficients
+// and 7 quotients per level), 39 as tiles; Laplacian, gradient and divergence at gl06
+// z40 FP64 in turn: 115 against 73.
+template <class P, class SRC, int NC>
+struct Oper7C {
+  static constexpr const char* kName = P::kName;
+  static constexpr bool kDiv = SRC::kFields == 3;
+  static constexpr int kNS = SRC::kFields;
+  static constexpr bool kMapped = false;
+  P pk;
+  SRC src;
+  Dims d;
+  const real* coef;
+  real* out[kDiv ? 1 : NC];
+  struct Col {
+    real c[NC][7];
+  };
+  struct Stg {};
+  struct Pre {};
+  NH_HD void begin(Pre&) const {}
+  NH_HD void init_stage(long, Stg&) const {}
+  NH_HD void pre(int, unsigned, const Stg&, Pre&) const {}
+  NH_HD bool stage_level(int) const { return true; }
+  NH_HD void stage(int, unsigned o, unsigned, const Stg&, real* v) const {
+    for (int f = 0; f < kNS; ++f) v[f] = src(f, o);
+  }
+  NH_HD void stage_own(int k, unsigned o, const Stg& sg, const Pre&, real* v) const { stage(k, o, o, sg, v); }
+  NH_HD void init_col(long ci, Col& col) const {
+    for (int dd = 0; dd < NC; ++dd)
+      for (int m = 0; m < 7; ++m) col.c[dd][m] = rc(coef, d.nreg, dd * 7 + m, ci);
+  }
+  NH_HD void pole(int pb) const { pk(d.lall * d.kall + pb, 0); }
+  // per direction the sum over the neighbours in stencil order, as lap7, grad7 and div7
+  template <class NB>
+  NH_HD void point(int, unsigned o, const Col& col, Pre&, NB nb) const {
+    real s[NC];
+    for (int dd = 0; dd < NC; ++dd) {
+      s[dd] = col.c[dd][0] * nb(0, kDiv ? dd : 0);
+#pragma unroll
+      for (int m = 1; m < 7; ++m) s[dd] = s[dd] + col.c[dd][m] * nb(m, kDiv ? dd : 0);
+    }
+    if constexpr (kDiv) {
+      at_off(out[0], o) = s[0] + s[1] + s[2];
+    } else {
+      for (int dd = 0; dd < NC; ++dd) at_off(out[dd], o) = s[dd];
+    }
+  }
+};
+
+// staged as they are: one field or three
+template <int N>
+struct SrcFields {
+  static constexpr int kFields = N;
+  const real* f[N];
+  NH_HD real operator()(int n, unsigned o) const { return at_off(f[n], o); }
+};
+
+// mixing ratio of a tracer mass
+struct SrcRatio {
+  static constexpr int kFields = 1;
+  const real* rq;
+  const real* rhog;
+  NH_HD real operator()(int, unsigned o) const { return at_off(rq, o) / at_off(rhog, o); }
+};
+
+template <int NC, class X, class P, class SRC>
+void run_oper7(X& x, const Dims& d, const P& pk, const SRC& src, const real* coef, real* const* out) {
+  ColStencil<Oper7C<P, SRC, NC>> cs;
+  cs.op.pk = pk;
+  cs.op.src = src;
+  cs.op.d = d;
+  cs.op.coef = coef;
+  for (int q = 0; q < (SRC::kFields == 3 ? 1 : NC); ++q) cs.op.out[q] = out[q];
+  cs.cg = st_geom(d);
+  x.run_cols(cs, cs.cg.nblocks, decltype(cs)::lds_elems(cs.cg));
+}
+
 // vi_main, horizontal part (ViMainH) as a column operator: the 21 divergence
 // coefficients in registers, the 8 stencil fields staged per level
 struct ViMainHC {

@@ -462,7 +462,7 @@ void tracer_transport(X& x, const Context& ctx, real* progq, int nq, double dt, 
       f.d = d; f.G = ctx.G;
       f.rq = rq; f.rhog1 = rhog1;
       for (int q = 0; q < 3; ++q) f.gq[q] = gq[q];
-      x.run_pts(f, d);
+      run_oper7<3>(x, d, f, SrcRatio{rq, rhog1}, ctx.G.cgrad, gq);
     }
     halo(x, ctx, gq, 3);
     {

@@ -97,8 +97,9 @@ int v_halo_fill(Context* c, void* const* fields, int nf, void* stream, std::stri
 
 int v_laplacian(Context* c, const void* scl, void* out, void* stream, std::string* err) {
   NHX x(c->device, stream, &c->prof);
-  OpLapP f{c->d, c->G, (const real*)scl, (real*)out};
-  x.run_pts(f, c->d);
+  real* o[1] = {(real*)out};
+  const OpLapP f{c->d, c->G, (const real*)scl, o[0]};
+  run_oper7<1>(x, c->d, f, SrcFields<1>{{(const real*)scl}}, c->G.clap, o);
   if (x.check("nh_laplacian")) return failv(err, NH_ERR_DEVICE, x.message());
   return 0;
 }
@@ -106,16 +107,18 @@ int v_laplacian(Context* c, const void* scl, void* out, void* stream, std::strin
 int v_divergence(Context* c, const void* vx, const void* vy, const void* vz, void* out, void* stream,
                  std::string* err) {
   NHX x(c->device, stream, &c->prof);
-  OpDivP f{c->d, c->G, (const real*)vx, (const real*)vy, (const real*)vz, (real*)out};
-  x.run_pts(f, c->d);
+  real* o[1] = {(real*)out};
+  const OpDivP f{c->d, c->G, (const real*)vx, (const real*)vy, (const real*)vz, o[0]};
+  run_oper7<3>(x, c->d, f, SrcFields<3>{{(const real*)vx, (const real*)vy, (const real*)vz}}, c->G.cdiv, o);
   if (x.check("nh_divergence")) return failv(err, NH_ERR_DEVICE, x.message());
   return 0;
 }
 
 int v_gradient(Context* c, const void* scl, void* gx, void* gy, void* gz, void* stream, std::string* err) {
   NHX x(c->device, stream, &c->prof);
-  OpGradP f{c->d, c->G, (const real*)scl, (real*)gx, (real*)gy, (real*)gz};
-  x.run_pts(f, c->d);
+  real* o[3] = {(real*)gx, (real*)gy, (real*)gz};
+  const OpGradP f{c->d, c->G, (const real*)scl, o[0], o[1], o[2]};
+  run_oper7<3>(x, c->d, f, SrcFields<1>{{(const real*)scl}}, c->G.cgrad, o);
   if (x.check("nh_gradient")) return failv(err, NH_ERR_DEVICE, x.message());
   return 0;
 }
@@ -151,13 +154,13 @@ int v_op(Context* c, int op, const void* const* in, void* const* out, double dt,
       break;
     }
     case OP_HDIFF: {
-      // the two passes into the step workspace (cleared, so that columns no
-      // halo fill reaches hold zeros), a halo fill after each, then the tendency
+      // the two passes into the step workspace (cleared first where the halo map
+      // leaves columns out, so that those hold zeros), then the tendency
       const real* prog = R(0);
       const real* diag = R(1);
       real* hda = c->field(W_HDA);
       real* hdb = c->field(W_HDB);
-      x.run(FillZero{hda}, 12 * NF);
+      if (!c->halo_full) x.run(FillZero{hda}, 12 * NF);
       const StageFields sf{hda, hdb, c->field(W_GT), c->field(W_ETHTOT), c->dfield(D_MC)};
       hdiff_passes(x, *c, prog, diag, sf, false, true);
       HDiffTendOp f;

@@ -61,6 +61,7 @@ template <int NK>
 struct ViSolveOp {
   static constexpr const char* kName = "op_vi_solve";
   static constexpr int kMax = NK > 0 ? NK : 78;
+  static constexpr int kUnroll = NK > 0 ? NK : 2;
   Dims d; Consts c; Geo G;
   double dt;
   const real *rhogw, *rhogw0, *preg0, *rhog0, *Srho, *Sw, *Spre;
@@ -78,25 +79,48 @@ struct ViSolveOp {
     const double rw_top = (double)rhogw[b + (long)(kmax + 1) * ks];
     double u[kMax], gm[kMax];
     double beta = 0.0;
+    // rows are loaded kAhead levels before they are formed (as in ViMainV): a
+    // column's loads overlap its divisions.  gl06 z40 mixed: 43.8 -> 35.4 us.
+    // Plain loads, since out may be any of the inputs
+    struct Row {
+      real rw0, sw, p0, sp, r0, sr;
+      double mc, mu, ml;
+    };
+    constexpr int kAhead = (NK > 0 && sizeof(real) == 8) ? 1 : 3;
+    auto load = [&](int n) {
+      const long a = b + (long)(kmin + 1 + (n < N ? n : N - 1)) * ks;
+      return Row{rhogw0[a], Sw[a], preg0[a], Spre[a], rhog0[a], Srho[a], Mc[a], Mu[a], Ml[a]};
+    };
+    Row ahead[kAhead];
+    for (int q = 0; q < kAhead; ++q) ahead[q] = load(q);
+    const long am = b + (long)kmin * ks;
+    double e_m = (double)preg0[am] + dt * (double)Spre[am], r_m = (double)rhog0[am] + dt * (double)Srho[am];
+    double mu_m = 0.0;
+#pragma unroll kUnroll
     for (int n = 0; n < N; ++n) {
       const int k = kmin + 1 + n;
-      const long a = b + (long)k * ks, am = a - ks;
-      const double A = (double)rhogw0[a] * C.ALPHA + dt * (double)Sw[a];
-      const double B = ((double)preg0[a] + dt * (double)Spre[a]) - ((double)preg0[am] + dt * (double)Spre[am]);
-      const double Cc = ((double)rhog0[a] + dt * (double)Srho[a]) * V.afact[k]
-                        + ((double)rhog0[am] + dt * (double)Srho[am]) * V.bfact[k];
+      const Row r = ahead[0];
+      for (int q = 0; q + 1 < kAhead; ++q) ahead[q] = ahead[q + 1];
+      ahead[kAhead - 1] = load(n + kAhead);
+      const double A = (double)r.rw0 * C.ALPHA + dt * (double)r.sw;
+      const double e_k = (double)r.p0 + dt * (double)r.sp, r_k = (double)r.r0 + dt * (double)r.sr;
+      const double B = e_k - e_m;
+      const double Cc = r_k * V.afact[k] + r_m * V.bfact[k];
       double S = (A - B * dt * V.rdgzh[k] - Cc * dt * C.GRAV) * CVovRt2;
-      if (n == 0) S = S - Ml[a] * rw_bot;
-      if (n == N - 1) S = S - Mu[a] * rw_top;
+      if (n == 0) S = S - r.ml * rw_bot;
+      if (n == N - 1) S = S - r.mu * rw_top;
       if (n == 0) {
-        beta = Mc[a];
+        beta = r.mc;
         u[0] = S / beta;
       } else {
-        const double g = Mu[am] / beta;
-        beta = Mc[a] - Ml[a] * g;
-        u[n] = (S - Ml[a] * u[n - 1]) / beta;
+        const double g = mu_m / beta;
+        beta = r.mc - r.ml * g;
+        u[n] = (S - r.ml * u[n - 1]) / beta;
         gm[n] = g;
       }
+      mu_m = r.mu;
+      e_m = e_k;
+      r_m = r_k;
     }
     // the rows below kmin and above kmax+1 are copied, the boundary rows scaled by GSGAM2H
     if (out != rhogw) {

@@ -15,7 +15,8 @@
 NH_BEGIN
 
 // ----------------------------------------------------------------------------
-// single operators (tests and callers of the C-ABI)
+// single operators (tests and callers of the C-ABI): the pole centres; the
+// regional points run as Oper7C
 // ----------------------------------------------------------------------------
 struct OpLapP {
   static constexpr const char* kName = "oprt_laplacian";
@@ -24,8 +25,8 @@ struct OpLapP {
   real* o;
   NH_HD void operator()(int plane, int x) const {
     Pt p;
-    if (!pt_of(d, plane, x, p) || !pt_compute(p)) return;
-    o[p.a] = p.pole ? lap_pl(G, p.lp, s, p.a) : lap7(G, d.nreg, p.ci, s, p.a, d.g);
+    if (!pt_of(d, plane, x, p) || !p.pole || p.v != 0) return;
+    o[p.a] = lap_pl(G, p.lp, s, p.a);
   }
 };
 
@@ -36,17 +37,10 @@ struct OpDivP {
   real* o;
   NH_HD void operator()(int plane, int x) const {
     Pt p;
-    if (!pt_of(d, plane, x, p) || !pt_compute(p)) return;
+    if (!pt_of(d, plane, x, p) || !p.pole || p.v != 0) return;
     const long a = p.a;
-    if (p.pole) {
-      o[a] = div_pl(G, p.lp, [&](int v) { return vx[a + v]; }, [&](int v) { return vy[a + v]; },
-                    [&](int v) { return vz[a + v]; });
-    } else {
-      long off[7];
-      stencil_offsets(d.g, off);
-      o[a] = div7(G, d.nreg, p.ci, [&](int m) { return vx[a + off[m]]; }, [&](int m) { return vy[a + off[m]]; },
-                  [&](int m) { return vz[a + off[m]]; });
-    }
+    o[a] = div_pl(G, p.lp, [&](int v) { return vx[a + v]; }, [&](int v) { return vy[a + v]; },
+                  [&](int v) { return vz[a + v]; });
   }
 };
 
@@ -57,10 +51,9 @@ struct OpGradP {
   real *ox, *oy, *oz;
   NH_HD void operator()(int plane, int x) const {
     Pt p;
-    if (!pt_of(d, plane, x, p) || !pt_compute(p)) return;
+    if (!pt_of(d, plane, x, p) || !p.pole || p.v != 0) return;
     real o[3];
-    if (p.pole) grad_pl(G, p.lp, s, p.a, o);
-    else grad7(G, d.nreg, p.ci, s, p.a, d.g, o);
+    grad_pl(G, p.lp, s, p.a, o);
     ox[p.a] = o[0];
     oy[p.a] = o[1];
     oz[p.a] = o[2];

@@ -367,41 +367,25 @@ struct TrcRhog2 {
 };
 
 // gradient of q = rhogq / rhog1 (OPRT_gradient, kernels/oprtgradient.py:45-88)
+// the pole centres (the regional points run as Oper7C over SrcRatio)
 struct TrcGradQ {
   static constexpr const char* kName = "trc_gradq";
   Dims d; Geo G;
   const real* rq;
   const real* rhog1;
   real* gq[3];
-  // the column launch walks every level; the point launch (more threads, the
-  // levels being independent) does one
-  NH_HD void operator()(long t) const { levels(cell_of(d, t), 0, d.kall); }
   NH_HD void operator()(int plane, int x) const {
     Pt p;
-    if (pt_of(d, plane, x, p)) levels(cell_of_pt(p), p.k, p.k + 1);
-  }
-  NH_HD void levels(const Cell& cl, int k0, int k1) const {
-    if (cl.pole ? cl.v != 0 : !cl.inner) return;
-    long nb[7];
-    int nn = neighbours(d, cl, nb);
-    for (int k = k0; k < k1; ++k) {
-      const long kk = k * cl.ks;
-      real qv[7];
-      for (int m = 0; m < nn; ++m) qv[m] = rq[nb[m] + kk] / rhog1[nb[m] + kk];
-      for (int dd = 0; dd < 3; ++dd) {
-        real acc;
-        if (cl.pole) {
-          acc = real(0.0);
-          for (int v = 0; v < 6; ++v) {
-            real pv = G.cgrad_pl[(v * 2 + cl.lp) * 3 + dd] * qv[v];
-            acc = (v == 0) ? pv : acc + pv;
-          }
-        } else {
-          acc = rcp(G.cgrad, d.nreg, dd * 7, cl.ci) * qv[0];
-          for (int m = 1; m < 7; ++m) acc = acc + rcp(G.cgrad, d.nreg, dd * 7 + m, cl.ci) * qv[m];
-        }
-        gq[dd][cl.base + kk] = acc;
+    if (!pt_of(d, plane, x, p) || !p.pole || p.v != 0) return;
+    real qv[6];
+    for (int v = 0; v < 6; ++v) qv[v] = rq[p.a + v] / rhog1[p.a + v];
+    for (int dd = 0; dd < 3; ++dd) {
+      real acc = real(0.0);
+      for (int v = 0; v < 6; ++v) {
+        const real pv = G.cgrad_pl[(v * 2 + p.lp) * 3 + dd] * qv[v];
+        acc = (v == 0) ? pv : acc + pv;
       }
+      gq[dd][p.a] = acc;
     }
   }
 };
