@@ -598,32 +598,32 @@ int tracer_step_adj(X& x, const Context& ctx, const real* prog, const real* prog
     }
     halo(x, ctx, gq, 3);
     {
-      TrcRemap f;
-      f.d = d; f.c = ctx.c; f.G = ctx.G;
-      f.dt = dt; f.rq = rq1; f.rhog1 = rhog1;
-      for (int q = 0; q < 3; ++q) { f.gq[q] = gq[q]; f.fa[q] = fa[q]; f.qa[q] = qa[q]; }
+      TrcRemap<1> f;
+      f.d = d; f.G = ctx.G;
+      f.dt = dt; f.rq[0] = rq1; f.rhog1 = rhog1;
+      for (int q = 0; q < 3; ++q) { f.gq[0][q] = gq[q]; f.fa[q] = fa[q]; f.qa[0][q] = qa[q]; }
       for (int q = 0; q < 9; ++q) f.xc[q] = xc[q];
       x.run_pts(f, d);
     }
     if (lim) {
       TrcQout f;
-      f.d = d; f.c = ctx.c; f.G = ctx.G;
+      f.d = d; f.G = ctx.G;
       f.dt = dt; f.rq = rq1; f.rhog1 = rhog1; f.frhog = frhog;
       for (int q = 0; q < 3; ++q) f.fa[q] = fa[q];
       f.qout[0] = qout[0]; f.qout[1] = qout[1];
-      x.run_pts(f, d);
+      run_trc_qout(x, f);
       halo(x, ctx, qout, 2);
     }
     {
       TrcApply f;
-      f.d = d; f.c = ctx.c; f.G = ctx.G;
+      f.d = d; f.G = ctx.G;
       f.dt = dt; f.rq = rq1; f.rhog1 = rhog1;
       for (int q = 0; q < 3; ++q) { f.fa[q] = fa[q]; f.qa[q] = qa[q]; }
       f.qout[0] = qout[0]; f.qout[1] = qout[1];
       f.out = rqh; f.limiter = lim;
       for (int q = 0; q < 3; ++q) f.gq[q] = gq[q];
       for (int q = 0; q < 9; ++q) f.xc[q] = xc[q];
-      x.run_pts(f, d);
+      run_trc_apply(x, f);
     }
     // reverse; rq_b becomes the bar of rq1 once the compute cells' bars have
     // gone through the second half step (elsewhere rq1 passes unchanged)

@@ -18,6 +18,7 @@
 #include <cstdint>
 #include <cstring>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "nh_step.h"
@@ -25,6 +26,7 @@
 #include "nh_point.h"
 #include "nh_tile.h"
 #include "nh_colstencil.h"
+#include "nh_trccol.h"
 #include "nh_budget.h"
 #include "nh_trcadv.h"
 #include "../../include/nicamhip.h"
@@ -454,44 +456,68 @@ void tracer_transport(X& x, const Context& ctx, real* progq, int nq, double dt, 
   // group's fields are the second hyperdiffusion pass's, dead by now.
   constexpr int kGroup = 6;
   real* rqg = ctx.field(W_HDB);
+  // gradients and face values of a second tracer at a time, so that one remap
+  // launch serves both: in the first hyperdiffusion pass's fields, whose halo
+  // columns are written here and must be filled again before they are read
+  const int npair = ctx.halo_full ? 2 : 1;
+  real* gqp[2][3];
+  real* qap[2][3];
+  for (int q = 0; q < 3; ++q) {
+    gqp[0][q] = gq[q];
+    qap[0][q] = qa[q];
+    gqp[1][q] = ctx.field(W_HDA + q);
+    qap[1][q] = ctx.field(W_HDA + 3 + q);
+  }
+  auto remap = [&](auto f, int iq, auto n_) {
+    constexpr int n = decltype(n_)::value;
+    real* gall[6];
+    f.d = d; f.G = ctx.G;
+    f.dt = (real)dt; f.rhog1 = rhog1;
+    for (int m = 0; m < n; ++m) {
+      real* rq = progq + (long)(iq + m) * NF;
+      TrcGradQ t;
+      t.d = d; t.G = ctx.G;
+      t.rq = rq; t.rhog1 = rhog1;
+      f.rq[m] = rq;
+      for (int q = 0; q < 3; ++q) {
+        t.gq[q] = gall[m * 3 + q] = gqp[m][q];
+        f.gq[m][q] = gqp[m][q];
+        f.qa[m][q] = qap[m][q];
+      }
+      run_oper7<3>(x, d, t, SrcRatio{rq, rhog1}, ctx.G.cgrad, gqp[m]);
+    }
+    for (int q = 0; q < 3; ++q) f.fa[q] = fa[q];
+    for (int q = 0; q < 9; ++q) f.xc[q] = xc[q];
+    halo(x, ctx, gall, 3 * n);
+    x.run_pts(f, d);
+  };
   for (int iq = 0; iq < nq; ++iq) {
     real* rq = progq + (long)iq * NF;
     real* rqh = rqg + (long)(iq % kGroup) * NF;
-    {
-      TrcGradQ f;
-      f.d = d; f.G = ctx.G;
-      f.rq = rq; f.rhog1 = rhog1;
-      for (int q = 0; q < 3; ++q) f.gq[q] = gq[q];
-      run_oper7<3>(x, d, f, SrcRatio{rq, rhog1}, ctx.G.cgrad, gq);
-    }
-    halo(x, ctx, gq, 3);
-    {
-      TrcRemap f;
-      f.d = d; f.c = ctx.c; f.G = ctx.G;
-      f.dt = (real)dt; f.rq = rq; f.rhog1 = rhog1;
-      for (int q = 0; q < 3; ++q) { f.gq[q] = gq[q]; f.fa[q] = fa[q]; f.qa[q] = qa[q]; }
-      for (int q = 0; q < 9; ++q) f.xc[q] = xc[q];
-      x.run_pts(f, d);
+    const int m = iq % npair;
+    if (m == 0) {
+      if (npair == 2 && iq + 1 < nq) remap(TrcRemap<2>{}, iq, std::integral_constant<int, 2>{});
+      else remap(TrcRemap<1>{}, iq, std::integral_constant<int, 1>{});
     }
     if (ctx.c.THUBURN_LIM) {
       TrcQout f;
-      f.d = d; f.c = ctx.c; f.G = ctx.G;
+      f.d = d; f.G = ctx.G;
       f.dt = (real)dt; f.rq = rq; f.rhog1 = rhog1; f.frhog = frhog;
       for (int q = 0; q < 3; ++q) f.fa[q] = fa[q];
       f.qout[0] = qout[0]; f.qout[1] = qout[1];
-      x.run_pts(f, d);
+      run_trc_qout(x, f);
       halo(x, ctx, qout, 2);
     }
     {
       TrcApply f;
-      f.d = d; f.c = ctx.c; f.G = ctx.G;
+      f.d = d; f.G = ctx.G;
       f.dt = (real)dt; f.rq = rq; f.rhog1 = rhog1;
-      for (int q = 0; q < 3; ++q) { f.fa[q] = fa[q]; f.qa[q] = qa[q]; }
+      for (int q = 0; q < 3; ++q) { f.fa[q] = fa[q]; f.qa[q] = qap[m][q]; }
       f.qout[0] = qout[0]; f.qout[1] = qout[1];
       f.out = rqh; f.limiter = ctx.c.THUBURN_LIM;
-      for (int q = 0; q < 3; ++q) f.gq[q] = gq[q];
+      for (int q = 0; q < 3; ++q) f.gq[q] = gqp[m][q];
       for (int q = 0; q < 9; ++q) f.xc[q] = xc[q];
-      x.run_pts(f, d);
+      run_trc_apply(x, f);
     }
     if (iq % kGroup == kGroup - 1 || iq == nq - 1) {
       const int n = iq % kGroup + 1;

@@ -393,64 +393,80 @@ struct TrcGradQ {
 // ----------------------------------------------------------------------------
 // upwind face values (horizontal_remap, mod_src_tracer.py:1642-1843)
 // ----------------------------------------------------------------------------
+// N tracers (1 or 2) per launch: the nine centroid fields and the three fluxes,
+// two thirds of what one tracer reads, are read once for both.  Every load of a
+// point is issued before the first use and an arc that does not exist is a
+// select (its operands are in bounds), so a point waits once for memory.
+// gl06 z60 FP64, two tracers: 274 us as two point launches of one, 121 as a pair
+// (28 fields, 131 us at the streaming rate from memory); gl07 z40 mixed, one
+// tracer: 176 -> 148 us.
+template <int N>
 struct TrcRemap {
   static constexpr const char* kName = "trc_remap";
-  Dims d; Consts c; Geo G;
+  Dims d; Geo G;
   real dt;
-  const real* rq;
+  const real* rq[N];
   const real* rhog1;
-  const real* gq[3];
+  const real* gq[N][3];
   const real* fa[3];
   const real* xc[9];
-  real* qa[3];
-  // the column launch walks every level; the point launch (more threads, the
-  // levels being independent) does one
-  NH_HD void operator()(long t) const { levels(cell_of(d, t), 0, d.kall); }
+  real* qa[N][3];
   NH_HD void operator()(int plane, int x) const {
     Pt p;
-    if (pt_of(d, plane, x, p)) levels(cell_of_pt(p), p.k, p.k + 1);
-  }
-  NH_HD void levels(const Cell& cl, int k0, int k1) const {
-    if (cl.pole) {
-      if (cl.v == 0) return;
+    if (!pt_of(d, plane, x, p)) return;
+    if (p.pole) {
+      if (p.v == 0) return;
       // pole arc v: upwind value from the pole centre or spoke v
-      const int lp = cl.lp, v = cl.v;
-      const long R0 = d.R + (long)lp * d.kall * 6;
+      const int lp = p.lp, v = p.v;
       const real* xp0 = G.gx_pl + (0 * 2 + lp) * 3;
       const real* xpv = G.gx_pl + (v * 2 + lp) * 3;
-      for (int k = k0; k < k1; ++k) {
-        const long a0 = R0 + k * 6, av = a0 + v;
-        const real q0 = rq[a0] / rhog1[a0], qv = rq[av] / rhog1[av];
-        const real xcx = xc[0][av], xcy = xc[1][av], xcz = xc[2][av];
-        const real qap = q0 + gq[0][a0] * (xcx - xp0[0]) + gq[1][a0] * (xcy - xp0[1]) + gq[2][a0] * (xcz - xp0[2]);
-        const real qam = qv + gq[0][av] * (xcx - xpv[0]) + gq[1][av] * (xcy - xpv[1]) + gq[2][av] * (xcz - xpv[2]);
-        const real ch = fa[0][av] * G.rarea_pl[lp] * dt / rhog1[a0];
-        const real cm = upwind_mask(ch);
-        qa[0][av] = cm * qam + (real(1.0) - cm) * qap;
+      const long av = p.a, a0 = av - v;
+      const real xcx = xc[0][av], xcy = xc[1][av], xcz = xc[2][av];
+      const real ch = fa[0][av] * G.rarea_pl[lp] * dt / rhog1[a0];
+      const real cm = upwind_mask(ch);
+      for (int n = 0; n < N; ++n) {
+        const real* const* gn = gq[n];
+        const real q0 = rq[n][a0] / rhog1[a0], qv = rq[n][av] / rhog1[av];
+        const real qap = q0 + gn[0][a0] * (xcx - xp0[0]) + gn[1][a0] * (xcy - xp0[1]) + gn[2][a0] * (xcz - xp0[2]);
+        const real qam = qv + gn[0][av] * (xcx - xpv[0]) + gn[1][av] * (xcy - xpv[1]) + gn[2][av] * (xcz - xpv[2]);
+        qa[n][0][av] = cm * qam + (real(1.0) - cm) * qap;
       }
       return;
     }
-    const int g = d.g, i = cl.i, j = cl.j;
+    const int g = d.g, i = p.i, j = p.j;
     if (i > g - 2 || j > g - 2) return;
-    const long nreg = d.nreg, ci = cl.ci, ks = cl.ks;
+    const long nreg = d.nreg, ci = p.ci;
+    const unsigned o = byte_off(p.a);
     // neighbour across each arc: AI (i+1, j), AIJ (i+1, j+1), AJ (i, j+1)
-    const long noff[3] = {1, 1 + (long)g, (long)g};
-    const bool valid[3] = {j >= 1, true, i >= 1};
-    for (int k = k0; k < k1; ++k) {
-      const long a = cl.base + k * ks;
-      for (int arc = 0; arc < 3; ++arc) {
-        if (!valid[arc]) { qa[arc][a] = real(0.0); continue; }
-        const long an = a + noff[arc];
-        const long cn = ci + noff[arc];
-        const real xcx = xc[arc * 3 + 0][a], xcy = xc[arc * 3 + 1][a], xcz = xc[arc * 3 + 2][a];
-        const real qc = rq[a] / rhog1[a], qn = rq[an] / rhog1[an];
-        const real qap = qc + gq[0][a] * (xcx - rcp(G.gx, nreg, 0, ci)) + gq[1][a] * (xcy - rcp(G.gx, nreg, 1, ci))
-                         + gq[2][a] * (xcz - rcp(G.gx, nreg, 2, ci));
-        const real qam = qn + gq[0][an] * (xcx - rcp(G.gx, nreg, 0, cn)) + gq[1][an] * (xcy - rcp(G.gx, nreg, 1, cn))
-                         + gq[2][an] * (xcz - rcp(G.gx, nreg, 2, cn));
-        const real ch = fa[arc][a] * rcp(G.rarea, nreg, 0, ci) * dt / rhog1[a];
-        const real cm = upwind_mask(ch);
-        qa[arc][a] = cm * qam + (real(1.0) - cm) * qap;
+    const int noff[3] = {1, 1 + g, g};
+    real xv[9], fv[3], r[4], xg[4][3], q[N][4], gv[N][4][3];
+    for (int m = 0; m < 9; ++m) xv[m] = at_off(xc[m], o);
+    for (int m = 0; m < 3; ++m) fv[m] = at_off(fa[m], o);
+    const real ra = rcp(G.rarea, nreg, 0, ci);
+    for (int m = 0; m < 4; ++m) {
+      const int of = m ? noff[m - 1] : 0;
+      r[m] = at_off(rhog1 + of, o);
+      for (int dd = 0; dd < 3; ++dd) xg[m][dd] = rcp(G.gx, nreg, dd, ci + of);
+      for (int n = 0; n < N; ++n) {
+        q[n][m] = at_off(rq[n] + of, o);
+        for (int dd = 0; dd < 3; ++dd) gv[n][m][dd] = at_off(gq[n][dd] + of, o);
+      }
+    }
+    for (int n = 0; n < N; ++n)
+      for (int m = 0; m < 4; ++m) q[n][m] = q[n][m] / r[m];
+    for (int arc = 0; arc < 3; ++arc) {
+      const real ch = fv[arc] * ra * dt / r[0];
+      const real cm = upwind_mask(ch);
+      const bool valid = arc == 1 || (arc == 0 ? j >= 1 : i >= 1);
+      const real* xa = xv + arc * 3;
+      for (int n = 0; n < N; ++n) {
+        const real* g0 = gv[n][0];
+        const real* g1 = gv[n][arc + 1];
+        const real* x1 = xg[arc + 1];
+        const real qap = q[n][0] + g0[0] * (xa[0] - xg[0][0]) + g0[1] * (xa[1] - xg[0][1]) + g0[2] * (xa[2] - xg[0][2]);
+        const real qam = q[n][arc + 1] + g1[0] * (xa[0] - x1[0]) + g1[1] * (xa[1] - x1[1]) + g1[2] * (xa[2] - x1[2]);
+        const real s = cm * qam + (real(1.0) - cm) * qap;
+        at_off(qa[n][arc], o) = valid ? s : real(0.0);
       }
     }
   }
@@ -537,86 +553,109 @@ NH_HD inline void trc_cell(const Geo& G, const Dims& d, const Cell& cl, long a, 
   x.cmo[5] = upwind_mask(fa[2][o5] * rcp(G.rarea, nreg, 0, c5) * dt / rhog1[o5]);
 }
 
+// outflow bounds of a regional cell
+NH_HD inline void trc_qout_cell(const TrcCellCtx& x, bool pentagon, real dk, real& o0, real& o1) {
+  FaceBounds fb;
+  face_bounds(x.q, x.cmo, pentagon, fb);
+  real nmin = x.q[0], nmax = x.q[0];
+  real lo[6], hi[6];
+  for (int m = 0; m < 6; ++m) {
+    qin_of_cell(fb, m, lo[m], hi[m]);
+    nmin = dmin(nmin, lo[m]);
+    nmax = dmax(nmax, hi[m]);
+  }
+  real Cin = -real(0.0), Cout = -real(0.0), CQmin = -real(0.0), CQmax = -real(0.0);
+  for (int m = 0; m < 6; ++m) {
+    const real chm = (x.ch[m] < real(0.0)) ? x.ch[m] : real(0.0);
+    Cin = Cin + chm;
+    Cout = Cout + (x.ch[m] - chm);
+    CQmin = CQmin + chm * lo[m];
+    CQmax = CQmax + chm * hi[m];
+  }
+  const real zsw = real(0.5) - nsign(real(0.5), nabs(Cout) - NH_EPS);
+  const real qq = x.q[0];
+  o0 = (qq - CQmax - nmax * (real(1.0) - Cin - Cout + dk)) / (Cout + zsw) * (real(1.0) - zsw) + qq * zsw;
+  o1 = (qq - CQmin - nmin * (real(1.0) - Cin - Cout + dk)) / (Cout + zsw) * (real(1.0) - zsw) + qq * zsw;
+}
+
+// the pole centres (the regional cells run as TrcQoutC)
 struct TrcQout {
   static constexpr const char* kName = "trc_qout";
-  Dims d; Consts c; Geo G;
+  Dims d; Geo G;
   real dt;
   const real* rq;
   const real* rhog1;
   const real* frhog;
   const real* fa[3];
   real* qout[2];
-  // the column launch walks every level; the point launch (more threads, the
-  // levels being independent) does one
-  NH_HD void operator()(long t) const { levels(cell_of(d, t), 0, d.kall); }
   NH_HD void operator()(int plane, int x) const {
     Pt p;
-    if (pt_of(d, plane, x, p)) levels(cell_of_pt(p), p.k, p.k + 1);
-  }
-  NH_HD void levels(const Cell& cl, int k0, int k1) const {
-    if (cl.pole ? cl.v != 0 : !cl.inner) return;
-    for (int k = k0; k < k1; ++k) {
-      const long a = cl.base + k * cl.ks;
-      const real dk = real(1.0) * frhog[a] / rhog1[a] * dt;
-      if (cl.pole) {
-        const real ra = G.rarea_pl[cl.lp];
-        const real q0 = rq[a] / rhog1[a];
-        real qv[6];
-        for (int v = 1; v <= 5; ++v) qv[v] = rq[a + v] / rhog1[a + v];
-        real nmin = q0, nmax = q0, Cin = real(0.0), Cout = real(0.0), CQmin = real(0.0), CQmax = real(0.0);
-        for (int v = 1; v <= 5; ++v) {
-          const int vp = (v == 5) ? 1 : v + 1, vm = (v == 1) ? 5 : v - 1;
-          const real mn = dmin(dmin(dmin(q0, qv[v]), qv[vm]), qv[vp]);
-          const real mx = dmax(dmax(dmax(q0, qv[v]), qv[vm]), qv[vp]);
-          const real ch = fa[0][a + v] * ra * dt / rhog1[a];
-          const real cm = upwind_mask(ch);
-          const real lo = (cm == real(1.0)) ? mn : NH_BIG;
-          const real hi = (cm == real(1.0)) ? mx : -NH_BIG;
-          nmin = dmin(nmin, lo);
-          nmax = dmax(nmax, hi);
-          const real chm = cm * ch;
-          Cin = Cin + chm;
-          Cout = Cout + (ch - chm);
-          CQmin = CQmin + chm * lo;
-          CQmax = CQmax + chm * hi;
-        }
-        const real zsw = real(0.5) - nsign(real(0.5), nabs(Cout) - NH_EPS);
-        const real den = Cout + zsw, fac = real(1.0) - zsw;
-        qout[0][a] = (q0 - CQmax - nmax * (real(1.0) - Cin - Cout + dk)) / den * fac + q0 * zsw;
-        qout[1][a] = (q0 - CQmin - nmin * (real(1.0) - Cin - Cout + dk)) / den * fac + q0 * zsw;
-        continue;
-      }
-      TrcCellCtx x;
-      trc_cell(G, d, cl, a, dt, rq, rhog1, fa, x);
-      FaceBounds fb;
-      face_bounds(x.q, x.cmo, cl.i == 1 && cl.j == 1 && G.sgp[cl.l], fb);
-      real nmin = x.q[0], nmax = x.q[0];
-      real lo[6], hi[6];
-      for (int m = 0; m < 6; ++m) {
-        qin_of_cell(fb, m, lo[m], hi[m]);
-        nmin = dmin(nmin, lo[m]);
-        nmax = dmax(nmax, hi[m]);
-      }
-      real Cin = -real(0.0), Cout = -real(0.0), CQmin = -real(0.0), CQmax = -real(0.0);
-      for (int m = 0; m < 6; ++m) {
-        const real chm = (x.ch[m] < real(0.0)) ? x.ch[m] : real(0.0);
-        Cin = Cin + chm;
-        Cout = Cout + (x.ch[m] - chm);
-        CQmin = CQmin + chm * lo[m];
-        CQmax = CQmax + chm * hi[m];
-      }
-      const real zsw = real(0.5) - nsign(real(0.5), nabs(Cout) - NH_EPS);
-      const real qq = x.q[0];
-      qout[0][a] = (qq - CQmax - nmax * (real(1.0) - Cin - Cout + dk)) / (Cout + zsw) * (real(1.0) - zsw) + qq * zsw;
-      qout[1][a] = (qq - CQmin - nmin * (real(1.0) - Cin - Cout + dk)) / (Cout + zsw) * (real(1.0) - zsw) + qq * zsw;
+    if (!pt_of(d, plane, x, p) || !p.pole || p.v != 0) return;
+    const long a = p.a;
+    const real dk = real(1.0) * frhog[a] / rhog1[a] * dt;
+    const real ra = G.rarea_pl[p.lp];
+    const real q0 = rq[a] / rhog1[a];
+    real qv[6];
+    for (int v = 1; v <= 5; ++v) qv[v] = rq[a + v] / rhog1[a + v];
+    real nmin = q0, nmax = q0, Cin = real(0.0), Cout = real(0.0), CQmin = real(0.0), CQmax = real(0.0);
+    for (int v = 1; v <= 5; ++v) {
+      const int vp = (v == 5) ? 1 : v + 1, vm = (v == 1) ? 5 : v - 1;
+      const real mn = dmin(dmin(dmin(q0, qv[v]), qv[vm]), qv[vp]);
+      const real mx = dmax(dmax(dmax(q0, qv[v]), qv[vm]), qv[vp]);
+      const real ch = fa[0][a + v] * ra * dt / rhog1[a];
+      const real cm = upwind_mask(ch);
+      const real lo = (cm == real(1.0)) ? mn : NH_BIG;
+      const real hi = (cm == real(1.0)) ? mx : -NH_BIG;
+      nmin = dmin(nmin, lo);
+      nmax = dmax(nmax, hi);
+      const real chm = cm * ch;
+      Cin = Cin + chm;
+      Cout = Cout + (ch - chm);
+      CQmin = CQmin + chm * lo;
+      CQmax = CQmax + chm * hi;
     }
+    const real zsw = real(0.5) - nsign(real(0.5), nabs(Cout) - NH_EPS);
+    const real den = Cout + zsw, fac = real(1.0) - zsw;
+    qout[0][a] = (q0 - CQmax - nmax * (real(1.0) - Cin - Cout + dk)) / den * fac + q0 * zsw;
+    qout[1][a] = (q0 - CQmin - nmin * (real(1.0) - Cin - Cout + dk)) / den * fac + q0 * zsw;
   }
 };
+
+// limited outflow of a regional cell: sum over the faces of flux times limited
+// value.  qa: unlimited face values, q0, q1: outflow bounds on the stencil
+NH_HD inline real trc_outflow_cell(const TrcCellCtx& x, bool pentagon, const real qa[6], const real q0[7],
+                                   const real q1[7]) {
+  FaceBounds fb;
+  face_bounds(x.q, x.cmo, pentagon, fb);
+  // owner cell and downstream cell of the owner's face (stencil indices)
+  const int own[6] = {0, 0, 0, 4, 5, 6};
+  const int dst[6] = {1, 2, 3, 0, 0, 0};
+  real s_face[6];
+  for (int m = 0; m < 6; ++m) {
+    const real cm = fb.cm[m];
+    real loA, hiA, loB, hiB;     // A: owner side, B: downstream side
+    if (m < 3) {
+      qin_of_cell(fb, m, loA, hiA);
+      // the downstream cell sees the complementary mask
+      loB = cm * NH_BIG + (real(1.0) - cm) * fb.mn[m];
+      hiB = cm * (-NH_BIG) + (real(1.0) - cm) * fb.mx[m];
+    } else {
+      qin_of_owner(fb, m, loA, hiA);
+      qin_of_cell(fb, m, loB, hiB);
+    }
+    const real s = qa[m];
+    const real v1 = cm * clip(s, loA, hiA) + (real(1.0) - cm) * clip(s, loB, hiB);
+    const int o = own[m], dn = dst[m];
+    s_face[m] = cm * dmax(dmin(v1, q1[dn]), q0[dn]) + (real(1.0) - cm) * dmax(dmin(v1, q1[o]), q0[o]);
+  }
+  return x.f[0] * s_face[0] + x.f[1] * s_face[1] + x.f[2] * s_face[2] + x.f[3] * s_face[3] + x.f[4] * s_face[4]
+         + x.f[5] * s_face[5];
+}
 
 // limited face values and the flux-form update of rhogq (mod_src_tracer.py:2536-2660, :838-874)
 struct TrcApply {
   static constexpr const char* kName = "trc_apply";
-  Dims d; Consts c; Geo G;
+  Dims d; Geo G;
   real dt;
   const real* rq;
   const real* rhog1;
@@ -646,85 +685,48 @@ struct TrcApply {
     const real cm = upwind_mask(fm / rhog1[a]);
     return cm * am + (real(1.0) - cm) * ap;
   }
-  // the column launch walks every level; the point launch (more threads, the
-  // levels being independent) does one
-  NH_HD void operator()(long t) const { levels(cell_of(d, t), 0, d.kall); }
+  // with the limiter the pole centres only (the regional cells run as TrcApplyC)
   NH_HD void operator()(int plane, int x) const {
     Pt p;
-    if (pt_of(d, plane, x, p)) levels(cell_of_pt(p), p.k, p.k + 1);
-  }
-  NH_HD void levels(const Cell& cl, int k0, int k1) const {
-    if (cl.pole ? cl.v != 0 : !cl.inner) return;
-    const int g = d.g;
-    for (int k = k0; k < k1; ++k) {
-      const long a = cl.base + k * cl.ks;
-      if (!limiter) {
-        if (cl.pole) {
-          real r = rq[a];
-          for (int v = 1; v <= 5; ++v) r -= fa[0][a + v] * G.rarea_pl[cl.lp] * dt * qa[0][a + v];
-          out[a] = r;
-        } else {
-          real f[6], s[6];
-          for (int m = 0; m < 6; ++m) f[m] = face_flux(G, d, fa, a, cl.ci, cl.i, cl.j, cl.l, m, dt);
-          for (int m = 0; m < 6; ++m) s[m] = face_unlimited(cl, a, m, f[m]);
-          out[a] = rq[a] - (f[0] * s[0] + f[1] * s[1] + f[2] * s[2] + f[3] * s[3] + f[4] * s[4] + f[5] * s[5]);
-        }
-        continue;
-      }
-      if (cl.pole) {
-        const real ra = G.rarea_pl[cl.lp];
-        const real q0 = rq[a] / rhog1[a];
-        real qv[6];
-        for (int v = 1; v <= 5; ++v) qv[v] = rq[a + v] / rhog1[a + v];
-        real r = rq[a];
-        for (int v = 1; v <= 5; ++v) {
-          const int vp = (v == 5) ? 1 : v + 1, vm = (v == 1) ? 5 : v - 1;
-          const real mn = dmin(dmin(dmin(q0, qv[v]), qv[vm]), qv[vp]);
-          const real mx = dmax(dmax(dmax(q0, qv[v]), qv[vm]), qv[vp]);
-          const real fl = fa[0][a + v] * ra * dt;
-          const real cm = upwind_mask(fl / rhog1[a]);
-          const real lo0 = (cm == real(1.0)) ? mn : NH_BIG, hi0 = (cm == real(1.0)) ? mx : -NH_BIG;
-          const real lo1 = (cm == real(1.0)) ? NH_BIG : mn, hi1 = (cm == real(1.0)) ? -NH_BIG : mx;
-          real s = qa[0][a + v];
-          const real s0 = clip(s, lo0, hi0), s1 = clip(s, lo1, hi1);
-          s = cm * s0 + (real(1.0) - cm) * s1;
-          const real s2 = dmax(dmin(s, qout[1][a + v]), qout[0][a + v]);
-          const real s3 = dmax(dmin(s, qout[1][a]), qout[0][a]);
-          s = cm * s2 + (real(1.0) - cm) * s3;
-          r -= fl * s;
-        }
-        out[a] = r;
-        continue;
-      }
-      TrcCellCtx x;
-      trc_cell(G, d, cl, a, dt, rq, rhog1, fa, x);
-      FaceBounds fb;
-      face_bounds(x.q, x.cmo, cl.i == 1 && cl.j == 1 && G.sgp[cl.l], fb);
-      // owner cell, downstream cell of the owner's face, and the face's unlimited value
-      const long own[6] = {a, a, a, a - 1, a - 1 - g, a - g};
-      const long dst[6] = {a + 1, a + 1 + g, a + g, a, a, a};
-      const int arc[6] = {0, 1, 2, 0, 1, 2};
-      real s_face[6];
-      for (int m = 0; m < 6; ++m) {
-        const real cm = fb.cm[m];
-        real loA, hiA, loB, hiB;     // A: owner side, B: downstream side
-        if (m < 3) {
-          qin_of_cell(fb, m, loA, hiA);
-          // the downstream cell sees the complementary mask
-          loB = cm * NH_BIG + (real(1.0) - cm) * fb.mn[m];
-          hiB = cm * (-NH_BIG) + (real(1.0) - cm) * fb.mx[m];
-        } else {
-          qin_of_owner(fb, m, loA, hiA);
-          qin_of_cell(fb, m, loB, hiB);
-        }
-        const real s = qa[arc[m]][own[m]];
-        const real v1 = cm * clip(s, loA, hiA) + (real(1.0) - cm) * clip(s, loB, hiB);
-        const long o = own[m], dn = dst[m];
-        s_face[m] = cm * dmax(dmin(v1, qout[1][dn]), qout[0][dn]) + (real(1.0) - cm) * dmax(dmin(v1, qout[1][o]), qout[0][o]);
-      }
-      out[a] = rq[a] - (x.f[0] * s_face[0] + x.f[1] * s_face[1] + x.f[2] * s_face[2] + x.f[3] * s_face[3]
-                        + x.f[4] * s_face[4] + x.f[5] * s_face[5]);
+    if (!pt_of(d, plane, x, p) || !pt_compute(p)) return;
+    const long a = p.a;
+    if (!p.pole) {
+      if (limiter) return;
+      const Cell cl = cell_of_pt(p);
+      real f[6], s[6];
+      for (int m = 0; m < 6; ++m) f[m] = face_flux(G, d, fa, a, cl.ci, cl.i, cl.j, cl.l, m, dt);
+      for (int m = 0; m < 6; ++m) s[m] = face_unlimited(cl, a, m, f[m]);
+      out[a] = rq[a] - (f[0] * s[0] + f[1] * s[1] + f[2] * s[2] + f[3] * s[3] + f[4] * s[4] + f[5] * s[5]);
+      return;
     }
+    const real ra = G.rarea_pl[p.lp];
+    if (!limiter) {
+      real r = rq[a];
+      for (int v = 1; v <= 5; ++v) r -= fa[0][a + v] * ra * dt * qa[0][a + v];
+      out[a] = r;
+      return;
+    }
+    const real q0 = rq[a] / rhog1[a];
+    real qv[6];
+    for (int v = 1; v <= 5; ++v) qv[v] = rq[a + v] / rhog1[a + v];
+    real r = rq[a];
+    for (int v = 1; v <= 5; ++v) {
+      const int vp = (v == 5) ? 1 : v + 1, vm = (v == 1) ? 5 : v - 1;
+      const real mn = dmin(dmin(dmin(q0, qv[v]), qv[vm]), qv[vp]);
+      const real mx = dmax(dmax(dmax(q0, qv[v]), qv[vm]), qv[vp]);
+      const real fl = fa[0][a + v] * ra * dt;
+      const real cm = upwind_mask(fl / rhog1[a]);
+      const real lo0 = (cm == real(1.0)) ? mn : NH_BIG, hi0 = (cm == real(1.0)) ? mx : -NH_BIG;
+      const real lo1 = (cm == real(1.0)) ? NH_BIG : mn, hi1 = (cm == real(1.0)) ? -NH_BIG : mx;
+      real s = qa[0][a + v];
+      const real s0 = clip(s, lo0, hi0), s1 = clip(s, lo1, hi1);
+      s = cm * s0 + (real(1.0) - cm) * s1;
+      const real s2 = dmax(dmin(s, qout[1][a + v]), qout[0][a + v]);
+      const real s3 = dmax(dmin(s, qout[1][a]), qout[0][a]);
+      s = cm * s2 + (real(1.0) - cm) * s3;
+      r -= fl * s;
+    }
+    out[a] = r;
   }
 };
 
