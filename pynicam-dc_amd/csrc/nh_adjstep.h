@@ -568,11 +568,12 @@ int tracer_step_adj(X& x, const Context& ctx, const real* prog, const real* prog
   x.run(FillZero{frhog}, NF);
   {
     TrcHFlux f;
-    f.d = d; f.c = ctx.c; f.G = ctx.G;
+    f.d = d; f.G = ctx.G;
     f.dt = dt; f.pm = prog;
     for (int q = 0; q < 3; ++q) f.fa[q] = fa[q];
     for (int q = 0; q < 9; ++q) f.xc[q] = xc[q];
-    x.run_pts(f, d);
+    f.KC = chunk_levels((d.nreg + 255) / 256, d.kall, kColLevels);
+    x.run(f, f.threads());
   }
   halo_block_adj(x, ctx, progq_b, nq);   // the final halo fill of progq
   for (int iq = 0; iq < nq; ++iq) {

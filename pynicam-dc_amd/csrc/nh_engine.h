@@ -433,11 +433,12 @@ void tracer_transport(X& x, const Context& ctx, real* progq, int nq, double dt, 
   for (int q = 0; q < 9; ++q) xc[q] = ctx.field(W_XC + q);
   {
     TrcHFlux f;
-    f.d = d; f.c = ctx.c; f.G = ctx.G;
+    f.d = d; f.G = ctx.G;
     f.dt = (real)dt; f.pm = pm;
     for (int q = 0; q < 3; ++q) f.fa[q] = fa[q];
     for (int q = 0; q < 9; ++q) f.xc[q] = xc[q];
-    x.run_pts(f, d);
+    f.KC = chunk_levels((d.nreg + 255) / 256, d.kall, kColLevels);
+    x.run(f, f.threads());
   }
   {
     TrcRhog2 f;

@@ -217,98 +217,120 @@ struct TrcVert2 {
 // horizontal mass fluxes (mod_src_tracer.py:1376-1533)
 // ----------------------------------------------------------------------------
 // field layout of the arc quantities: fa[arc] (0.5 * rhov.HN of the arc), xc[arc*3+d]
+//
+// One thread per column and KC levels: its 30 coefficients stay in registers,
+// each of the four triangles is formed once for the arcs that share it, and all
+// loads of a level come before its 12 stores.  16 fields, 96 us at the streaming
+// rate at gl07 z40 mixed.  As points with triangles formed per arc, as points with
+// shared triangles, and so: gl07 mixed 223, 188, 166 us; gl07 FP64 448, 362, 299;
+// gl06 z60 FP64 184, 147, 118.
 struct TrcHFlux {
   static constexpr const char* kName = "trc_hflux";
-  Dims d; Consts c; Geo G;
+  Dims d; Geo G;
   real dt;
-  const real* pm;     // 5 mean-flux fields: rhog, rhogvx, rhogvy, rhogvz, rhogw
+  const real* pm;   // rhog, rhogvx, rhogvy, rhogvz (field stride NF)
   real* fa[3];
   real* xc[9];
-  // the column launch walks every level; the point launch (more threads, the
-  // levels being independent) does one
-  NH_HD void operator()(long t) const { levels(cell_of(d, t), 0, d.kall); }
-  NH_HD void operator()(int plane, int x) const {
-    Pt p;
-    if (pt_of(d, plane, x, p)) levels(cell_of_pt(p), p.k, p.k + 1);
-  }
-  NH_HD void levels(const Cell& cl, int k0, int k1) const {
-    const long NF = d.NF;
-    if (cl.pole) {
-      if (cl.v != 0) return;
-      const int lp = cl.lp;
-      for (int k = k0; k < k1; ++k) {
-        const long a0 = cl.base + k * 6;
-        real rt[6][4];
-        for (int v = 1; v <= 5; ++v) {
-          int vp = (v == 5) ? 1 : v + 1;
-          const real* w = G.twt_pl + (v * 2 + lp) * 3;
-          for (int q = 0; q < 4; ++q) {
-            const real* f = pm + q * NF;
-            rt[v][q] = f[a0] * w[0] + f[a0 + v] * w[1] + f[a0 + vp] * w[2];
-          }
-        }
-        for (int v = 1; v <= 5; ++v) {
-          int vm = (v == 1) ? 5 : v - 1;
-          const real rr = real(1.0) / dmax(rt[vm][0] + rt[v][0], NH_EPS);
-          const real v2x = rt[vm][1] + rt[v][1], v2y = rt[vm][2] + rt[v][2], v2z = rt[vm][3] + rt[v][3];
-          const real* hn = G.ahn_pl + (v * 2 + lp) * 3;
-          fa[0][a0 + v] = real(0.5) * (v2x * hn[0] + v2y * hn[1] + v2z * hn[2]);
-          const real* xr = G.axr_pl + (v * 2 + lp) * 3;
-          xc[0][a0 + v] = xr[0] - v2x * rr * dt * real(0.5);
-          xc[1][a0 + v] = xr[1] - v2y * rr * dt * real(0.5);
-          xc[2][a0 + v] = xr[2] - v2z * rr * dt * real(0.5);
-        }
-      }
+  int KC;           // levels per thread
+  long threads() const { return (d.nreg + 2) * ((d.kall + KC - 1) / KC); }
+  NH_HD void operator()(long t) const {
+    const long NF = d.NF, nc = d.nreg + 2;
+    const long chunk = t / nc, c = t - chunk * nc;
+    const int k0 = (int)chunk * KC, k1 = (k0 + KC < d.kall) ? k0 + KC : d.kall;
+    if (c >= d.nreg) {
+      const int lp = (int)(c - d.nreg);
+      for (int k = k0; k < k1; ++k) pole(lp, d.R + (long)(lp * d.kall + k) * 6);
       return;
     }
-    const int g = d.g, i = cl.i, j = cl.j;
+    const int g = d.g, gg = g * g;
+    const long ci = c;
+    const int l = (int)(ci / gg), h = (int)(ci - (long)l * gg), j = h / g, i = h - j * g;
     if (i > g - 2 || j > g - 2) return;
-    const long nreg = d.nreg, ci = cl.ci, ks = cl.ks;
-    const real m0 = G.sgp[cl.l] ? real(0.0) : real(1.0), m1 = G.sgp[cl.l] ? real(1.0) : real(0.0);
+    const long nreg = d.nreg;
+    // the four triangles of a point's arcs: TI and TJ of the point, TJ of
+    // (i, j-1) and TI of (i-1, j) (the point's own where there is none: the
+    // arc is then dropped)
+    const int south = j >= 1 ? -g : 0, west = i >= 1 ? -1 : 0;
+    real wi[3], wj[3], ws[3], ww[3], hn[9], xr[9];
+    for (int m = 0; m < 3; ++m) {
+      wi[m] = rcp(G.twt, nreg, m, ci);
+      wj[m] = rcp(G.twt, nreg, 3 + m, ci);
+      ws[m] = rcp(G.twt, nreg, 3 + m, ci + south);
+      ww[m] = rcp(G.twt, nreg, m, ci + west);
+    }
+    for (int m = 0; m < 9; ++m) {
+      hn[m] = rcp(G.ahn, nreg, m, ci);
+      xr[m] = rcp(G.axr, nreg, m, ci);
+    }
     for (int k = k0; k < k1; ++k) {
-      const long a = cl.base + k * ks;
-      // triangle value of type T with corner at offset (di, dj) from this cell
-      auto tri = [&](int T, int di, int dj, int q) -> real {
-        const real* f = pm + q * NF;
-        const long o = a + di + (long)dj * g;
-        const long cc = ci + di + (long)dj * g;
-        const real w1 = rcp(G.twt, nreg, T * 3 + 0, cc), w2 = rcp(G.twt, nreg, T * 3 + 1, cc),
-                     w3 = rcp(G.twt, nreg, T * 3 + 2, cc);
-        if (T == 0) {
-          real s = f[o] * w1 + f[o + 1] * w2;
-          return s + f[o + 1 + g] * w3;
-        }
-        real s = f[o] * w1;
-        return s + (f[o + 1 + g] * w2 + f[o + g] * w3);
-      };
-      // the (0, 0) TI triangle is replaced by TJ(1, 0) on pentagon regions (arithmetic mask, all regions)
-      auto triv = [&](int T, int di, int dj, int q) -> real {
-        real v = tri(T, di, dj, q);
-        if (T == 0 && i + di == 0 && j + dj == 0) v = v * m0 + tri(1, 1 - i, -j, q) * m1;
-        return v;
-      };
-      // arcs: AI (TJ(i, j-1) + TI(i, j)), AIJ (TI(i, j) + TJ(i, j)), AJ (TJ(i, j) + TI(i-1, j))
-      for (int arc = 0; arc < 3; ++arc) {
-        int Ta, dia, dja, Tb, dib, djb;
-        bool valid = true;
-        if (arc == 0) { Ta = 1; dia = 0; dja = -1; Tb = 0; dib = 0; djb = 0; valid = (j >= 1); }
-        else if (arc == 1) { Ta = 0; dia = 0; dja = 0; Tb = 1; dib = 0; djb = 0; }
-        else { Ta = 1; dia = 0; dja = 0; Tb = 0; dib = -1; djb = 0; valid = (i >= 1); }
-        if (!valid) {
-          fa[arc][a] = real(0.0);
-          for (int dd = 0; dd < 3; ++dd) xc[arc * 3 + dd][a] = real(0.0);
-          continue;
-        }
-        const real rs = triv(Ta, dia, dja, 0) + triv(Tb, dib, djb, 0);
-        const real rr = real(1.0) / dmax(rs, NH_EPS);
-        real v2[3];
-        for (int q = 0; q < 3; ++q) v2[q] = triv(Ta, dia, dja, q + 1) + triv(Tb, dib, djb, q + 1);
-        const real hx = rcp(G.ahn, nreg, arc * 3 + 0, ci), hy = rcp(G.ahn, nreg, arc * 3 + 1, ci),
-                     hz = rcp(G.ahn, nreg, arc * 3 + 2, ci);
-        fa[arc][a] = real(0.5) * (v2[0] * hx + v2[1] * hy + v2[2] * hz);
-        for (int dd = 0; dd < 3; ++dd)
-          xc[arc * 3 + dd][a] = rcp(G.axr, nreg, arc * 3 + dd, ci) - v2[dd] * rr * dt * real(0.5);
+      const long a = ((long)l * d.kall + k) * gg + h;
+      const unsigned o = byte_off(a);
+      real f[4][6];
+      for (int q = 0; q < 4; ++q) {
+        const real* pq = pm + q * NF;
+        f[q][0] = at_off(pq, o);
+        f[q][1] = at_off(pq + 1, o);
+        f[q][2] = at_off(pq + 1 + g, o);
+        f[q][3] = at_off(pq + g, o);
+        f[q][4] = at_off(pq, o + (unsigned)(south * (int)sizeof(real)));
+        f[q][5] = at_off(pq, o + (unsigned)(west * (int)sizeof(real)));
       }
+      // arcs: AI (TJ(i, j-1) + TI(i, j)), AIJ (TI(i, j) + TJ(i, j)), AJ (TJ(i, j) + TI(i-1, j))
+      real s[3][4];
+      for (int q = 0; q < 4; ++q) {
+        const real* e = f[q];
+        real ti = (e[0] * wi[0] + e[1] * wi[1]) + e[2] * wi[2];
+        const real tj = e[0] * wj[0] + (e[2] * wj[1] + e[3] * wj[2]);
+        const real ts = e[4] * ws[0] + (e[1] * ws[1] + e[0] * ws[2]);
+        real tw = (e[5] * ww[0] + e[0] * ww[1]) + e[3] * ww[2];
+        if (j == 0 && i <= 1) {
+          // the (0, 0) TI triangle is replaced by TJ(1, 0) on pentagon regions (arithmetic mask, all regions)
+          const real m0 = G.sgp[l] ? real(0.0) : real(1.0), m1 = G.sgp[l] ? real(1.0) : real(0.0);
+          const real* b = pm + q * NF + a + (1 - i);
+          const long c1 = ci + (1 - i);
+          const real t1 = b[0] * rcp(G.twt, nreg, 3, c1)
+                          + (b[1 + g] * rcp(G.twt, nreg, 4, c1) + b[g] * rcp(G.twt, nreg, 5, c1));
+          if (i == 0) ti = ti * m0 + t1 * m1;
+          else tw = tw * m0 + t1 * m1;
+        }
+        s[0][q] = ts + ti;
+        s[1][q] = ti + tj;
+        s[2][q] = tj + tw;
+      }
+      for (int arc = 0; arc < 3; ++arc) {
+        const bool valid = arc == 1 || (arc == 0 ? j >= 1 : i >= 1);
+        const real* v2 = s[arc] + 1;
+        const real rr = real(1.0) / dmax(s[arc][0], NH_EPS);
+        const real fl = real(0.5) * (v2[0] * hn[arc * 3] + v2[1] * hn[arc * 3 + 1] + v2[2] * hn[arc * 3 + 2]);
+        at_off(fa[arc], o) = valid ? fl : real(0.0);
+        for (int dd = 0; dd < 3; ++dd) {
+          const real xv = xr[arc * 3 + dd] - v2[dd] * rr * dt * real(0.5);
+          at_off(xc[arc * 3 + dd], o) = valid ? xv : real(0.0);
+        }
+      }
+    }
+  }
+  NH_HD void pole(int lp, long a0) const {
+    const long NF = d.NF;
+    real rt[6][4];
+    for (int v = 1; v <= 5; ++v) {
+      int vp = (v == 5) ? 1 : v + 1;
+      const real* w = G.twt_pl + (v * 2 + lp) * 3;
+      for (int q = 0; q < 4; ++q) {
+        const real* f = pm + q * NF;
+        rt[v][q] = f[a0] * w[0] + f[a0 + v] * w[1] + f[a0 + vp] * w[2];
+      }
+    }
+    for (int v = 1; v <= 5; ++v) {
+      int vm = (v == 1) ? 5 : v - 1;
+      const real rr = real(1.0) / dmax(rt[vm][0] + rt[v][0], NH_EPS);
+      const real v2x = rt[vm][1] + rt[v][1], v2y = rt[vm][2] + rt[v][2], v2z = rt[vm][3] + rt[v][3];
+      const real* hn = G.ahn_pl + (v * 2 + lp) * 3;
+      fa[0][a0 + v] = real(0.5) * (v2x * hn[0] + v2y * hn[1] + v2z * hn[2]);
+      const real* xr = G.axr_pl + (v * 2 + lp) * 3;
+      xc[0][a0 + v] = xr[0] - v2x * rr * dt * real(0.5);
+      xc[1][a0 + v] = xr[1] - v2y * rr * dt * real(0.5);
+      xc[2][a0 + v] = xr[2] - v2z * rr * dt * real(0.5);
     }
   }
 };
