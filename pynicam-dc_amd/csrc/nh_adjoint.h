@@ -199,7 +199,7 @@ struct ProgUpdateA {
 // ----------------------------------------------------------------------------
 // divergence damping: helpers of the transposes (the kernels are below)
 // ----------------------------------------------------------------------------
-// transpose of hex_sum over the three directions: o[dd] -> Tb[6]
+// transpose of the cdiff-weighted hexagon sum over the three directions: o[dd] -> Tb[6]
 NH_HD inline void hex_sum_t(const Geo& G, long nreg, long ci, const real o[3], real Tb[6]) {
   for (int n = 0; n < 6; ++n) Tb[n] = real(0.0);
   for (int dd = 0; dd < 3; ++dd) {
@@ -1919,16 +1919,16 @@ struct SfcPresP {
 
 // ----------------------------------------------------------------------------
 // divergence damping, gather form.  Both operators are out(cell) =
-// hex_sum(cell, T) over the six triangles around the cell of triangle values
-// T = tri_div (+ the vertical rhogw term for the first operator).
+// cdiff-weighted hexagon sum over the six triangles around the cell of triangle
+// divergences T (+ the vertical rhogw term for the first operator).
 // Kernel S: per corner b and level the bars of its two triangles, S(TI(b)) and
 // S(TJ(b)), each the sum over the triangle's three cells of the weight
 // w_n = sum_dd H_n(dd) o_dd that the cell's output bar o sends to it (H_n: the
-// hex_sum coefficient of triangle n of the cell; in the first operator the
+// hexagon-sum coefficient of triangle n of the cell; in the first operator the
 // pentagon corner (1,1) of an sgp region sends triangle 4's share to triangle
 // 5, as the forward substitutes T5 for T4 there).  The pole centre stores its
 // five ring-triangle bars in the pole slots 1..5 of the first field.
-// Kernel G: per point x the tri_div transposes at x's corner of each of the
+// Kernel G: per point x the triangle divergences' transposes at x's corner of each of the
 // six triangles around it (and, first operator, the vertical term from the
 // triangle sums at x's level and the one below).
 // ----------------------------------------------------------------------------
@@ -2016,7 +2016,7 @@ struct DivDampGA {
   Dims d; Consts c; Geo G;
   const real* S[2];   // the triangle bars of DivDampSA
   real* vb[4];        // OP 1: bars of rhogvx..vz, rhogw (added); OP 2: bars of the first result (set)
-  // the six triangles' bars at level offset (0 or -1) and their tri_div transposes at x
+  // the six triangles' bars at level offset (0 or -1) and their transposes at x
   NH_HD void operator()(int plane, int x) const {
     Pt p;
     if (!pt_of(d, plane, x, p)) return;

@@ -189,7 +189,7 @@ struct Oper7C {
       for (int m = 0; m < 7; ++m) col.c[dd][m] = rc(coef, d.nreg, dd * 7 + m, ci);
   }
   NH_HD void pole(int pb) const { pk(d.lall * d.kall + pb, 0); }
-  // per direction the sum over the neighbours in stencil order, as lap7, grad7 and div7
+  // per direction the sum over the neighbours in stencil order, the divergence's x + y + z
   template <class NB>
   NH_HD void point(int, unsigned o, const Col& col, Pre&, NB nb) const {
     real s[NC];

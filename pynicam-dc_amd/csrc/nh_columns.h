@@ -283,20 +283,6 @@ NH_HD inline T rcp(const T* a, long nreg, int comp, long ci) {
   else return a[comp * nreg + ci];
 }
 
-// 7-point divergence of (ax, ay, az)(point) at one level for a regional cell
-template <class FX, class FY, class FZ>
-NH_HD inline real div7(const Geo& G, long nreg, long ci, FX fx, FY fy, FZ fz) {
-  real sx, sy, sz;
-  // same association as the reference: sum over m for each direction, then x + y + z
-  sx = rc(G.cdiv, nreg, 0, ci) * fx(0);
-  for (int m = 1; m < 7; ++m) sx = sx + rc(G.cdiv, nreg, m, ci) * fx(m);
-  sy = rc(G.cdiv, nreg, 7, ci) * fy(0);
-  for (int m = 1; m < 7; ++m) sy = sy + rc(G.cdiv, nreg, 7 + m, ci) * fy(m);
-  sz = rc(G.cdiv, nreg, 14, ci) * fz(0);
-  for (int m = 1; m < 7; ++m) sz = sz + rc(G.cdiv, nreg, 14 + m, ci) * fz(m);
-  return sx + sy + sz;
-}
-
 // pole-centre divergence: sum over v = 0..5 of (cx*ax + cy*ay + cz*az)
 template <class FX, class FY, class FZ>
 NH_HD inline real div_pl(const Geo& G, int lp, FX fx, FY fy, FZ fz) {

@@ -248,13 +248,12 @@ struct HDiffPassP {
   }
   NH_HD void operator()(int plane, int x) const {
     Pt p;
-    if (!pt_of(d, plane, x, p) || !pt_compute(p)) return;
+    if (!pt_of(d, plane, x, p) || !p.pole || p.v != 0) return;
     if (!LAST) {
       at(p, [&](int f, long b) { return input(f, b, p.k); });
       return;
     }
     const long a = p.a;
-    const Cell cl = cell_of_pt(p);
     auto pa = [&](int v) { return src_pole(d, cs, p.lp, v, p.k); };
     for (int q = 0; q < 6; ++q) {
       real r;
@@ -263,9 +262,9 @@ struct HDiffPassP {
         const real* rg = rhog;
         const real gam = c.GAMMA_H;
         auto kh = [rg, fac, gam](long xx) { return rg[xx] * fac * gam; };
-        r = p.pole ? diffusion_pl(G, p.lp, in[q], kh, a, pa) : diffusion7(G, d, cl, in[q], kh, a);
+        r = diffusion_pl(G, p.lp, in[q], kh, a, pa);
       } else {
-        r = p.pole ? lap_pl_at(G, p.lp, in[q], pa) : lap7(G, d.nreg, p.ci, in[q], a, d.g);
+        r = lap_pl_at(G, p.lp, in[q], pa);
       }
       out[q][a] = -r;
     }
@@ -275,20 +274,10 @@ struct HDiffPassP {
   NH_HD void at(const Pt& p, LD ld) const {
     const long a = p.a;
     for (int q = 0; q < 6; ++q) {
-      real r;
-      if (p.pole) {
-        r = real(0.0);
-        for (int v = 0; v < 6; ++v) {
-          const real pv = G.clap_pl[v * 2 + p.lp] * ld(q, a + v);
-          r = (v == 0) ? pv : r + pv;
-        }
-      } else {
-        const long g = d.g;
-        r = rc(G.clap, d.nreg, 0, p.ci) * ld(q, a);
-        for (int m = 1; m < 7; ++m) {
-          const long off = (((4201 >> (2 * m)) & 3) - 1) + (((421 >> (2 * m)) & 3) - 1) * g;
-          r = r + rc(G.clap, d.nreg, m, p.ci) * ld(q, a + off);
-        }
+      real r = real(0.0);
+      for (int v = 0; v < 6; ++v) {
+        const real pv = G.clap_pl[v * 2 + p.lp] * ld(q, a + v);
+        r = (v == 0) ? pv : r + pv;
       }
       out[q][a] = -r;
     }
@@ -306,61 +295,39 @@ struct DivDamp1P {
   const int* cs;   // source columns of the inputs' halo values (read at the poles)
   NH_HD void operator()(int plane, int x) const {
     Pt p;
-    if (!pt_of(d, plane, x, p) || !pt_compute(p)) return;
-    const int kmin = d.kmin, kmax = d.kmax, g = d.g, k = p.k;
+    if (!pt_of(d, plane, x, p) || !p.pole || p.v != 0) return;
+    const int kmin = d.kmin, kmax = d.kmax, k = p.k;
     const long ks = p.ks, a = p.a;
     if (k < kmin || k > kmax) {
       for (int q = 0; q < 3; ++q) out[q][a] = real(0.0);
       return;
     }
     auto rwv = [&](long aa, int kk) { return (kk >= kmin + 1 && kk <= kmax) ? (real(0.0) * real(1.0) + rw[aa] * real(1.0)) : real(0.0); };
-    if (p.pole) {
-      real sclt[5];
-      auto pa = [&](int v, int kk) { return src_pole(d, cs, p.lp, v, kk); };
-      const real* vv[3] = {rvx, rvy, rvz};
-      for (int v = 1; v <= 5; ++v) {
-        const int vp = (v == 5) ? 1 : v + 1;
-        real s = real(0.0);
-        for (int dd = 0; dd < 3; ++dd) {
-          const real* cI = G.cintp_pl + ((v * 2 + p.lp) * 3 + dd) * 3;
-          const real t0 = cI[0] * (vv[dd][a] * real(1.0)), t1 = cI[1] * (vv[dd][pa(v, k)] * real(1.0)),
-                       t2 = cI[2] * (vv[dd][pa(vp, k)] * real(1.0));
-          s = (dd == 0) ? (t0 + t1 + t2) : (s + t0 + t1 + t2);
-        }
-        const real up = (rwv(a + ks, k + 1) + rwv(pa(v, k + 1), k + 1) + rwv(pa(vp, k + 1), k + 1));
-        const real dn = (rwv(a, k) + rwv(pa(v, k), k) + rwv(pa(vp, k), k));
-        sclt[v - 1] = s + (up - dn) / real(3.0) * G.rdgz[k];
-      }
+    real sclt[5];
+    auto pa = [&](int v, int kk) { return src_pole(d, cs, p.lp, v, kk); };
+    const real* vv[3] = {rvx, rvy, rvz};
+    for (int v = 1; v <= 5; ++v) {
+      const int vp = (v == 5) ? 1 : v + 1;
+      real s = real(0.0);
       for (int dd = 0; dd < 3; ++dd) {
-        real row = real(0.0);
-        for (int v = 1; v <= 5; ++v) {
-          const int vm = (v == 1) ? 5 : v - 1;
-          const real cb = G.cdiff_pl[(v * 2 + p.lp) * 3 + dd] * (sclt[vm - 1] + sclt[v - 1]);
-          row = (v == 1) ? cb : row + cb;
-        }
-        out[dd][a] = row;
+        const real* cI = G.cintp_pl + ((v * 2 + p.lp) * 3 + dd) * 3;
+        const real t0 = cI[0] * (vv[dd][a] * real(1.0)), t1 = cI[1] * (vv[dd][pa(v, k)] * real(1.0)),
+                     t2 = cI[2] * (vv[dd][pa(vp, k)] * real(1.0));
+        s = (dd == 0) ? (t0 + t1 + t2) : (s + t0 + t1 + t2);
       }
-      return;
+      const real up = (rwv(a + ks, k + 1) + rwv(pa(v, k + 1), k + 1) + rwv(pa(vp, k + 1), k + 1));
+      const real dn = (rwv(a, k) + rwv(pa(v, k), k) + rwv(pa(vp, k), k));
+      sclt[v - 1] = s + (up - dn) / real(3.0) * G.rdgz[k];
     }
-    const long nreg = d.nreg, ci = p.ci;
-    const long co[6] = {0, 0, -1, -1 - (long)g, -1 - (long)g, -(long)g};
-    const int ty[6] = {0, 1, 0, 1, 0, 1};
-    real T[6];
-    for (int n = 0; n < 6; ++n) {
-      const long aa = a + co[n];
-      const long cj = ci + co[n];
-      const long o1 = (ty[n] == 0) ? 1 : 1 + g;
-      const long o2 = (ty[n] == 0) ? 1 + g : g;
-      const real s = tri_div(G, nreg, cj, ty[n], rvx, rvy, rvz, aa, g, real(1.0));
-      const real up = (rwv(aa + ks, k + 1) + rwv(aa + o1 + ks, k + 1) + rwv(aa + o2 + ks, k + 1));
-      const real dn = (rwv(aa, k) + rwv(aa + o1, k) + rwv(aa + o2, k));
-      T[n] = s + (up - dn) / real(3.0) * G.rdgz[k];
+    for (int dd = 0; dd < 3; ++dd) {
+      real row = real(0.0);
+      for (int v = 1; v <= 5; ++v) {
+        const int vm = (v == 1) ? 5 : v - 1;
+        const real cb = G.cdiff_pl[(v * 2 + p.lp) * 3 + dd] * (sclt[vm - 1] + sclt[v - 1]);
+        row = (v == 1) ? cb : row + cb;
+      }
+      out[dd][a] = row;
     }
-    if (p.i == 1 && p.j == 1) {
-      const real m0 = G.sgp[p.l] ? real(0.0) : real(1.0), m1 = G.sgp[p.l] ? real(1.0) : real(0.0);
-      T[4] = T[4] * m0 + T[5] * m1;
-    }
-    for (int dd = 0; dd < 3; ++dd) out[dd][a] = hex_sum(G, nreg, ci, dd, T);
   }
 };
 
@@ -372,18 +339,14 @@ struct DivDamp2P {
   const int* cs;   // source columns of the inputs' halo values (read at the poles)
   NH_HD void operator()(int plane, int x) const {
     Pt p;
-    if (!pt_of(d, plane, x, p)) return;
+    if (!pt_of(d, plane, x, p) || !p.pole || p.v != 0) return;
     const long a = p.a;
-    const int kmin = d.kmin, kmax = d.kmax, g = d.g, k = p.k;
-    if (!pt_compute(p)) {
-      for (int q = 0; q < 3; ++q) out[q][a] = real(0.0);
-      return;
-    }
+    const int kmin = d.kmin, kmax = d.kmax, k = p.k;
     const real R = c.RADIUS;
     real o[3];
     if (k < kmin || k > kmax) {
       o[0] = o[1] = o[2] = real(0.0);
-    } else if (p.pole) {
+    } else {
       real sclt[5];
       for (int v = 1; v <= 5; ++v) {
         const int vp = (v == 5) ? 1 : v + 1;
@@ -405,28 +368,13 @@ struct DivDamp2P {
         }
         o[dd] = row;
       }
-    } else {
-      const long nreg = d.nreg, ci = p.ci;
-      const long co[6] = {0, 0, -1, -1 - (long)g, -1 - (long)g, -(long)g};
-      const int ty[6] = {0, 1, 0, 1, 0, 1};
-      real T[6];
-      for (int n = 0; n < 6; ++n) T[n] = tri_div(G, nreg, ci + co[n], ty[n], in[0], in[1], in[2], a + co[n], g, -real(1.0));
-      for (int dd = 0; dd < 3; ++dd) o[dd] = hex_sum(G, nreg, ci, dd, T);
     }
     const real gd[3] = {c.ALPHA_D * o[0], c.ALPHA_D * o[1], c.ALPHA_D * o[2]};
-    if (p.pole) {
-      const real gx = G.gx_pl[p.lp * 3 + 0], gy = G.gx_pl[p.lp * 3 + 1], gz = G.gx_pl[p.lp * 3 + 2];
-      const real prd = gd[0] * gx / R + gd[1] * gy / R + gd[2] * gz / R;
-      out[0][a] = gd[0] - prd * gx / R;
-      out[1][a] = gd[1] - prd * gy / R;
-      out[2][a] = gd[2] - prd * gz / R;
-    } else {
-      const real gx = G.gx[p.ci], gy = G.gx[d.nreg + p.ci], gz = G.gx[2 * d.nreg + p.ci];
-      const real prd = (gd[0] * gx + gd[1] * gy + gd[2] * gz) / R;
-      out[0][a] = gd[0] - prd * gx / R;
-      out[1][a] = gd[1] - prd * gy / R;
-      out[2][a] = gd[2] - prd * gz / R;
-    }
+    const real gx = G.gx_pl[p.lp * 3 + 0], gy = G.gx_pl[p.lp * 3 + 1], gz = G.gx_pl[p.lp * 3 + 2];
+    const real prd = gd[0] * gx / R + gd[1] * gy / R + gd[2] * gz / R;
+    out[0][a] = gd[0] - prd * gx / R;
+    out[1][a] = gd[1] - prd * gy / R;
+    out[2][a] = gd[2] - prd * gz / R;
   }
 };
 
@@ -539,7 +487,7 @@ struct ViPath0P {
     if (k >= kmin && k <= kmax) {
       // div(rhogv), div(rhogv eth)
       real dvs[2];
-      hdiv_multi<2>(G, d, p, [&](int, long bn, real (*v)[3]) {
+      hdiv_multi<2>(G, p, [&](int, long bn, real (*v)[3]) {
         const real e = ld(3, bn);
         const real r3[3] = {ld(0, bn), ld(1, bn), ld(2, bn)};
         for (int q = 0; q < 3; ++q) {
@@ -805,7 +753,7 @@ struct ViMainH {
     const long NF = d.NF, a = p.a;
     // div(dv), div(dv eth), div((prog + dv) ethtot)
     real dvs[3];
-    hdiv_multi<3>(G, d, p, [&](int, long b, real (*v)[3]) {
+    hdiv_multi<3>(G, p, [&](int, long b, real (*v)[3]) {
       const real e = ld(3, b), et = ld(4, b);
       for (int q = 0; q < 3; ++q) {
         const real dq = ld(q, b);

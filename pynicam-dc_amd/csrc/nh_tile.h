@@ -203,7 +203,7 @@ struct DivDampK {
     }
     return k1 - k0;
   }
-  // triangle T of the corner from the level's loads (tri_div's arithmetic)
+  // triangle T of the corner from the level's loads (per vertex cintp times its value)
   NH_HD real tri(const State& s, int T) const {
     const int n1 = (T == 0) ? 1 : 2, n2 = (T == 0) ? 2 : 3;
     const real sgn = (OP == 1) ? real(1.0) : -real(1.0);
@@ -298,7 +298,7 @@ struct DivDampK {
 // column tiles, the same layout as DivDampK: corner threads form the triangle
 // gradients of both fields from their 18 held cintp coefficients, tile points
 // the Kh-weighted hexagon sums from their 18 held cdiff coefficients.
-// Results equal the point form's (diffusion7, kernels/oprtdiffusion.py:59-177).
+// (kernels/oprtdiffusion.py:59-177)
 // ----------------------------------------------------------------------------
 template <bool MAP>
 struct DiffKhK {
