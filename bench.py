@@ -50,7 +50,9 @@ def kernel_bytes(t, nq: int = 1, elem: int = 8) -> dict:
     the FP64 fields of the tridiagonal solve (matrix, forward-sweep scratch)
     D = 8 bytes per point; each per-column coefficient component counts
     C = elem bytes per column; k-only profiles are ignored.  Field counts
-    follow the arrays each kernel touches.
+    follow the arrays each kernel touches; where launches of one kernel differ
+    (first small step of a stage, accumulation of the tracer's mean fluxes) the
+    mean over a step's launches is given (3 stages, 2 + 3 + 6 small steps).
     """
     ncell = t.lall * t.gall_1d ** 2
     npts = ncell * t.kall + 12 * t.kall
@@ -66,47 +68,48 @@ def kernel_bytes(t, nq: int = 1, elem: int = 8) -> dict:
         "divdamp_3d": 7 * F + 36 * Cc,          # 4 in, 3 out; intp + diff coefs
         "divdamp_post": 6 * F + 39 * Cc,        # 3 in, 3 out; intp + diff + xyz
         "vi_path0": 31 * F + 3 * D + 45 * Cc,   # 23 in, 8 out + FP64 matrix 3 out; div + grad + xyz
-        "ethtot_mean": 12 * F,                  # prog 5 + eth in; ethtot + 5 means out
+        "ethtot_mean": 26 / 3 * F,              # prog 5 + eth in; ethtot out, last stage + 5 means
         "split_init": 15 * F,                   # prog0 6 + prog 6 in (2 of 3 stages), 6 out
-        "vi_path1": 20 * F + 24 * Cc,           # 14 in, 6 out; grad + xyz
+        "vi_path1": 161 / 11 * F + 24 * Cc,     # 10 in, 3 out; 3 of 11 launches + 3 means in and out; grad + xyz
         "vi_main_h": 12 * F + 21 * Cc,          # dv 3, prog 3, eth, ethtot, gT_e in; 3 out; div coefs
         "vi_main_v": 8 * F + 5 * D,             # split rho/w/e, gT rho/w, divergences 2 in, rhogw out;
                                                 # FP64 matrix 3 in, sweep scratch u, gamma
-        "vi_main_post": 26 * F,                 # state 5, split 6, dv 3, ethtot, gT, getot, div 2, rhogw, means 2 in; 4 out
+        "vi_main_post": 255 / 11 * F,           # state 5, split 2, dv 3, div 3, ethtot, gT, getot, rhogw, kinetic
+                                                # energy in, 3 out; first of a stage: split 4 for kinetic energy;
+                                                # 3 of 11 launches + split, 2 means in, 2 out
         "prog_update": 18 * F + 3 * Cc,         # 12 in, 6 out
-        "trc_vert1": (5 + 2 * nq) * F,          # w mean, rhog_in, frhog + tracers in; flux, rhog1 + tracers out
+        "trc_flux": 5 * F,                      # w mean, rhog_in, frhog in; flux, rhog1 out
+        "trc_vert1": (3 + 2 * nq) * F,          # w mean, rhog_in, frhog + tracers in; tracers out
         "trc_hflux": 16 * F + 24 * Cc,          # 4 mean fluxes in; 3 arc fluxes + 9 centroids out
         "trc_rhog2": 6 * F + 1 * Cc,
         "trc_gradq": 5 * F + 21 * Cc,
-        "trc_remap": 20 * F + 4 * Cc,
+        "trc_remap": 20 * F + 4 * Cc,           # one tracer (two in one launch: 28 F)
         "trc_qout": 8 * F + 1 * Cc,
         "trc_apply": 11 * F + 1 * Cc,
-        "trc_vert2": 5 * F,
+        "trc_vert2": (3 + 2 * nq) * F,
     }
 
 
-# rocprof kernel name -> library kernel name (the functor type inside k_run / k_pts)
+# functor type in a rocprof kernel name (without template arguments) -> library
+# kernel name; the rest is told apart by the first template argument
 KERNEL_TYPES = {
-    "PrePostP": "prepost", "AdvMomP": "adv_mom", "HDiffPassP<0>": "hdiff_pass1", "HDiffPassP<1>": "hdiff_pass2",
-    "DivDamp1P": "divdamp_3d", "DivDamp2P": "divdamp_post", "ViPath0P": "vi_path0", "EthTotPMP": "ethtot_mean",
-    "SplitInit": "split_init", "Path1P": "vi_path1", "ViMainH": "vi_main_h", "ViMainV<39>": "vi_main_v",
-    "ViMainV<0>": "vi_main_v",
-    "ViMainPost": "vi_main_post",
-    "ProgUpdateP": "prog_update", "HaloGather": "halo_gather", "TrcVert1": "trc_vert1", "TrcVert2": "trc_vert2",
-    "TrcHFlux": "trc_hflux", "TrcRhog2": "trc_rhog2", "TrcGradQ": "trc_gradq", "TrcRemap": "trc_remap",
-    "TrcQout": "trc_qout", "TrcApply": "trc_apply", "DivDampK<1>": "divdamp_3d", "DivDampK<2>": "divdamp_post",
-    "ViMainHC": "vi_main_h", "DiffKhK": "hdiff_pass2_kh", "AdvMomC": "adv_mom",
+    "PrePostP": "prepost", "AdvMomC": "adv_mom", "DiffKhK": "hdiff_pass2_kh", "ViPath0C": "vi_path0",
+    "EthTotPMP": "ethtot_mean", "SplitInit": "split_init", "Path1C": "vi_path1", "ViMainHC": "vi_main_h",
+    "ViMainV": "vi_main_v", "ViMainPost": "vi_main_post", "ProgUpdateP": "prog_update", "HaloGather": "halo_gather",
+    "TrcFlux": "trc_flux", "TrcVert1": "trc_vert1", "TrcVert2": "trc_vert2", "TrcHFlux": "trc_hflux",
+    "TrcRhog2": "trc_rhog2", "TrcRemap": "trc_remap", "TrcQoutC": "trc_qout", "TrcApplyC": "trc_apply",
+    "DivDampK<1": "divdamp_3d", "DivDampK<2": "divdamp_post", "LapC<6": "hdiff_pass1", "LapC<4": "hdiff_pass2_lap",
+    "Oper7C<TrcGradQ": "trc_gradq",
 }
 
 
 def _kernel_key(name: str):
     import re
-    lap = re.search(r"ColStencil<nh::f(?:64|32)::LapC<(\d+),", name)
-    if lap:
-        return "hdiff_pass1" if lap.group(1) == "6" else "hdiff_pass2_lap"
-    m = re.search(r"k_(?:pts|run|tiles|cols)<nh::f(?:64|32)::(?:(?:StagedPointT|ColStencil)<nh::f(?:64|32)::)?"
-                  r"(\w+(?:<\d+>)?)\s*>", name)
-    return KERNEL_TYPES.get(m.group(1)) if m else None
+    name = re.sub(r"nh::f(?:64|32)::", "", name)
+    m = re.search(r"k_(?:pts|run|tiles|cols)<(?:ColStencil<)?(\w+)(<\w+)?", name)
+    if not m:
+        return None
+    return KERNEL_TYPES.get(m.group(1)) or KERNEL_TYPES.get(m.group(1) + (m.group(2) or ""))
 
 
 def hbm_traffic(glevel: int, precision: str, timeout: float = 300.0):
