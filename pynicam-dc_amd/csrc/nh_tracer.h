@@ -4,8 +4,9 @@
 //   vertical half step   TrcFlux (fluxes, density), TrcVert1 (every column, all
 //                        tracers in place)
 //   horizontal step      TrcHFlux (arc mass fluxes, mass centroids), TrcRhog2,
-//                        then per tracer TrcGradQ -> halo -> TrcRemap -> TrcQout
-//                        -> halo -> TrcApply
+//                        then for one or two tracers TrcGradQ -> halo -> TrcRemap
+//                        and for each TrcQout -> halo -> TrcApply (both as column
+//                        tiles where the limiter is on, nh_trccol.h)
 //   vertical half step   TrcVert2 (compute cells, a group of tracers)
 //
 // The face mass fluxes of the reference's flx_h(i, j, face) are formed on the
@@ -363,9 +364,6 @@ struct TrcRhog2 {
   const real* rhog1;
   const real* frhog;
   real* rhog2;
-  // the column launch walks every level; the point launch (more threads, the
-  // levels being independent) does one
-  NH_HD void operator()(long t) const { levels(cell_of(d, t), 0, d.kall); }
   NH_HD void operator()(int plane, int x) const {
     Pt p;
     if (pt_of(d, plane, x, p)) levels(cell_of_pt(p), p.k, p.k + 1);
