@@ -259,72 +259,81 @@ int upload_geometry(X& x, Context& ctx, const nh_geometry* g) {
 // largest field (values) whose halo values are read at their source with 8-byte fields
 constexpr long kDirectMax64 = 4000000;
 
+// A map that is refused or does not fit leaves the context's present one in use.
 template <class X>
 int upload_halo(X& x, Context& ctx, const int32_t* dst, const int32_t* src, long n) {
-  const long ncol = ctx.d.nreg + 12;
+  const Dims& d = ctx.d;
+  const long ncol = d.nreg + 12;
   for (long h = 0; h < n; ++h) {
     if (dst[h] < 0 || dst[h] >= ncol || src[h] < 0 || src[h] >= ncol) return NH_ERR_ARG;
   }
-  if (ctx.halo_dst) { x.release(ctx.halo_dst); ctx.halo_dst = nullptr; }
-  if (ctx.halo_src) { x.release(ctx.halo_src); ctx.halo_src = nullptr; }
-  if (ctx.col_own) { x.release(ctx.col_own); ctx.col_own = ctx.col_src = nullptr; }
-  ctx.halo_n = n;
-  ctx.halo_direct = ctx.halo_full = false;
-  // the adjoint of the gather scatters destination bars onto sources in one
-  // pass: that needs every destination once and no destination as a source
-  {
-    std::vector<char> role((size_t)ncol, 0);
-    bool ok = true;
-    for (long h = 0; h < n && ok; ++h) {
-      if (role[dst[h]] & 1) ok = false;
-      role[dst[h]] |= 1;
-    }
-    for (long h = 0; h < n && ok; ++h) ok = !(role[src[h]] & 1);
-    ctx.halo_adj_ok = ok;
-    // col_src reads stand for a filled field only where no filled point is a
-    // compute point (a kernel's own value, or its neighbour's, would differ)
-    const int g = ctx.d.g;
-    for (long h = 0; h < n && ok; ++h) {
-      const long c = dst[h];
-      const long r = c % ((long)g * g), j = r / g, i = r - j * g;
-      ok = c < ctx.d.nreg ? !(i >= 1 && i <= g - 2 && j >= 1 && j <= g - 2) : (c - ctx.d.nreg) % 6 != 0;
-    }
-    // Reading halo values at their source saves three launches per small step
-    // (8 us each at gl05, 12-16 at gl06, 22-26 at gl07) and makes the readers
-    // slower, since the first and last column of a region are one value per
-    // cache line for them too.  With 4-byte fields it is the faster form at
-    // every size (step 4.66 -> 4.41 ms at gl06, 13.6 -> 13.3 at gl07); with
-    // 8-byte fields the corner kernels lose their paired loads (CornerPts),
-    // which pays up to about gl06 (gl05 2.78 -> 2.63 ms) and not at gl07.
-    ctx.halo_full = ok && n == ncol - (long)ctx.d.lall * (g - 2) * (g - 2) - 2;
-    ctx.halo_direct = ok && (sizeof(real) == 4 || ctx.d.NF <= kDirectMax64);
-  }
-  if (n == 0) return 0;
   // the kernels index halo slot and level in 32 bits and take level-0 field
   // addresses in 32 bits
-  if (n * ctx.d.kall >= (1L << 31) || ctx.d.NF >= (1L << 31)) return NH_ERR_ARG;
-  std::vector<int> db((size_t)n), sb((size_t)n);
-  for (long h = 0; h < n; ++h) {
-    long ks;
-    db[(size_t)h] = (int)halo_colbase(ctx.d, dst[h], &ks);
-    sb[(size_t)h] = (int)halo_colbase(ctx.d, src[h], &ks);
+  if (n > 0 && (n * d.kall >= (1L << 31) || d.NF >= (1L << 31))) return NH_ERR_ARG;
+  // the adjoint of the gather scatters destination bars onto sources in one
+  // pass: that needs every destination once and no destination as a source
+  std::vector<char> role((size_t)ncol, 0);
+  bool ok = true;
+  for (long h = 0; h < n && ok; ++h) {
+    if (role[dst[h]] & 1) ok = false;
+    role[dst[h]] |= 1;
   }
-  ctx.halo_dst = (int*)x.alloc(n * sizeof(int));
-  ctx.halo_src = (int*)x.alloc(n * sizeof(int));
-  if (!ctx.halo_dst || !ctx.halo_src) return NH_ERR_ALLOC;
-  x.h2d(ctx.halo_dst, db.data(), n * sizeof(int));
-  x.h2d(ctx.halo_src, sb.data(), n * sizeof(int));
-  std::vector<int> cols((size_t)(2 * ncol));
-  for (long c = 0; c < ncol; ++c) {
-    long ks;
-    cols[(size_t)c] = cols[(size_t)(ncol + c)] = (int)halo_colbase(ctx.d, c, &ks);
+  for (long h = 0; h < n && ok; ++h) ok = !(role[src[h]] & 1);
+  const bool adj_ok = ok;
+  // col_src reads stand for a filled field only where no filled point is a
+  // compute point (a kernel's own value, or its neighbour's, would differ)
+  const int g = d.g;
+  for (long h = 0; h < n && ok; ++h) {
+    const long c = dst[h];
+    const long r = c % ((long)g * g), j = r / g, i = r - j * g;
+    ok = c < d.nreg ? !(i >= 1 && i <= g - 2 && j >= 1 && j <= g - 2) : (c - d.nreg) % 6 != 0;
   }
-  if (ctx.halo_direct)
-    for (long h = 0; h < n; ++h) cols[(size_t)(ncol + dst[h])] = sb[(size_t)h];
-  ctx.col_own = (int*)x.alloc(2 * ncol * sizeof(int));
-  if (!ctx.col_own) return NH_ERR_ALLOC;
-  ctx.col_src = ctx.col_own + ncol;
-  x.h2d(ctx.col_own, cols.data(), 2 * ncol * sizeof(int));
+  // Reading halo values at their source saves three launches per small step
+  // (8 us each at gl05, 12-16 at gl06, 22-26 at gl07) and makes the readers
+  // slower, since the first and last column of a region are one value per
+  // cache line for them too.  With 4-byte fields it is the faster form at
+  // every size (step 4.66 -> 4.41 ms at gl06, 13.6 -> 13.3 at gl07); with
+  // 8-byte fields the corner kernels lose their paired loads (CornerPts),
+  // which pays up to about gl06 (gl05 2.78 -> 2.63 ms) and not at gl07.
+  const bool full = ok && n == ncol - (long)d.lall * (g - 2) * (g - 2) - 2;
+  const bool direct = ok && (sizeof(real) == 4 || d.NF <= kDirectMax64);
+  int *hd = nullptr, *hs = nullptr, *own = nullptr;
+  if (n > 0) {
+    std::vector<int> db((size_t)n), sb((size_t)n), cols((size_t)(2 * ncol));
+    long ks;
+    for (long h = 0; h < n; ++h) {
+      db[(size_t)h] = (int)halo_colbase(d, dst[h], &ks);
+      sb[(size_t)h] = (int)halo_colbase(d, src[h], &ks);
+    }
+    for (long c = 0; c < ncol; ++c) cols[(size_t)c] = cols[(size_t)(ncol + c)] = (int)halo_colbase(d, c, &ks);
+    if (direct)
+      for (long h = 0; h < n; ++h) cols[(size_t)(ncol + dst[h])] = sb[(size_t)h];
+    hd = (int*)x.alloc(n * sizeof(int));
+    hs = (int*)x.alloc(n * sizeof(int));
+    own = (int*)x.alloc(2 * ncol * sizeof(int));
+    int rc = (hd && hs && own) ? 0 : NH_ERR_ALLOC;
+    if (!rc) {
+      x.h2d(hd, db.data(), n * sizeof(int));
+      x.h2d(hs, sb.data(), n * sizeof(int));
+      x.h2d(own, cols.data(), 2 * ncol * sizeof(int));
+      rc = x.check("upload_halo");
+    }
+    if (rc) {
+      for (int* p : {hd, hs, own})
+        if (p) x.release(p);
+      return rc;
+    }
+  }
+  for (int* p : {ctx.halo_dst, ctx.halo_src, ctx.col_own})
+    if (p) x.release(p);
+  ctx.halo_dst = hd;
+  ctx.halo_src = hs;
+  ctx.col_own = own;
+  ctx.col_src = own ? own + ncol : nullptr;
+  ctx.halo_n = n;
+  ctx.halo_adj_ok = adj_ok;
+  ctx.halo_direct = n > 0 && direct;
+  ctx.halo_full = n > 0 && full;
   return x.check("upload_halo");
 }
 

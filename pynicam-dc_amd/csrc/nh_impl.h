@@ -80,8 +80,13 @@ int v_upload_geometry(Context* c, const nh_geometry* g, std::string* err) {
 
 int v_upload_halo(Context* c, const int32_t* dst, const int32_t* src, long n, std::string* err) {
   NHX x(c->device, nullptr, &c->prof);
-  int rc = upload_halo(x, *c, dst, src, n);
-  if (rc == NH_ERR_ARG) return failv(err, rc, "column id out of range");
+  int rc;
+  try {
+    rc = upload_halo(x, *c, dst, src, n);
+  } catch (const std::bad_alloc&) {
+    return failv(err, NH_ERR_ALLOC, "host allocation");
+  }
+  if (rc == NH_ERR_ARG) return failv(err, rc, "column id out of range or too many slots");
   if (rc == NH_ERR_ALLOC) return failv(err, rc, "device allocation");
   if (rc) return failv(err, rc, x.message());
   return 0;
