@@ -59,8 +59,8 @@ NH_HD inline T ldc(const T* p) {
 
 // Values at a 32-bit byte offset from a uniform base: one vector register
 // addresses the same point of every field (the loads take the base from scalar
-// registers).  A field is below 4 GiB: a context's 92 workspace fields of that
-// size are 395 GB, so its creation has failed on the card's 288 GB before.
+// registers).  A field is below 4 GiB: a context's 91 workspace fields of that
+// size are 391 GB, so its creation has failed on the card's 288 GB before.
 NH_HD inline unsigned byte_off(long a) { return (unsigned)a * (unsigned)sizeof(real); }
 template <class T>
 NH_HD inline const T& at_off(const T* p, unsigned off) {

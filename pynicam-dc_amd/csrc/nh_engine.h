@@ -59,10 +59,10 @@ enum WsField {
   W_GQ = 79,              // 3  gradient of the mixing ratio
   W_QA = 82,              // 3  upwind face values (faces 0..2)
   W_QOUT = 85,            // 2  limiter outflow bounds
-  W_RQ = 87,              // 1  tracer after the horizontal step (adjoint)
+  W_RQ = 87,              // 1  tracer after the horizontal step (tracer adjoint)
+  W_KIN = W_RQ,           // 1  kinetic energy of the small-step state (the dynamics step leaves W_RQ free)
   W_HV = 88,              // 3  horizontal divergences of the small-step momentum
-  W_KIN = 91,             // 1  kinetic energy of the small-step state
-  W_NFIELDS = 92
+  W_NFIELDS = 91
 };
 
 // FP64 fields (every form): the tridiagonal matrix, the forward-sweep scratch
