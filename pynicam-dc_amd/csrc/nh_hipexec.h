@@ -112,6 +112,8 @@ class HipExec {
     hipError_t e = hipMalloc(&p, bytes);
     if (e != hipSuccess) {
       note(e, "hipMalloc");
+      // reported by the null pointer: left pending, it would fail the caller's next launch check
+      (void)hipGetLastError();
       return nullptr;
     }
     return p;
