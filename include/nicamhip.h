@@ -196,7 +196,7 @@ int nh_vi_matrix_f32(nh_context* ctx, const float* eth_h, const float* g_tilde, 
 
 /* rhogw column solve (FP64 arithmetic in both forms): source assembly, the two
  * boundary rows and the Thomas sweeps on rows kmin+1..kmax; out rows below kmin
- * and above kmax+1 are copies of rhogw; out may be rhogw.  Replaces
+ * and above kmax+1 are copies of rhogw; out may be any of the field inputs.  Replaces
  * compute_rhow_solver_reg/_pl (nhm/dynamics/kernels/virhowsolver.py:67-172;
  * called from mod_vi.py:2433-2504 vi_rhow_solver). */
 int nh_vi_solve(nh_context* ctx, const double* rhogw, const double* rhogw0, const double* preg0, const double* rhog0,

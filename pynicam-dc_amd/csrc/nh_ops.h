@@ -56,12 +56,22 @@ struct ViMatrixOp {
 // ----------------------------------------------------------------------------
 // one thread per column; the forward sweep keeps u and gamma in registers
 // (NK = kmax - kmin unknowns, or a 78-entry private array for NK = 0).  out
-// may be rhogw itself: each column reads its boundary rows before it stores.
+// may be any of the inputs: each column reads its rows before it stores.
+//
+// The row copies stand last: as a branch between the sweeps they let the
+// compiler move every division of the unrolled form below it, with all rows'
+// loads held until there (FP64: 512 registers and 306 spilled; now 226 and
+// none).  z40, kernel time: FP64 gl05 72 -> 16 us, gl06 92 -> 25, gl07 359 -> 120;
+// mixed gl05 20 -> 13, gl06 33 -> 19, gl07 118 -> 82.  The NK = 0 form, both sweeps
+// unrolled by 4 and stepping one address (before: by 2, an address per row): gl06 z60
+// FP64 78 -> 60, mixed 58 -> 41, gl07 z60 FP64 246 -> 220.
 template <int NK>
 struct ViSolveOp {
   static constexpr const char* kName = "op_vi_solve";
   static constexpr int kMax = NK > 0 ? NK : 78;
-  static constexpr int kUnroll = NK > 0 ? NK : 2;
+  static constexpr int kUnroll = NK > 0 ? NK : 4;
+  // rows in flight: a column's loads overlap its divisions
+  static constexpr int kAhead = 3;
   Dims d; Consts c; Geo G;
   double dt;
   const real *rhogw, *rhogw0, *preg0, *rhog0, *Srho, *Sw, *Spre;
@@ -79,17 +89,15 @@ struct ViSolveOp {
     const double rw_top = (double)rhogw[b + (long)(kmax + 1) * ks];
     double u[kMax], gm[kMax];
     double beta = 0.0;
-    // rows are loaded kAhead levels before they are formed (as in ViMainV): a
-    // column's loads overlap its divisions.  gl06 z40 mixed: 43.8 -> 35.4 us.
-    // Plain loads, since out may be any of the inputs
     struct Row {
       real rw0, sw, p0, sp, r0, sr;
       double mc, mu, ml;
     };
-    constexpr int kAhead = (NK > 0 && sizeof(real) == 8) ? 1 : 3;
+    // the next row, from the last one on that one again (not used)
+    long al = b + (long)kmin * ks;
     auto load = [&](int n) {
-      const long a = b + (long)(kmin + 1 + (n < N ? n : N - 1)) * ks;
-      return Row{rhogw0[a], Sw[a], preg0[a], Spre[a], rhog0[a], Srho[a], Mc[a], Mu[a], Ml[a]};
+      if (n < N) al += ks;
+      return Row{rhogw0[al], Sw[al], preg0[al], Spre[al], rhog0[al], Srho[al], Mc[al], Mu[al], Ml[al]};
     };
     Row ahead[kAhead];
     for (int q = 0; q < kAhead; ++q) ahead[q] = load(q);
@@ -122,19 +130,21 @@ struct ViSolveOp {
       e_m = e_k;
       r_m = r_k;
     }
-    // the rows below kmin and above kmax+1 are copied, the boundary rows scaled by GSGAM2H
+    double x = u[N - 1];
+    long ab = b + (long)kmax * ks;
+    out[ab] = (real)x;
+#pragma unroll kUnroll
+    for (int n = N - 2; n >= 0; --n) {
+      ab -= ks;
+      x = u[n] - gm[n + 1] * x;
+      out[ab] = (real)x;
+    }
+    out[b + (long)kmin * ks] = (real)rw_bot;
+    out[b + (long)(kmax + 1) * ks] = (real)rw_top;
     if (out != rhogw) {
       for (int k = 0; k < kmin; ++k) out[b + (long)k * ks] = rhogw[b + (long)k * ks];
       for (int k = kmax + 2; k < d.kall; ++k) out[b + (long)k * ks] = rhogw[b + (long)k * ks];
     }
-    double x = u[N - 1];
-    out[b + (long)kmax * ks] = (real)x;
-    for (int n = N - 2; n >= 0; --n) {
-      x = u[n] - gm[n + 1] * x;
-      out[b + (long)(kmin + 1 + n) * ks] = (real)x;
-    }
-    out[b + (long)kmin * ks] = (real)rw_bot;
-    out[b + (long)(kmax + 1) * ks] = (real)rw_top;
   }
 };
 
