@@ -11,6 +11,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #ifndef NH_HD
@@ -35,12 +36,19 @@ __device__ inline int xcd_block(int L, int nblk) {
   return (rem == 0 || xcd < rem) ? xcd * per + idx : rem * per + (xcd - rem) * (per - 1) + idx;
 }
 
+// a functor with kDealt = true keeps the hardware's round-robin order
+template <class F, class = void>
+inline constexpr bool kDealtOrder = false;
+template <class F>
+inline constexpr bool kDealtOrder<F, std::void_t<decltype(F::kDealt)>> = F::kDealt;
+
 // flat launch.  With the round-robin order the halo gathers fetched the lines
 // of their strided edge columns into several L2s: 26.8 -> 22.1 us per launch at
 // gl07 mixed, 15.9 -> 11.9 at gl06; the column sweeps are level.
 template <class F>
 __global__ __launch_bounds__(256) void k_run(F f, long n) {
-  long t = (long)xcd_block((int)blockIdx.x, (int)gridDim.x) * blockDim.x + threadIdx.x;
+  const int blk = kDealtOrder<F> ? (int)blockIdx.x : xcd_block((int)blockIdx.x, (int)gridDim.x);
+  long t = (long)blk * blockDim.x + threadIdx.x;
   if (t < n) f(t);
 }
 
