@@ -293,8 +293,13 @@ int upload_halo(X& x, Context& ctx, const int32_t* dst, const int32_t* src, long
   // slower, since the first and last column of a region are one value per
   // cache line for them too.  With 4-byte fields it is the faster form at
   // every size (step 4.66 -> 4.41 ms at gl06, 13.6 -> 13.3 at gl07); with
-  // 8-byte fields the corner kernels lose their paired loads (CornerPts),
-  // which pays up to about gl06 (gl05 2.78 -> 2.63 ms) and not at gl07.
+  // 8-byte fields the corner kernels lose their paired loads (CornerPts), a
+  // loss per value, against a gain per launch that depends less on the size.
+  // FP64 step filled against read at the source: gl06 z20 (1.0 M values) 3.59,
+  // 3.51 ms; gl06 z40 (1.9 M) 6.12, 6.00; gl07 z14 (2.8 M) 8.53, 8.48; gl06 z78
+  // (3.7 M) 12.14, 12.03; gl07 z20 (3.8 M) 11.65, 11.65; gl07 z30 (5.6 M) 16.92,
+  // 17.05; gl07 z40 (7.3 M) 21.42, 21.72.  (Alone, the hyperdiffusion operator
+  // still gains 1 % at 7.3 M and the damping loses 1 % from 2.1 M on.)
   const bool full = ok && n == ncol - (long)d.lall * (g - 2) * (g - 2) - 2;
   const bool direct = ok && (sizeof(real) == 4 || d.NF <= kDirectMax64);
   int *hd = nullptr, *hs = nullptr, *own = nullptr;
