@@ -68,7 +68,7 @@ def kernel_bytes(t, nq: int = 1, elem: int = 8) -> dict:
         "divdamp_3d": 7 * F + 36 * Cc,          # 4 in, 3 out; intp + diff coefs
         "divdamp_post": 6 * F + 39 * Cc,        # 3 in, 3 out; intp + diff + xyz
         "vi_path0": 31 * F + 3 * D + 45 * Cc,   # 23 in, 8 out + FP64 matrix 3 out; div + grad + xyz
-        "ethtot_mean": 26 / 3 * F,              # prog 5 + eth in; ethtot out, last stage + 5 means
+        "ethtot_mean": 7 * F,                   # prog 5 + eth in; ethtot out
         "split_init": 15 * F,                   # prog0 6 + prog 6 in (2 of 3 stages), 6 out
         "vi_path1": 161 / 11 * F + 24 * Cc,     # 10 in, 3 out; 3 of 11 launches + 3 means in and out; grad + xyz
         "vi_main_h": 12 * F + 21 * Cc,          # dv 3, prog 3, eth, ethtot, gT_e in; 3 out; div coefs

@@ -299,7 +299,8 @@ int upload_halo(X& x, Context& ctx, const int32_t* dst, const int32_t* src, long
   // 3.51 ms; gl06 z40 (1.9 M) 6.12, 6.00; gl07 z14 (2.8 M) 8.53, 8.48; gl06 z78
   // (3.7 M) 12.14, 12.03; gl07 z20 (3.8 M) 11.65, 11.65; gl07 z30 (5.6 M) 16.92,
   // 17.05; gl07 z40 (7.3 M) 21.42, 21.72.  (Alone, the hyperdiffusion operator
-  // still gains 1 % at 7.3 M and the damping loses 1 % from 2.1 M on.)
+  // still gains 1 % at 7.3 M; the damping is level from 2.1 to 3.8 M and loses 2 to
+  // 4 % beyond.)
   const bool full = ok && n == ncol - (long)d.lall * (g - 2) * (g - 2) - 2;
   const bool direct = ok && (sizeof(real) == 4 || d.NF <= kDirectMax64);
   int *hd = nullptr, *hs = nullptr, *own = nullptr;

@@ -600,7 +600,9 @@ struct MeanFlux {
   }
 };
 
-// total specific energy of the large-step state and the start of the time-mean fluxes
+// total specific energy of the large-step state; pm (null elsewhere): the start of the
+// time-mean fluxes in the last stage under a halo map that leaves columns out, where
+// the copy stands for the fill (a full map's small steps start from prog itself)
 struct EthTotPMP {
   static constexpr const char* kName = "ethtot_mean";
   Dims d; Consts c; Geo G;
@@ -627,7 +629,7 @@ struct EthTotPMP {
     };
     const real kin0 = rhogkin_k(G, d.kmin, d.kmax, k, get);
     ethtot[a] = e + kin0 / rg[1] + G.phi[k];
-    if (pm) {   // null: the mean fluxes are not wanted (adjoint recompute)
+    if (pm) {
       pm[a] = rg[1];
       for (int q = 0; q < 3; ++q) pm[(1 + q) * NF + a] = rv[q];
       pm[4 * NF + a] = rw[0];
