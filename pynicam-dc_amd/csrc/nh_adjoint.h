@@ -1323,18 +1323,6 @@ struct ViMainVAb {
 // rhoge splits (we[0], we[2], consumed) -> inputs; we_b[1] receives the bar
 // of the new rhogw split it read
 // ----------------------------------------------------------------------------
-// the point of a compute column at level k
-NH_HD inline Pt pt_at(const Dims& d, const Cell& cl, int k) {
-  Pt p;
-  p.pole = cl.pole; p.inner = cl.inner;
-  p.i = cl.i; p.j = cl.j; p.l = cl.l; p.v = cl.v; p.lp = cl.lp; p.k = k;
-  p.ks = cl.ks;
-  p.a = cl.base + (long)k * cl.ks;
-  p.ci = cl.ci;
-  (void)d;
-  return p;
-}
-
 struct ViMainPostA {
   static constexpr const char* kName = "vi_main_post_adj";
   // the bar fields it adds to: PROG 0..4, split 0..5, dv 0..2, the new rhogw

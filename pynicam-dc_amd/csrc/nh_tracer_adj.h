@@ -109,9 +109,7 @@ struct TrcApplyA {
   int limiter;
   real* gq_b[3];       // limiter off: bars of the gradient (faces 3..5)
   const real* xc[9];
-  // per level on the point grid (levels independent; the adds to other
-  // points are atomic), or every level of a column
-  NH_HD void operator()(long t) const { levels(cell_of(d, t), 0, d.kall); }
+  // levels are independent; the adds to other points are atomic
   NH_HD void operator()(int plane, int x) const {
     Pt p;
     if (pt_of(d, plane, x, p)) levels(cell_of_pt(p), p.k, p.k + 1);
@@ -216,9 +214,7 @@ struct TrcQoutA {
   const real* fa[3];
   real* qo_b[2];
   TgSink sk;
-  // per level on the point grid (levels independent; the adds to other
-  // points are atomic), or every level of a column
-  NH_HD void operator()(long t) const { levels(cell_of(d, t), 0, d.kall); }
+  // levels are independent; the adds to other points are atomic
   NH_HD void operator()(int plane, int x) const {
     Pt p;
     if (pt_of(d, plane, x, p)) levels(cell_of_pt(p), p.k, p.k + 1);
@@ -310,9 +306,7 @@ struct TrcRemapA {
   real* qa_b[3];
   real* rq_b;
   real* gq_b[3];
-  // per level on the point grid (levels independent; the adds to other
-  // points are atomic), or every level of a column
-  NH_HD void operator()(long t) const { levels(cell_of(d, t), 0, d.kall); }
+  // levels are independent; the adds to other points are atomic
   NH_HD void operator()(int plane, int x) const {
     Pt p;
     if (pt_of(d, plane, x, p)) levels(cell_of_pt(p), p.k, p.k + 1);
@@ -370,9 +364,7 @@ struct TrcGradQA {
   const real* rhog1;
   real* gq_b[3];
   real* rq_b;
-  // per level on the point grid (levels independent; the adds to other
-  // points are atomic), or every level of a column
-  NH_HD void operator()(long t) const { levels(cell_of(d, t), 0, d.kall); }
+  // levels are independent; the adds to other points are atomic
   NH_HD void operator()(int plane, int x) const {
     Pt p;
     if (pt_of(d, plane, x, p)) levels(cell_of_pt(p), p.k, p.k + 1);
